@@ -522,25 +522,6 @@ __device__ __forceinline__ void fluid_pair_gp(const FluidElem& E, T mu, double m
     }
 }
 
-// The whole (a,b) block: the four Gauss points in order.
-template <typename T>
-__device__ __forceinline__ void fluid_pair(const FluidElem& E, T mu, const AsmParams& P, const Tet4Rule& rule,
-                                           int a, int b, bool want_r, T k[16], T r[4])
-{
-    FluidAB S;
-    fluid_ab(E, rule, a, b, S);
-#pragma unroll
-    for (int q = 0; q < 16; ++q) k[q] = scal<T>(0.0);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) r[q] = scal<T>(0.0);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        FluidGP<T> G;
-        fluid_gp(E, mu, P, rule, g, G);
-        fluid_pair_gp(E, mu, 0.0, P, rule, g, G, S, want_r, k, r);
-    }
-}
-
 __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const int* __restrict__ ien,
                                                    const int* __restrict__ elemId,
                                                    const int* __restrict__ emap,
@@ -625,9 +606,16 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
 
 // Viscosity sensitivity of the fluid element (no reference counterpart):
 // g_e = lam_e^T (dR_e/dmu_e - dK_e/dmu_e du_e), the element term of
-// dL/dmu_e when K du = R and K^T lam = dL/du.  Sixteen lanes per element
-// (one per (a,b) block) evaluate the dual-number element routine; the
-// element sum is a fixed-order shuffle reduction over the 16 lanes.
+// dL/dmu_e when K du = R and K^T lam = dL/du.  Four lanes per element, one
+// per Gauss point.  The element matrix is never formed: lam_e^T K_e du_e
+// needs the block sums of FLUID3D_M/C only through the values and gradients
+// of the two nodal fields at the point (l, lp and Lx, Lpx of lam; D, Dp and
+// Dx, Dpx of du), so a lane gathers those with the state's while it reads
+// the nodes and evaluates the bilinear form once in dual numbers (mu_e, 1).
+// Bound by FP64 arithmetic: the geometry and stabilisation parameters, about
+// 700 flops per lane.  One lane per (a, b) block, each repeating the
+// geometry and all four points in dual numbers, took 432 us on the
+// 197,696-tet cylinder; this takes about 40 us (adjoint terms of one gradient: 454 -> 96 us).
 __global__ __launch_bounds__(256) void k_fluid_dmu(int nEl, const int* __restrict__ ien,
                                                    const int* __restrict__ elemId, const double* __restrict__ x,
                                                    int tDof, const double* __restrict__ Ag,
@@ -636,28 +624,132 @@ __global__ __launch_bounds__(256) void k_fluid_dmu(int nEl, const int* __restric
                                                    const double* __restrict__ du, double* __restrict__ g)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nEl * 16) return;
-    const int p = t >> 4;
-    const int ab = t & 15;
-    const int a = ab >> 2, b = ab & 3;
-    FluidElem E;
-    fluid_elem(p, ien, x, tDof, Ag, Yg, E);
-    const Dual mu = {muEl ? muEl[elemId[p]] : P.mu, 1.0};
-    Dual k[16], r[4];
-    fluid_pair<Dual>(E, mu, P, rule, a, b, b == 0, k, r);
-    const double* la = lam + (size_t)ien[(size_t)p * 4 + a] * 4;
-    const double* ub = du + (size_t)ien[(size_t)p * 4 + b] * 4;
-    double s = 0.0;
+    if (t >= nEl * 4) return;
+    const int p = t >> 2, gp = t & 3;
+    int nd[4];
+    double xl[4][3];
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-        double kd = 0.0;
+    for (int q = 0; q < 4; ++q) {
+        nd[q] = ien[(size_t)p * 4 + q];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) kd += k[rr * 4 + c].d * ub[c];
-        s += la[rr] * ((b == 0 ? r[rr].d : 0.0) - kd);
+        for (int i = 0; i < 3; ++i) xl[q][i] = x[(size_t)nd[q] * 3 + i];
     }
+    double Nx[4][3], ks[3][3], Jac;
+    gnn_tet4(xl, Nx, Jac, ks);
+    // N and the weight of this lane's point, without a lane-dependent index
+    double N[4], w = 0.0;
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 16);
-    if (ab == 0) g[elemId[p]] = s;
+    for (int q = 0; q < 4; ++q) {
+        N[q] = 0.0;
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            if (m == gp) N[q] = rule.N[m][q];
+        if (q == gp) w = rule.w[q] * Jac;
+    }
+    double u[3] = {0, 0, 0}, ud[3] = {-P.fb[0], -P.fb[1], -P.fb[2]}, pp = 0.0;
+    double ux[3][3] = {}, px[3] = {0, 0, 0};
+    double l[3] = {0, 0, 0}, lp = 0.0, Lx[3][3] = {}, Lpx[3] = {0, 0, 0};
+    double D[3] = {0, 0, 0}, Dp = 0.0, Dx[3][3] = {}, Dpx[3] = {0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const double* yq = Yg + (size_t)nd[q] * tDof;
+        const double* aq = Ag + (size_t)nd[q] * tDof;
+        const double* lq = lam + (size_t)nd[q] * 4;
+        const double* dq = du + (size_t)nd[q] * 4;
+        const double y3 = yq[3], l3 = lq[3], d3 = dq[3];
+        pp += N[q] * y3;
+        lp += N[q] * l3;
+        Dp += N[q] * d3;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            px[i] += Nx[q][i] * y3;
+            Lpx[i] += Nx[q][i] * l3;
+            Dpx[i] += Nx[q][i] * d3;
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double yc = yq[c], lc = lq[c], dc = dq[c];
+            u[c] += N[q] * yc;
+            ud[c] += N[q] * aq[c];
+            l[c] += N[q] * lc;
+            D[c] += N[q] * dc;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                ux[i][c] += Nx[q][i] * yc;
+                Lx[i][c] += Nx[q][i] * lc;
+                Dx[i][c] += Nx[q][i] * dc;
+            }
+        }
+    }
+    const double rho = P.rho;
+    const Dual mu = {muEl ? muEl[elemId[p]] : P.mu, 1.0};
+    const double divU = ux[0][0] + ux[1][1] + ux[2][2];
+    const double divL = Lx[0][0] + Lx[1][1] + Lx[2][2];
+    const double divD = Dx[0][0] + Dx[1][1] + Dx[2][2];
+    // stabilisation parameters and fine-scale velocity (fluid_gp)
+    double kS0 = 0.0, kU = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            kS0 += ks[i][j] * ks[i][j];
+            kU += u[i] * u[j] * ks[i][j];
+        }
+    const Dual kS = 36.0 * kS0 * (mu / rho) * (mu / rho);
+    const double kT = 4.0 * (1.0 / P.dt) * (1.0 / P.dt);
+    const double trK = ks[0][0] + ks[1][1] + ks[2][2];
+    const Dual tauM = 1.0 / (rho * dsqrt(kT + kU + kS));
+    const Dual tauC = 1.0 / (tauM * trK);
+    Dual up[3], ua[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const double rV = ud[c] + u[0] * ux[0][c] + u[1] * ux[1][c] + u[2] * ux[2][c];
+        up[c] = -tauM * (rho * rV + px[c]);
+        ua[c] = u[c] + up[c];
+    }
+    Dual tauB = mkd(0.0);
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) tauB = tauB + up[i] * up[j] * ks[i][j];
+    if (iszero_d(tauB.v)) tauB = mkd(2.220446049250313e-16);
+    tauB = rho / dsqrt(tauB);
+
+    const double T1c = P.af * P.gam * P.dt;
+    const double amd = P.am / T1c;
+    // lam^T K du (fluid_pair_gp's blocks summed over a and b), over w T1c
+    double mm = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) mm += Lx[i][c] * (Dx[i][c] + Dx[c][i]);
+    Dual k = mu * mm + tauC * (divL * divD) - divL * Dp + lp * divD
+           + tauM * (Lpx[0] * Dpx[0] + Lpx[1] * Dpx[1] + Lpx[2] * Dpx[2]);
+    // lam^T R: w times the gradient terms, w rho times the inertia
+    const Dual pa = pp - tauC * divU;
+    Dual r = mkd(lp * divU) - up[0] * Lpx[0] - up[1] * Lpx[1] - up[2] * Lpx[2] - pa * divL;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const double uD = u[0] * Dx[0][c] + u[1] * Dx[1][c] + u[2] * Dx[2][c];
+        const Dual upL = up[0] * Lx[0][c] + up[1] * Lx[1][c] + up[2] * Lx[2][c];
+        const Dual upD = up[0] * Dx[0][c] + up[1] * Dx[1][c] + up[2] * Dx[2][c];
+        const Dual uaL = (u[0] * Lx[0][c] + u[1] * Lx[1][c] + u[2] * Lx[2][c]) + upL;
+        const Dual upU = up[0] * ux[0][c] + up[1] * ux[1][c] + up[2] * ux[2][c];
+        const double uU = u[0] * ux[0][c] + u[1] * ux[1][c] + u[2] * ux[2][c];
+        const Dual tL = rho * tauM * uaL;
+        const double acc = rho * (amd * D[c] + uD);
+        k = k + tL * (acc + Dpx[c]) + (rho * l[c]) * (amd * D[c] + uD + upD) + tauB * upL * upD
+          + (tauM * acc) * Lpx[c];
+        // rM[i][c] = mu es - rho up_c ua_i + rVb_c up_i, contracted with Lx
+        double es = 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) es += Lx[i][c] * (ux[i][c] + ux[c][i]);
+        r = r + mu * es - rho * up[c] * uaL + tauB * upU * upL + (rho * l[c]) * (ud[c] + uU + upU);
+    }
+    double s = w * (r.d - T1c * k.d);
+    s += __shfl_xor(s, 1, 4);
+    s += __shfl_xor(s, 2, 4);
+    if (gp == 0) g[elemId[p]] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -1421,7 +1513,7 @@ int launch_fluid_dmu(const Mesh& M, const AsmParams& P, const Tet4Rule& rule, in
                      hipStream_t s)
 {
     if (M.nEl == 0) return SVFSI_OK;
-    const unsigned grid = (unsigned)(((size_t)M.nEl * 16 + 255) / 256);
+    const unsigned grid = (unsigned)(((size_t)M.nEl * 4 + 255) / 256);
     hipLaunchKernelGGL(k_fluid_dmu, dim3(grid), dim3(256), 0, s, M.nEl, M.ien.as<int>(), M.elemId.as<int>(),
                        M.x.as<double>(), tDof, Ag, Yg, muEl, P, rule, lam, du, g);
     SV_HIP(hipGetLastError());
