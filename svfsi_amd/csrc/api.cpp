@@ -707,9 +707,12 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
     M->eNoN = eNoN;
     std::vector<int> order;
     color_items(nEl, eNoN, ien.data(), nNo, order, M->colorOff);
+    // element p of the stored arrays: colour-sorted for tet10, the caller's
+    // element id for tet4, whose gather assembly reads neighbours together
+    auto elem = [&](int p) { return eNoN == 4 ? p : order[p]; };
     std::vector<int> sien((size_t)nEl * eNoN), emap((size_t)nEl * eNoN * eNoN);
     for (int p = 0; p < nEl; ++p) {
-        const int e = order[p];
+        const int e = elem(p);
         for (int a = 0; a < eNoN; ++a) sien[(size_t)p * eNoN + a] = ien[(size_t)e * eNoN + a];
         for (int a = 0; a < eNoN; ++a)
             for (int b = 0; b < eNoN; ++b) {
@@ -726,7 +729,7 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
     // gather lists, filled in element-id order
     const int NN = eNoN * eNoN;
     std::vector<int> slot(nEl);
-    for (int p = 0; p < nEl; ++p) slot[order[p]] = p;
+    for (int p = 0; p < nEl; ++p) slot[elem(p)] = p;
     std::vector<int> gptr((size_t)L.nnz + 1, 0), rptr((size_t)nNo + 1, 0);
     for (int k : emap) gptr[(size_t)k + 1]++;
     for (int nd : sien) rptr[(size_t)nd + 1]++;
@@ -740,6 +743,11 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
             for (int ab = 0; ab < NN; ++ab) gslot[(size_t)p * NN + ab] = gpos[emap[(size_t)p * NN + ab]]++;
             for (int a = 0; a < eNoN; ++a) rslot[(size_t)p * eNoN + a] = rpos[sien[(size_t)p * eNoN + a]]++;
         }
+    }
+    std::vector<int> gsrc;
+    if (eNoN == 4) {
+        gsrc.resize(gslot.size());
+        for (size_t q = 0; q < gslot.size(); ++q) gsrc[gslot[q]] = (int)q;
     }
     std::vector<double> xv(x, x + (size_t)3 * nNo);
     // mid-edge nodes (local 5..10 of a tet10), whose pressure rows
@@ -756,6 +764,7 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
     int rc = SVFSI_OK;
     if ((rc = upload(M->ien, sien)) || (rc = upload(M->elemId, order)) || (rc = upload(M->emap, emap)) ||
         (rc = upload(M->x, xv)) || (rc = upload(M->gPtr, gptr)) || (rc = upload(M->gSlot, gslot)) ||
+        (eNoN == 4 && (rc = upload(M->gSrc, gsrc))) ||
         (rc = upload(M->rPtr, rptr)) || (rc = upload(M->rSlot, rslot)) ||
         (!mids.empty() && (rc = upload(M->midNodes, mids)))) {
         delete M;
@@ -788,7 +797,7 @@ int svfsi_mesh_add_face(void* mesh, int nFe, const int* fIEN, const int* fEl, in
     SV_HIP(hipMemcpy(hien.data(), M.ien.p, hien.size() * sizeof(int), hipMemcpyDeviceToHost));
     SV_HIP(hipMemcpy(elemId.data(), M.elemId.p, elemId.size() * sizeof(int), hipMemcpyDeviceToHost));
     std::vector<int> slot(M.nEl);
-    for (int p = 0; p < M.nEl; ++p) slot[elemId[p]] = p;
+    for (int p = 0; p < M.nEl; ++p) slot[M.eNoN == 4 ? p : elemId[p]] = p;
     for (int f = 0; f < nFe; ++f) {
         for (int a = 0; a < 3; ++a) {
             fien[(size_t)f * 3 + a] = fIEN[(size_t)f * 3 + a] - 1;

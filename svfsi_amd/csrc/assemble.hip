@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_asm_lelas(int begin, int count, const i
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= count * 16) return;
-    const int p = begin + (t >> 4);
+    const int p = ke ? t >> 4 : elemId[begin + (t >> 4)];
     const int ab = t & 15;
     const int a = ab >> 2, b = ab & 3;
     int nd[4];
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void k_asm_lelas(int begin, int count, const i
     }
     double Nx[4][3], ks[3][3], Jac;
     gnn_tet4(xl, Nx, Jac, ks);
-    const double E = Eel ? Eel[elemId[p]] : P.E;
+    const double E = Eel ? Eel[p] : P.E;
     const double nu = P.nu, rho = P.rho;
     const double lambda = E * nu / (1.0 + nu) / (1.0 - 2.0 * nu);
     const double mu = E * 0.5 / (1.0 + nu);
@@ -295,8 +295,8 @@ template <typename T> struct FluidGP {
 };
 
 template <typename T>
-__device__ __forceinline__ void fluid_gp(const FluidElem& E, T mu, const AsmParams& P, const Tet4Rule& rule, int g,
-                                         FluidGP<T>& G)
+__device__ __forceinline__ void fluid_gp_n(const FluidElem& E, T mu, const AsmParams& P, const double N[4],
+                                           FluidGP<T>& G)
 {
     const double rho = P.rho;
     const double ctM = 1.0, ctC = 36.0;
@@ -313,7 +313,7 @@ __device__ __forceinline__ void fluid_gp(const FluidElem& E, T mu, const AsmPara
     double pp = 0.0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const double Nq = rule.N[g][q];
+        const double Nq = N[q];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             ud[c] += Nq * E.al[q][c];
@@ -522,6 +522,8 @@ __device__ __forceinline__ void fluid_pair_gp(const FluidElem& E, T mu, double m
     }
 }
 
+// The coloured scatter path (SVFSI_ASM_GATHER=0): 16 lanes per element, one
+// per (a,b) block, read-modify-write of Val.
 __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const int* __restrict__ ien,
                                                    const int* __restrict__ elemId,
                                                    const int* __restrict__ emap,
@@ -530,19 +532,17 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
                                                    const double* __restrict__ Yg,
                                                    const double* __restrict__ muEl, AsmParams P,
                                                    Tet4Rule rule, double* __restrict__ val,
-                                                   double* __restrict__ R, double* __restrict__ ke,
-                                                   double* __restrict__ re, const int* __restrict__ gslot,
-                                                   const int* __restrict__ rslot)
+                                                   double* __restrict__ R)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= count * 16) return;
-    const int p = begin + (t >> 4);
+    const int p = elemId[begin + (t >> 4)];
     const int ab = t & 15;
     const int a = ab >> 2, b = ab & 3;
     FluidElem E;
     fluid_elem(p, ien, x, tDof, Ag, Yg, E);
     double mu, mug;
-    fluid_visc(E, P, muEl ? muEl[elemId[p]] : P.mu, mu, mug);
+    fluid_visc(E, P, muEl ? muEl[p] : P.mu, mu, mug);
     double k[16], r[4];
     // the 16 lanes of an element (consecutive lanes of one wave; count * 16
     // threads, so a group is active or inactive as a whole) evaluate the
@@ -554,7 +554,7 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
         FluidGP<double> G;
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-            if (g == (ab & 3)) fluid_gp<double>(E, mu, P, rule, g, mine);
+            if (g == (ab & 3)) fluid_gp_n<double>(E, mu, P, rule.N[g], mine);
         (void)G;
     }
     FluidAB S;
@@ -580,17 +580,6 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
         G.tauB = __shfl(mine.tauB, src, kWave);
         fluid_pair_gp<double>(E, mu, mug, P, rule, g, G, S, b == 0, k, r);
     }
-    if (ke) {
-        double* kb = ke + (size_t)gslot[(size_t)p * 16 + ab] * 16;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) kb[q] = k[q];
-        if (b == 0) {
-            double* rr = re + (size_t)rslot[(size_t)p * 4 + a] * 4;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) rr[c] = r[c];
-        }
-        return;
-    }
     double* vb = val + (size_t)emap[(size_t)p * 16 + ab] * 16;
 #pragma unroll
     for (int q = 0; q < 16; ++q) vb[q] += k[q];
@@ -602,6 +591,259 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
 #pragma unroll
         for (int c = 0; c < 4; ++c) Rr[c] += r[c];
     }
+}
+
+// ---------------------------------------------------------------------------
+// FLUID gather assembly, two launches.
+//
+// The (a,b) block of an element, summed over its Gauss points g, needs only
+//   u-u  T_ab I + c0 Nx_b Nx_a^T + c1 Nx_a Nx_b^T
+//        (+ c4 esNx_a esNx_b^T with a shear-rate dependent viscosity)
+//   u-p  Nx_b A_a - c2 Nx_a        p-u  c2 Nx_b + B_b Nx_a
+//   p-p  c3 Nx_a.Nx_b
+// with wl_g = w_g Jac af gam dt and
+//   T_ab = sum_g wl_g [rho am/(af gam dt) N_b (N_a + rho tauM ua.Nx_a) + rho N_a ua.Nx_b
+//                      + tauB (u'.Nx_a)(u'.Nx_b) + rho^2 tauM (ua.Nx_a)(u.Nx_b)] + c0 Nx_a.Nx_b
+//   A_a = sum_g wl_g rho tauM ua.Nx_a,   B_b = sum_g wl_g tauM rho (u.Nx_b + am/(af gam dt) N_b)
+//   c0 = sum_g wl_g mu, c1 = sum_g wl_g tauC, c2 = sum_g wl_g N_b, c3 = sum_g wl_g tauM
+// (FLUID.f:494-557, 1052-1081).  k_fluid_rec evaluates these 40 numbers (56
+// with esNx) per element, four lanes each, a lane per Gauss point, the sums
+// over g by exchanges inside the quad; k_fluid_gather forms and sums the
+// blocks of each Val entry from the records of its elements.
+//
+// What bounds it: the element blocks themselves (2 KB per element) would be
+// written and read back, 810 MB on the 197,696-tet cylinder, against 320 B
+// per element of record, which the gather mostly finds in L2.  And the
+// element arithmetic: geometry and point quantities are evaluated 4 times
+// per element instead of 16, and the sum over g is taken once per element
+// instead of inside every entry.  FLUID assembly of that mesh: k_fluid_rec 45
+// us and k_fluid_gather 94 us, where the element blocks took 315 us (16 lanes
+// per element, each its block with the geometry repeated) and their gather
+// 119 + 12 us.
+// ---------------------------------------------------------------------------
+constexpr int FR_T = 0, FR_N = 16, FR_B = 32, FR_C = 36, FR_ES = 40;
+template <bool NN> struct FluidRec { static constexpr int SZ = NN ? 56 : 40; };
+
+typedef double d2_t __attribute__((ext_vector_type(2)));
+
+// v of the lane ^1 / ^2 in the same group of four lanes
+template <int X>
+__device__ __forceinline__ double quad_xor(double v)
+{
+    constexpr int ctrl = X == 1 ? 0xB1 : 0x4E; // quad_perm [1,0,3,2] / [2,3,0,1]
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// v of lane K of the group of four lanes
+template <int K>
+__device__ __forceinline__ double quad_get(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), K * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), K * 0x55, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double quad_sum(double v)
+{
+    v += quad_xor<2>(v);
+    v += quad_xor<1>(v);
+    return v;
+}
+// Sum over the four lanes of a quad of v[4][W], lane g keeping row g.
+template <int W>
+__device__ __forceinline__ void quad_rows(int g, const double (&v)[4][W], double (&o)[W])
+{
+    const bool hi = g & 2, lo = g & 1;
+    double m[2][W];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int b = 0; b < W; ++b)
+            m[i][b] = (hi ? v[2 + i][b] : v[i][b]) + quad_xor<2>(hi ? v[i][b] : v[2 + i][b]);
+#pragma unroll
+    for (int b = 0; b < W; ++b) o[b] = (lo ? m[1][b] : m[0][b]) + quad_xor<1>(lo ? m[0][b] : m[1][b]);
+}
+
+template <bool NN>
+__global__ __launch_bounds__(256) void k_fluid_rec(int nEl, const int* __restrict__ ien,
+                                                   const double* __restrict__ x, int tDof,
+                                                   const double* __restrict__ Ag, const double* __restrict__ Yg,
+                                                   const double* __restrict__ muEl, AsmParams P, Tet4Rule rule,
+                                                   double* __restrict__ rec,
+                                                   double* __restrict__ re, const int* __restrict__ rslot)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nEl * 4) return;
+    const int p = t >> 2, g = t & 3;
+    FluidElem E;
+    fluid_elem(p, ien, x, tDof, Ag, Yg, E);
+    double mu, mug;
+    fluid_visc(E, P, muEl ? muEl[p] : P.mu, mu, mug);
+    FluidGP<double> G;
+    double N[4], wg = 0.0, Nxg[3] = {0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) N[q] = 0.0;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        if (m == g) {
+            wg = rule.w[m];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) N[q] = rule.N[m][q];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) Nxg[i] = E.Nx[m][i];
+        }
+    fluid_gp_n<double>(E, mu, P, N, G);
+    const double rho = P.rho;
+    const double T1c = P.af * P.gam * P.dt;
+    const double amd = P.am / T1c;
+    const double w = wg * E.Jac;
+    const double wl = w * T1c;
+    const double tauM = G.tauM;
+    double uN[4], upN[4], uaN[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        uN[a] = G.u[0] * E.Nx[a][0] + G.u[1] * E.Nx[a][1] + G.u[2] * E.Nx[a][2];
+        upN[a] = G.up[0] * E.Nx[a][0] + G.up[1] * E.Nx[a][1] + G.up[2] * E.Nx[a][2];
+        uaN[a] = uN[a] + upN[a];
+    }
+    double v[4][6], o[6];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const double adv = rho * tauM * uaN[a];
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+            v[a][b] = wl * (rho * amd * N[b] * (N[a] + adv) + rho * N[a] * uaN[b] + G.tauB * upN[a] * upN[b]
+                            + adv * (rho * uN[b]));
+        v[a][4] = wl * adv;
+        v[a][5] = wl * tauM * (rho * uN[a] + rho * amd * N[a]);
+    }
+    quad_rows<6>(g, v, o);
+    const double W = quad_sum(wl);
+    const double c0 = W * mu, c1 = quad_sum(wl * G.tauC), c2 = quad_sum(wl * N[0]), c3 = quad_sum(wl * tauM);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+        o[b] += c0 * (Nxg[0] * E.Nx[b][0] + Nxg[1] * E.Nx[b][1] + Nxg[2] * E.Nx[b][2]);
+    double* rc = rec + (size_t)p * FluidRec<NN>::SZ;
+    *reinterpret_cast<d2_t*>(rc + FR_T + 4 * g) = d2_t{o[0], o[1]};
+    *reinterpret_cast<d2_t*>(rc + FR_T + 4 * g + 2) = d2_t{o[2], o[3]};
+    *reinterpret_cast<d2_t*>(rc + FR_N + 4 * g) = d2_t{Nxg[0], Nxg[1]};
+    *reinterpret_cast<d2_t*>(rc + FR_N + 4 * g + 2) = d2_t{Nxg[2], o[4]};
+    rc[FR_B + g] = o[5];
+    rc[FR_C + g] = g == 0 ? c0 : (g == 1 ? c1 : (g == 2 ? c2 : c3));
+    if constexpr (NN) {
+        double es[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            es[c] = (E.ux[0][c] + E.ux[c][0]) * Nxg[0] + (E.ux[1][c] + E.ux[c][1]) * Nxg[1]
+                  + (E.ux[2][c] + E.ux[c][2]) * Nxg[2];
+        *reinterpret_cast<d2_t*>(rc + FR_ES + 4 * g) = d2_t{es[0], es[1]};
+        *reinterpret_cast<d2_t*>(rc + FR_ES + 4 * g + 2) = d2_t{es[2], W * mug};
+    }
+    // residual rows (FLUID.f:429-465, 1046-1049)
+    const double ua[3] = {G.u[0] + G.up[0], G.u[1] + G.up[1], G.u[2] + G.up[2]};
+    const double pa = G.pp - G.tauC * E.divU;
+    double rV[3], rVb[3], rM[3][3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        rV[c] = G.ud[c] + ua[0] * E.ux[0][c] + ua[1] * E.ux[1][c] + ua[2] * E.ux[2][c];
+        rVb[c] = G.tauB * (G.up[0] * E.ux[0][c] + G.up[1] * E.ux[1][c] + G.up[2] * E.ux[2][c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            rM[i][c] = mu * (E.ux[i][c] + E.ux[c][i]) - rho * G.up[c] * ua[i] + rVb[c] * G.up[i]
+                     - (i == c ? pa : 0.0);
+    double rv[4][4], ro[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            rv[a][c] = w * rho * N[a] * rV[c]
+                     + w * (E.Nx[a][0] * rM[0][c] + E.Nx[a][1] * rM[1][c] + E.Nx[a][2] * rM[2][c]);
+        rv[a][3] = w * (N[a] * E.divU - upN[a]);
+    }
+    quad_rows<4>(g, rv, ro);
+    double* rr = re + (size_t)rslot[t] * 4;
+    *reinterpret_cast<d2_t*>(rr) = d2_t{ro[0], ro[1]};
+    *reinterpret_cast<d2_t*>(rr + 2) = d2_t{ro[2], ro[3]};
+}
+
+// Val(:, j) += the blocks of nnz entry j, 16 lanes per entry: lane (h, r)
+// forms row r of the contributions gPtr[j] + h, + 4, ... (gSrc[k] = 16 e +
+// 4 a + b names the k-th, in element-id order) and the four partial sums meet
+// by shuffles, in a fixed order.  Each contribution is a chain of two
+// dependent loads (gSrc, then the record) and a diagonal entry has two dozen
+// of them, so four chains run side by side, and the workgroups go in
+// XCD-contiguous order (xcd_part), since the entries of neighbouring rows
+// read the same records, which otherwise every XCD's L2 fetches: 230 us with
+// one chain per entry, hardware order and the records in colour order, 122
+// us with these.  The workgroups from nbVal on sum the R rows.  Val may be
+// only 8-byte aligned.
+template <bool NN>
+__global__ __launch_bounds__(256) void k_fluid_gather(int nnz, int nNo, unsigned nbVal, const int* __restrict__ gPtr,
+                                                      const int* __restrict__ gSrc, const double* __restrict__ rec,
+                                                      double* __restrict__ val, const int* __restrict__ rPtr,
+                                                      const double* __restrict__ re, double* __restrict__ R)
+{
+    if (blockIdx.x >= nbVal) {
+        const unsigned t = (blockIdx.x - nbVal) * 256 + threadIdx.x;
+        const int i = (int)(t >> 2), c = (int)(t & 3);
+        if (i >= nNo) return;
+        const double* src = re + (size_t)c;
+        const int k1 = rPtr[i + 1];
+        double s = 0.0;
+#pragma unroll 4
+        for (int k = rPtr[i]; k < k1; ++k) s += src[(size_t)k * 4];
+        R[(size_t)i * 4 + c] += s;
+        return;
+    }
+    const size_t t = (size_t)xcd_part(blockIdx.x, nbVal) * 256 + threadIdx.x;
+    const size_t j = t >> 4;
+    const int r = (int)(t & 3), h = (int)(t >> 2) & 3;
+    if (j >= (size_t)nnz) return; // whole groups of 16 lanes
+    const int k1 = gPtr[j + 1];
+    const bool mom = r < 3;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    for (int k = gPtr[j] + h; k < k1; k += 4) {
+        const unsigned src = (unsigned)gSrc[k];
+        const int a = (int)(src >> 2) & 3, b = (int)src & 3;
+        const double* rc = rec + (size_t)(src >> 4) * FluidRec<NN>::SZ;
+        // the four lanes of a quad load a quarter of the 112 B each and pass
+        // it on: two load instructions instead of eight (122 -> 94 us)
+        const d2_t m = *reinterpret_cast<const d2_t*>(rc + FR_N + 4 * (r < 2 ? a : b) + 2 * (r & 1));
+        const d2_a8 n = *reinterpret_cast<const d2_a8*>(
+            rc + (r == 0 ? FR_C : (r == 1 ? FR_C + 2 : (r == 2 ? FR_T + 4 * a + b : FR_B + b))));
+        const d2_t a0 = {quad_get<0>(m.x), quad_get<0>(m.y)}, a1 = {quad_get<1>(m.x), quad_get<1>(m.y)};
+        const d2_t b0 = {quad_get<2>(m.x), quad_get<2>(m.y)}, b1 = {quad_get<3>(m.x), quad_get<3>(m.y)};
+        const d2_t c01 = {quad_get<0>(n.x), quad_get<0>(n.y)}, c23 = {quad_get<1>(n.x), quad_get<1>(n.y)};
+        const double T = quad_get<2>(n.x), Bb = quad_get<3>(n.x);
+        const double ar = r == 0 ? a0.x : (r == 1 ? a0.y : a1.x);
+        const double br = r == 0 ? b0.x : (r == 1 ? b0.y : b1.x);
+        const double fx = mom ? c01.x * br : Bb;     // factor of Nx_a
+        const double fy = mom ? c01.y * ar : c23.x;  // factor of Nx_b
+        double v0 = fx * a0.x + fy * b0.x;
+        double v1 = fx * a0.y + fy * b0.y;
+        double v2 = fx * a1.x + fy * b1.x;
+        if constexpr (NN) {
+            const double ea = rc[FR_ES + 4 * a + r], eb = rc[FR_ES + 4 * b + r]; // lane 3: c4
+            const double c4 = quad_get<3>(ea); // by all four lanes, before the choice below
+            const double er = mom ? c4 * ea : 0.0;
+            v0 += er * quad_get<0>(eb);
+            v1 += er * quad_get<1>(eb);
+            v2 += er * quad_get<2>(eb);
+        }
+        s0 += v0 + (r == 0 ? T : 0.0);
+        s1 += v1 + (r == 1 ? T : 0.0);
+        s2 += v2 + (r == 2 ? T : 0.0);
+        s3 += mom ? br * a1.y - c23.x * ar : c23.y * (a0.x * b0.x + a0.y * b0.y + a1.x * b1.x);
+    }
+    // the lanes h of a row: sum over h, lane h keeps column h
+    const bool hi = h & 2, lo = h & 1;
+    const double p0 = (hi ? s2 : s0) + __shfl_xor(hi ? s0 : s2, 8, 16);
+    const double p1 = (hi ? s3 : s1) + __shfl_xor(hi ? s1 : s3, 8, 16);
+    const double q = (lo ? p1 : p0) + __shfl_xor(lo ? p0 : p1, 4, 16);
+    val[j * 16 + 4 * r + h] += q;
 }
 
 // Viscosity sensitivity of the fluid element (no reference counterpart):
@@ -617,10 +859,10 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
 // geometry and all four points in dual numbers, took 432 us on the
 // 197,696-tet cylinder; this takes about 40 us (adjoint terms of one gradient: 454 -> 96 us).
 __global__ __launch_bounds__(256) void k_fluid_dmu(int nEl, const int* __restrict__ ien,
-                                                   const int* __restrict__ elemId, const double* __restrict__ x,
-                                                   int tDof, const double* __restrict__ Ag,
-                                                   const double* __restrict__ Yg, const double* __restrict__ muEl,
-                                                   AsmParams P, Tet4Rule rule, const double* __restrict__ lam,
+                                                   const double* __restrict__ x, int tDof,
+                                                   const double* __restrict__ Ag, const double* __restrict__ Yg,
+                                                   const double* __restrict__ muEl, AsmParams P, Tet4Rule rule,
+                                                   const double* __restrict__ lam,
                                                    const double* __restrict__ du, double* __restrict__ g)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -682,7 +924,7 @@ __global__ __launch_bounds__(256) void k_fluid_dmu(int nEl, const int* __restric
         }
     }
     const double rho = P.rho;
-    const Dual mu = {muEl ? muEl[elemId[p]] : P.mu, 1.0};
+    const Dual mu = {muEl ? muEl[p] : P.mu, 1.0};
     const double divU = ux[0][0] + ux[1][1] + ux[2][2];
     const double divL = Lx[0][0] + Lx[1][1] + Lx[2][2];
     const double divD = Dx[0][0] + Dx[1][1] + Dx[2][2];
@@ -749,7 +991,7 @@ __global__ __launch_bounds__(256) void k_fluid_dmu(int nEl, const int* __restric
     double s = w * (r.d - T1c * k.d);
     s += __shfl_xor(s, 1, 4);
     s += __shfl_xor(s, 2, 4);
-    if (gp == 0) g[elemId[p]] = s;
+    if (gp == 0) g[p] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -857,7 +1099,6 @@ __global__ void k_face_backflow(int begin, int count, const int* __restrict__ or
 // never stored.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_lelas_dkde(int nEl, const int* __restrict__ ien,
-                                                    const int* __restrict__ elemId,
                                                     const double* __restrict__ x, AsmParams P,
                                                     Tet4Rule rule, const double* __restrict__ lam,
                                                     const double* __restrict__ u,
@@ -902,7 +1143,7 @@ __global__ __launch_bounds__(256) void k_lelas_dkde(int nEl, const int* __restri
                     s += la[a][i] * (wsum * v) * ub[b][j];
                 }
         }
-    g[elemId[p]] = -s;
+    g[p] = -s;
 }
 
 // ---------------------------------------------------------------------------
@@ -1441,24 +1682,43 @@ int launch_gather(Mesh& M, int dof, double* val, double* R, hipStream_t s)
     return SVFSI_OK;
 }
 
+template <bool NN>
+static int launch_fluid_rec(Mesh& M, const AsmParams& P, const Tet4Rule& rule, int tDof, const double* Ag,
+                            const double* Yg, const double* muEl, double* val, double* R, hipStream_t s)
+{
+    SV_TRY(M.ke.ensure((size_t)M.nEl * FluidRec<NN>::SZ * sizeof(double)));
+    double* rec = M.ke.as<double>();
+    double* re = M.re.as<double>();
+    hipLaunchKernelGGL(k_fluid_rec<NN>, dim3((unsigned)(((size_t)M.nEl * 4 + 255) / 256)), dim3(256), 0, s, M.nEl,
+                       M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Yg, muEl, P, rule, rec, re,
+                       M.rSlot.as<int>());
+    const int nnz = M.lhs->nnz;
+    const unsigned nbVal = (unsigned)(((size_t)nnz * 16 + 255) / 256);
+    const unsigned nbR = (unsigned)(((size_t)M.nNo * 4 + 255) / 256);
+    hipLaunchKernelGGL(k_fluid_gather<NN>, dim3(nbVal + nbR), dim3(256), 0, s, nnz, M.nNo, nbVal, M.gPtr.as<int>(),
+                       M.gSrc.as<int>(), (const double*)rec, val, M.rPtr.as<int>(), (const double*)re, R);
+    SV_HIP(hipGetLastError());
+    return SVFSI_OK;
+}
+
 int launch_asm_tet4(Mesh& M, int phys, const AsmParams& P, const Tet4Rule& rule, int tDof, const double* Ag,
                     const double* Yg, const double* Dg, const double* prop, double* val, double* R, hipStream_t s)
 {
     const int dof = phys == SVFSI_PHYS_LELAS ? 3 : 4;
     if (gather_enabled(M.eNoN)) {
-        SV_TRY(M.ke.ensure((size_t)M.nEl * 16 * dof * dof * sizeof(double)));
         SV_TRY(M.re.ensure((size_t)M.nEl * 4 * dof * sizeof(double)));
-        const unsigned grid = (unsigned)(((size_t)M.nEl * 16 + 255) / 256);
-        if (phys == SVFSI_PHYS_LELAS)
+        if (phys == SVFSI_PHYS_LELAS) {
+            SV_TRY(M.ke.ensure((size_t)M.nEl * 16 * dof * dof * sizeof(double)));
+            const unsigned grid = (unsigned)(((size_t)M.nEl * 16 + 255) / 256);
             hipLaunchKernelGGL(k_asm_lelas, dim3(grid), dim3(256), 0, s, 0, M.nEl, M.ien.as<int>(),
                                M.elemId.as<int>(), M.emap.as<int>(), M.x.as<double>(), tDof, Ag, Dg, prop, P, rule,
                                val, R, M.ke.as<double>(), M.re.as<double>(), M.gSlot.as<int>(), M.rSlot.as<int>());
-        else
-            hipLaunchKernelGGL(k_asm_fluid, dim3(grid), dim3(256), 0, s, 0, M.nEl, M.ien.as<int>(),
-                               M.elemId.as<int>(), M.emap.as<int>(), M.x.as<double>(), tDof, Ag, Yg, prop, P, rule,
-                               val, R, M.ke.as<double>(), M.re.as<double>(), M.gSlot.as<int>(), M.rSlot.as<int>());
-        SV_HIP(hipGetLastError());
-        return launch_gather(M, dof, val, R, s);
+            SV_HIP(hipGetLastError());
+            return launch_gather(M, dof, val, R, s);
+        }
+        // mu_g is zero with the constant viscosity, whose record leaves esNx out
+        if (P.viscType == SVFSI_VISC_CONST) return launch_fluid_rec<false>(M, P, rule, tDof, Ag, Yg, prop, val, R, s);
+        return launch_fluid_rec<true>(M, P, rule, tDof, Ag, Yg, prop, val, R, s);
     }
     const int nC = (int)M.colorOff.size() - 1;
     for (int c = 0; c < nC; ++c) {
@@ -1472,7 +1732,7 @@ int launch_asm_tet4(Mesh& M, int phys, const AsmParams& P, const Tet4Rule& rule,
         else
             hipLaunchKernelGGL(k_asm_fluid, dim3(grid), dim3(256), 0, s, begin, count, M.ien.as<int>(),
                                M.elemId.as<int>(), M.emap.as<int>(), M.x.as<double>(), tDof, Ag, Yg, prop,
-                               P, rule, val, R, nullptr, nullptr, nullptr, nullptr);
+                               P, rule, val, R);
     }
     SV_HIP(hipGetLastError());
     return SVFSI_OK;
@@ -1514,8 +1774,7 @@ int launch_fluid_dmu(const Mesh& M, const AsmParams& P, const Tet4Rule& rule, in
 {
     if (M.nEl == 0) return SVFSI_OK;
     const unsigned grid = (unsigned)(((size_t)M.nEl * 4 + 255) / 256);
-    hipLaunchKernelGGL(k_fluid_dmu, dim3(grid), dim3(256), 0, s, M.nEl, M.ien.as<int>(), M.elemId.as<int>(),
-                       M.x.as<double>(), tDof, Ag, Yg, muEl, P, rule, lam, du, g);
+    hipLaunchKernelGGL(k_fluid_dmu, dim3(grid), dim3(256), 0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Yg, muEl, P, rule, lam, du, g);
     SV_HIP(hipGetLastError());
     return SVFSI_OK;
 }
@@ -1525,7 +1784,7 @@ int launch_lelas_dkde(const Mesh& M, const AsmParams& P, const Tet4Rule& rule, c
 {
     if (M.nEl == 0) return SVFSI_OK;
     hipLaunchKernelGGL(k_lelas_dkde, dim3((M.nEl + 255) / 256), dim3(256), 0, s, M.nEl, M.ien.as<int>(),
-                       M.elemId.as<int>(), M.x.as<double>(), P, rule, lam, u, g);
+                       M.x.as<double>(), P, rule, lam, u, g);
     SV_HIP(hipGetLastError());
     return SVFSI_OK;
 }

@@ -20,6 +20,13 @@ __device__ __forceinline__ int xcd_block(int on)
     return (int)(x * q + (x < r ? x : r) + j);
 }
 
+// The same for the first nb blocks of a grid (block b of them).
+__device__ __forceinline__ unsigned xcd_part(unsigned b, unsigned nb)
+{
+    const unsigned q = nb >> 3, r = nb & 7u, x = b & 7u, j = b >> 3;
+    return x * q + (x < r ? x : r) + j;
+}
+
 // Sum over the 64 lanes of a wavefront (butterfly; every lane gets the sum).
 __device__ __forceinline__ double wave_sum(double v)
 {

@@ -186,9 +186,9 @@ struct Mesh {
     Lhs* lhs = nullptr;
     int nNo = 0, nEl = 0, eNoN = 0;
     DBuf x;          // (3, nNo)
-    DBuf ien;        // (eNoN, nEl) colour-sorted, 0-based
-    DBuf elemId;     // original element id of each colour-sorted slot
-    DBuf emap;       // (eNoN*eNoN, nEl) colour-sorted nnz index of block (a,b)
+    DBuf ien;        // (eNoN, nEl) 0-based; tet10 colour-sorted, tet4 in element-id order
+    DBuf elemId;     // original element id of each position of the colour-sorted list
+    DBuf emap;       // (eNoN*eNoN, nEl) nnz index of block (a,b), elements as in ien
     std::vector<int> colorOff; // nColors+1 offsets into the colour-sorted list
     struct FaceSet {
         int nFe = 0;
@@ -211,8 +211,10 @@ struct Mesh {
     // block j are ke positions gPtr[j] .. gPtr[j+1]-1, in element-id order
     // (the order of DOASSEM's element loop); likewise element row (p, a) at
     // rSlot[p*eNoN + a] of re, node i's rows at rPtr[i] .. rPtr[i+1]-1.
-    DBuf gPtr, gSlot, rPtr, rSlot;
-    DBuf ke, re;     // element blocks / element residual rows, grown on demand
+    // gSrc is gSlot's inverse: position k of ke holds block gSrc[k] =
+    // p*eNoN^2 + a*eNoN + b (tet4: the gather forms the blocks from records).
+    DBuf gPtr, gSlot, gSrc, rPtr, rSlot;
+    DBuf ke, re;     // element blocks or records / element residual rows, grown on demand
     ~Mesh() {
         for (auto* f : faceSets) delete f;
     }

@@ -57,3 +57,33 @@ def test_fluid_dmu_sizes(gpu, orc, nEl, tDof, uniform):
     st.dmesh.fluid_dmu_dot(prob.eq, st.Ag, st.Yg, st.prop, dl, dd, g)
     go = orc.fluid_dmu_dot(prob, lam, du)
     assert np.abs(g.cpu().numpy() - go).max() <= 1e-12 * np.abs(go).max()
+
+
+def assembled(prob, orc):
+    import torch
+
+    from svfsi_amd.step import NewtonStep
+
+    st = NewtonStep(prob)
+    # the element loop accumulates into what is there
+    V0 = torch.rand_like(st.Val)
+    R0 = torch.rand_like(st.R)
+    st.Val.copy_(V0)
+    st.R.copy_(R0)
+    st.dmesh.assemble(prob.phys, prob.eq, st.Ag, st.Yg, st.Dg, st.Val, st.R, prop_el=st.prop, quad=prob.quad)
+    Vo, Ro = orc.assemble(prob, st.rowPtr - 1, st.colPtr - 1)
+    return [(a.cpu().numpy() - b.cpu().numpy(), c) for a, b, c in ((st.Val, V0, Vo), (st.R, R0, Ro))]
+
+
+VISC = {"const": {}, "cy": dict(viscType=697, mu=0.035, mu_o=0.56, lam=3.313, visc_a=2.0, visc_n=0.3568),
+        "cass": dict(viscType=696, mu=0.2, mu_o=0.3, lam=0.5)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", list(VISC))
+@pytest.mark.parametrize("nEl,tDof,uniform", [(1, 4, True), (13, 7, False), (65, 4, False), (130, 5, True)])
+def test_fluid_assembly_sizes(gpu, orc, nEl, tDof, uniform, model):
+    prob = fluid_case(nEl, tDof, uniform)
+    prob.eq = dict(prob.eq, fb=(0.3, -0.2, 0.1), **VISC[model])
+    for got, want in assembled(prob, orc):
+        assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * max(1.0, np.abs(want).max())
