@@ -227,6 +227,25 @@ static void color_items(int nItems, int nPer, const int* conn, int nNo, std::vec
     for (int e = 0; e < nItems; ++e) order[pos[col[e]]++] = e;
 }
 
+// Groups the positions of key by value: dst the distinct values, ascending,
+// src[ptr[i] .. ptr[i+1]) the positions where key = dst[i], ascending.
+static void group_by(const std::vector<int>& key, std::vector<int>& ptr, std::vector<int>& src,
+                     std::vector<int>& dst)
+{
+    src.resize(key.size());
+    for (size_t q = 0; q < key.size(); ++q) src[q] = (int)q;
+    std::stable_sort(src.begin(), src.end(), [&](int u, int v) { return key[u] < key[v]; });
+    ptr.assign(1, 0);
+    dst.clear();
+    for (size_t q = 0; q < src.size(); ++q) {
+        if (q == 0 || key[src[q]] != dst.back()) {
+            if (q) ptr.push_back((int)q);
+            dst.push_back(key[src[q]]);
+        }
+    }
+    if (!src.empty()) ptr.push_back((int)src.size());
+}
+
 static int find_block(const Lhs& L, int row, int col)
 {
     const int* cp = L.hColPtr.data();
@@ -824,11 +843,15 @@ int svfsi_mesh_add_face(void* mesh, int nFe, const int* fIEN, const int* fEl, in
     }
     auto* F = new Mesh::FaceSet();
     F->nFe = nFe;
-    std::vector<int> order;
-    color_items(nFe, 3, fien.data(), M.nNo, order, F->colorOff);
+    std::vector<int> np, ns, nd, bp, bs, bd;
+    group_by(fien, np, ns, nd);
+    group_by(fmap, bp, bs, bd);
+    F->nNodes = (int)nd.size();
+    F->nBlk = (int)bd.size();
     int rc = SVFSI_OK;
-    if ((rc = upload(F->fien, fien)) || (rc = upload(F->fel, fel)) || (rc = upload(F->inner, inner)) ||
-        (rc = upload(F->fmap, fmap)) || (rc = upload(F->order, order))) {
+    if ((rc = upload(F->fien, fien)) || (rc = upload(F->inner, inner)) || (rc = upload(F->nPtr, np)) ||
+        (rc = upload(F->nSrc, ns)) || (rc = upload(F->nDst, nd)) || (rc = upload(F->bPtr, bp)) ||
+        (rc = upload(F->bSrc, bs)) || (rc = upload(F->bDst, bd))) {
         delete F;
         return rc;
     }
@@ -840,12 +863,11 @@ int svfsi_mesh_add_face(void* mesh, int nFe, const int* fIEN, const int* fEl, in
 int svfsi_zero_dev(void* mesh, int dof, double* dVal, double* dR, void* stream)
 {
     SV_ARG(mesh && dVal && dR, "NULL argument");
+    SV_ARG(dof >= 0, "dof < 0");
     SV_TRY(require_device());
     Mesh& M = *static_cast<Mesh*>(mesh);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    SV_HIP(hipMemsetAsync(dVal, 0, (size_t)M.lhs->nnz * dof * dof * sizeof(double), s));
-    SV_HIP(hipMemsetAsync(dR, 0, (size_t)M.nNo * dof * sizeof(double), s));
-    return SVFSI_OK;
+    return launch_zero2((size_t)M.lhs->nnz * dof * dof, dVal, (size_t)M.nNo * dof, dR, s);
 }
 
 int svfsi_assemble_dev(void* mesh, int phys, const svfsi_eq_params* p, int tDof, const double* dAg,

@@ -1017,78 +1017,144 @@ __device__ __forceinline__ void gnnb_tri3(const double* x, int n0, int n1, int n
     }
 }
 
-// SETBCTRACL (svFSI/SETBC.f:319-416): lR(:,a) -= w N_a h ; one thread per
-// (face, a).
-__global__ void k_face_traction(int begin, int count, const int* __restrict__ order,
-                                const int* __restrict__ fien, const int* __restrict__ inner,
-                                const double* __restrict__ x, int dof, double h0, double h1,
-                                double h2, Tri3Rule rule, double* __restrict__ R)
+// The face terms are gathered like the elements': eight lanes per node (or
+// Val block) share its faces, in face order, and meet by shuffles, so a face
+// set is one launch whatever its colouring (FaceSet::nPtr, bPtr).  At these
+// sizes (a few hundred faces) a launch is all there is to time: one per
+// colour took 7 x 1.9 us (36 faces) to 10 x 4.8 us (the outlet of the
+// 197,696-tet cylinder), one for the whole set 4-5 us.
+constexpr int kFaceLanes = 8;
+
+__device__ __forceinline__ double face_lanes_sum(double v)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count * 3) return;
-    const int f = order[begin + t / 3];
-    const int a = t % 3;
-    const int n0 = fien[f * 3], n1 = fien[f * 3 + 1], n2 = fien[f * 3 + 2];
-    double n[3];
-    gnnb_tri3(x, n0, n1, n2, inner[f], n);
-    const double Jac = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
-    const double h[3] = {h0, h1, h2};
-    double r[3] = {0, 0, 0};
 #pragma unroll
-    for (int g = 0; g < 3; ++g) {
-        const double w = rule.w[g] * Jac;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) r[i] -= w * rule.N[g][a] * h[i];
-    }
-    const int node = fien[f * 3 + a];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) R[(size_t)node * dof + i] += r[i];
+    for (int o = kFaceLanes / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kFaceLanes);
+    return v;
 }
 
-// BFLUID with h = 0 (svFSI/FLUID.f:1280-1336); one thread per (face, a, b).
-__global__ void k_face_backflow(int begin, int count, const int* __restrict__ order,
-                                const int* __restrict__ fien, const int* __restrict__ inner,
-                                const int* __restrict__ fmap, const double* __restrict__ x,
-                                int tDof, const double* __restrict__ Yg, AsmParams P,
-                                Tri3Rule rule, double* __restrict__ val, double* __restrict__ R)
+// SETBCTRACL (svFSI/SETBC.f:319-416): lR(:,a) -= w N_a h.
+__global__ __launch_bounds__(256) void k_face_traction(int nNodes, const int* __restrict__ nPtr,
+                                                       const int* __restrict__ nSrc, const int* __restrict__ nDst,
+                                                       const int* __restrict__ fien, const int* __restrict__ inner,
+                                                       const double* __restrict__ x, int dof, double h0, double h1,
+                                                       double h2, Tri3Rule rule, double* __restrict__ R)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count * 9) return;
-    const int f = order[begin + t / 9];
-    const int ab = t % 9;
-    const int a = ab / 3, b = ab % 3;
-    const int nd[3] = {fien[f * 3], fien[f * 3 + 1], fien[f * 3 + 2]};
-    double n[3];
-    gnnb_tri3(x, nd[0], nd[1], nd[2], inner[f], n);
-    const double Jac = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
-    const double nV[3] = {n[0] / Jac, n[1] / Jac, n[2] / Jac};
-    double kd = 0.0;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int i = t / kFaceLanes, l = t % kFaceLanes;
+    if (i >= nNodes) return; // whole groups
+    const double h[3] = {h0, h1, h2};
     double r[3] = {0, 0, 0};
+    for (int k = nPtr[i] + l; k < nPtr[i + 1]; k += kFaceLanes) {
+        const int f = nSrc[k] / 3, a = nSrc[k] % 3;
+        double n[3];
+        gnnb_tri3(x, fien[f * 3], fien[f * 3 + 1], fien[f * 3 + 2], inner[f], n);
+        const double Jac = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
 #pragma unroll
-    for (int g = 0; g < 3; ++g) {
-        const double w = rule.w[g] * Jac;
-        double y[3] = {0, 0, 0};
+        for (int g = 0; g < 3; ++g) {
+            const double w = rule.w[g] * Jac;
+            const double Na = a == 0 ? rule.N[g][0] : (a == 1 ? rule.N[g][1] : rule.N[g][2]);
 #pragma unroll
-        for (int q = 0; q < 3; ++q)
-#pragma unroll
-            for (int i = 0; i < 3; ++i) y[i] += rule.N[g][q] * Yg[(size_t)nd[q] * tDof + i];
-        const double wl = w * P.af * P.gam * P.dt;
-        double udn = y[0] * nV[0] + y[1] * nV[1] + y[2] * nV[2];
-        udn = 0.5 * P.bstab * P.rho * (udn - fabs(udn));
-        kd -= wl * rule.N[g][a] * rule.N[g][b] * udn;
-        if (b == 0) {
-#pragma unroll
-            for (int i = 0; i < 3; ++i) r[i] -= w * rule.N[g][a] * (udn * y[i]);
+            for (int c = 0; c < 3; ++c) r[c] -= w * Na * h[c];
         }
     }
-    double* vb = val + (size_t)fmap[f * 9 + ab] * 16;
-    vb[0] += kd;
-    vb[5] += kd;
-    vb[10] += kd;
-    if (b == 0) {
+    double* Rr = R + (size_t)nDst[i] * dof;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) R[(size_t)nd[a] * 4 + i] += r[i];
+    for (int c = 0; c < 3; ++c) {
+        const double s = face_lanes_sum(r[c]);
+        if (l == c) Rr[c] += s;
     }
+}
+
+// BFLUID with h = 0 (svFSI/FLUID.f:1280-1336): the nBlk Val blocks of the
+// face set first, then its nodes' rows of R.
+__global__ __launch_bounds__(256) void k_face_backflow(int nBlk, const int* __restrict__ bPtr,
+                                                       const int* __restrict__ bSrc, const int* __restrict__ bDst,
+                                                       int nNodes, const int* __restrict__ nPtr,
+                                                       const int* __restrict__ nSrc, const int* __restrict__ nDst,
+                                                       const int* __restrict__ fien, const int* __restrict__ inner,
+                                                       const double* __restrict__ x, int tDof,
+                                                       const double* __restrict__ Yg, AsmParams P, Tri3Rule rule,
+                                                       double* __restrict__ val, double* __restrict__ R)
+{
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    const int item = t / kFaceLanes, l = t % kFaceLanes;
+    if (item >= nBlk + nNodes) return; // whole groups
+    const bool blk = item < nBlk;
+    const int i = blk ? item : item - nBlk;
+    const int* ptr = blk ? bPtr : nPtr;
+    const int* src = blk ? bSrc : nSrc;
+    double s[3] = {0, 0, 0}; // a block's diagonal in s[0], or a node's three rows
+    for (int k = ptr[i] + l; k < ptr[i + 1]; k += kFaceLanes) {
+        const int q = src[k];
+        const int f = blk ? q / 9 : q / 3;
+        const int a = blk ? (q % 9) / 3 : q % 3, b = q % 3;
+        const int nd[3] = {fien[f * 3], fien[f * 3 + 1], fien[f * 3 + 2]};
+        double n[3];
+        gnnb_tri3(x, nd[0], nd[1], nd[2], inner[f], n);
+        const double Jac = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+        const double nV[3] = {n[0] / Jac, n[1] / Jac, n[2] / Jac};
+#pragma unroll
+        for (int g = 0; g < 3; ++g) {
+            const double w = rule.w[g] * Jac;
+            double y[3] = {0, 0, 0};
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) y[c] += rule.N[g][m] * Yg[(size_t)nd[m] * tDof + c];
+            const double wl = w * P.af * P.gam * P.dt;
+            double udn = y[0] * nV[0] + y[1] * nV[1] + y[2] * nV[2];
+            udn = 0.5 * P.bstab * P.rho * (udn - fabs(udn));
+            const double Na = a == 0 ? rule.N[g][0] : (a == 1 ? rule.N[g][1] : rule.N[g][2]);
+            const double Nb = b == 0 ? rule.N[g][0] : (b == 1 ? rule.N[g][1] : rule.N[g][2]);
+            if (blk) {
+                s[0] -= wl * Na * Nb * udn;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) s[c] -= w * Na * (udn * y[c]);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) s[c] = face_lanes_sum(s[c]);
+    if (l >= 3) return;
+    if (blk)
+        val[(size_t)bDst[i] * 16 + 5 * l] += s[0];
+    else
+        R[(size_t)nDst[i] * 4 + l] += l == 0 ? s[0] : (l == 1 ? s[1] : s[2]);
+}
+
+// LSALLOC's zeroing of both arrays in one launch (16-byte stores where the
+// arrays allow).
+template <bool V>
+__global__ __launch_bounds__(256) void k_zero2(size_t n1, double* __restrict__ a, size_t n2, double* __restrict__ b,
+                                               unsigned nb1)
+{
+    const bool first = blockIdx.x < nb1;
+    double* p = first ? a : b;
+    const size_t n = first ? n1 : n2;
+    const size_t q0 = (size_t)(first ? blockIdx.x : blockIdx.x - nb1) * 2048 + (size_t)threadIdx.x * (V ? 2 : 1);
+#pragma unroll
+    for (int m = 0; m < (V ? 4 : 8); ++m) {
+        const size_t q = q0 + (size_t)m * (V ? 512 : 256);
+        if constexpr (V) {
+            if (q + 1 < n) *reinterpret_cast<d2_t*>(p + q) = d2_t{0.0, 0.0};
+            else if (q < n) p[q] = 0.0;
+        } else {
+            if (q < n) p[q] = 0.0;
+        }
+    }
+}
+
+int launch_zero2(size_t n1, double* a, size_t n2, double* b, hipStream_t s)
+{
+    const unsigned nb1 = (unsigned)((n1 + 2047) / 2048), nb2 = (unsigned)((n2 + 2047) / 2048);
+    if (nb1 + nb2 == 0) return SVFSI_OK;
+    if ((((uintptr_t)a | (uintptr_t)b) & 15) == 0)
+        hipLaunchKernelGGL(k_zero2<true>, dim3(nb1 + nb2), dim3(256), 0, s, n1, a, n2, b, nb1);
+    else
+        hipLaunchKernelGGL(k_zero2<false>, dim3(nb1 + nb2), dim3(256), 0, s, n1, a, n2, b, nb1);
+    SV_HIP(hipGetLastError());
+    return SVFSI_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1738,17 +1804,15 @@ int launch_asm_tet4(Mesh& M, int phys, const AsmParams& P, const Tet4Rule& rule,
     return SVFSI_OK;
 }
 
+static dim3 face_grid(int items) { return dim3((unsigned)(((size_t)items * kFaceLanes + 255) / 256)); }
+
 int launch_face_traction(const Mesh& M, const Mesh::FaceSet& F, int dof, const double* h,
                          const Tri3Rule& rule, double* R, hipStream_t s)
 {
-    const int nC = (int)F.colorOff.size() - 1;
-    for (int c = 0; c < nC; ++c) {
-        const int begin = F.colorOff[c], count = F.colorOff[c + 1] - begin;
-        if (count == 0) continue;
-        hipLaunchKernelGGL(k_face_traction, dim3((count * 3 + 255) / 256), dim3(256), 0, s, begin, count,
-                           F.order.as<int>(), F.fien.as<int>(), F.inner.as<int>(), M.x.as<double>(), dof,
-                           h[0], h[1], h[2], rule, R);
-    }
+    if (F.nNodes == 0) return SVFSI_OK;
+    hipLaunchKernelGGL(k_face_traction, face_grid(F.nNodes), dim3(256), 0, s, F.nNodes, F.nPtr.as<int>(),
+                       F.nSrc.as<int>(), F.nDst.as<int>(), F.fien.as<int>(), F.inner.as<int>(), M.x.as<double>(), dof,
+                       h[0], h[1], h[2], rule, R);
     SV_HIP(hipGetLastError());
     return SVFSI_OK;
 }
@@ -1756,14 +1820,11 @@ int launch_face_traction(const Mesh& M, const Mesh::FaceSet& F, int dof, const d
 int launch_face_backflow(const Mesh& M, const Mesh::FaceSet& F, const AsmParams& P, int tDof,
                          const double* Yg, const Tri3Rule& rule, double* val, double* R, hipStream_t s)
 {
-    const int nC = (int)F.colorOff.size() - 1;
-    for (int c = 0; c < nC; ++c) {
-        const int begin = F.colorOff[c], count = F.colorOff[c + 1] - begin;
-        if (count == 0) continue;
-        hipLaunchKernelGGL(k_face_backflow, dim3((count * 9 + 255) / 256), dim3(256), 0, s, begin, count,
-                           F.order.as<int>(), F.fien.as<int>(), F.inner.as<int>(), F.fmap.as<int>(),
-                           M.x.as<double>(), tDof, Yg, P, rule, val, R);
-    }
+    if (F.nNodes == 0) return SVFSI_OK;
+    hipLaunchKernelGGL(k_face_backflow, face_grid(F.nBlk + F.nNodes), dim3(256), 0, s, F.nBlk, F.bPtr.as<int>(),
+                       F.bSrc.as<int>(), F.bDst.as<int>(), F.nNodes, F.nPtr.as<int>(), F.nSrc.as<int>(),
+                       F.nDst.as<int>(), F.fien.as<int>(), F.inner.as<int>(), M.x.as<double>(), tDof, Yg, P, rule,
+                       val, R);
     SV_HIP(hipGetLastError());
     return SVFSI_OK;
 }

@@ -39,6 +39,8 @@ AsmParams to_asm(const svfsi_eq_params& p);
 int launch_asm_tet4(Mesh& M, int phys, const AsmParams& P, const Tet4Rule& rule, int tDof,
                     const double* Ag, const double* Yg, const double* Dg, const double* prop,
                     double* val, double* R, hipStream_t s);
+// zeroes a[0..n1) and b[0..n2)
+int launch_zero2(size_t n1, double* a, size_t n2, double* b, hipStream_t s);
 int launch_face_traction(const Mesh& M, const Mesh::FaceSet& F, int dof, const double* h,
                          const Tri3Rule& rule, double* R, hipStream_t s);
 int launch_face_backflow(const Mesh& M, const Mesh::FaceSet& F, const AsmParams& P, int tDof,

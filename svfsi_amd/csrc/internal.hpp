@@ -190,14 +190,15 @@ struct Mesh {
     DBuf elemId;     // original element id of each position of the colour-sorted list
     DBuf emap;       // (eNoN*eNoN, nEl) nnz index of block (a,b), elements as in ien
     std::vector<int> colorOff; // nColors+1 offsets into the colour-sorted list
+    // Faces with the lists their gathers read: node i's contributions are
+    // nSrc[k] = 3 f + a, k = nPtr[i] .. nPtr[i+1]-1, in face order, for row
+    // nDst[i] of R; likewise block i's bSrc[k] = 9 f + 3 a + b for block
+    // bDst[i] of Val.
     struct FaceSet {
-        int nFe = 0;
+        int nFe = 0, nNodes = 0, nBlk = 0;
         DBuf fien;   // (3, nFe) 0-based
-        DBuf fel;    // (nFe) 0-based volume element
         DBuf inner;  // (nFe) first element node not on the face
-        std::vector<int> colorOff;
-        DBuf fmap;   // (9, nFe) nnz index of face block (a,b)
-        DBuf order;  // colour-sorted face ids
+        DBuf nPtr, nSrc, nDst, bPtr, bSrc, bDst;
     };
     std::vector<FaceSet*> faceSets;
     DBuf rule10[2];  // TET10 quadrature tables (15-point, 4-point), built on first use

@@ -87,3 +87,45 @@ def test_fluid_assembly_sizes(gpu, orc, nEl, tDof, uniform, model):
     prob.eq = dict(prob.eq, fb=(0.3, -0.2, 0.1), **VISC[model])
     for got, want in assembled(prob, orc):
         assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,size", [("lelas", 1), ("lelas", 5), ("fluid", 0.45), ("fluid", 0.2)])
+def test_face_terms_sizes(gpu, orc, kind, size):
+    """Two faces, a handful to several hundred faces, nodes of up to eight faces, one launch each."""
+    prob = problems.lelas_cube(size) if kind == "lelas" else problems.fluid_cylinder(h=size)
+    import torch
+
+    from svfsi_amd.step import NewtonStep
+
+    st = NewtonStep(prob)
+    rng = np.random.default_rng(1)
+    st.Yg.copy_(torch.from_numpy(rng.normal(size=prob.Yg.shape)))
+    prob.Yg = st.Yg.cpu().numpy()
+    st.assemble()
+    got = st.Val.cpu().numpy(), st.R.cpu().numpy()
+    want = orc.assemble(prob, st.rowPtr - 1, st.colPtr - 1)
+    for a, b in zip(got, want):
+        assert np.abs(a - b.reshape(a.shape)).max() <= 1e-12 * np.abs(b).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nEl,shift", [(1, 0), (13, 1), (130, 1), (1200, 0)])
+def test_zero_sizes(gpu, nEl, shift):
+    """Val and R cleared to their ends and no further, on 16- and 8-byte boundaries."""
+    import torch
+
+    from svfsi_amd import fsils
+    from svfsi_amd.assembly import DeviceMesh
+
+    prob = fluid_case(nEl, 4, True)
+    rowPtr, colPtr = fsils.lhsa(prob.nNo, prob.mesh.ien)
+    lhs = fsils.fsils_lhs_create(prob.nNo, len(colPtr), rowPtr, colPtr)
+    dm = DeviceMesh(lhs, prob.mesh)
+    for dof in (3, 4):
+        nV, nR = len(colPtr) * dof * dof, prob.nNo * dof
+        V, R = (torch.ones(n + 4, dtype=torch.float64, device=gpu) for n in (nV, nR))
+        dm.zero(dof, V[shift:shift + nV], R[shift:shift + nR])
+        for t, n in ((V, nV), (R, nR)):
+            assert t[shift:shift + n].abs().max().item() == 0.0
+            assert t[:shift].eq(1).all() and t[shift + n:].eq(1).all()
