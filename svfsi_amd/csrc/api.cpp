@@ -782,8 +782,7 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
     M->nMid = (int)mids.size();
     int rc = SVFSI_OK;
     if ((rc = upload(M->ien, sien)) || (rc = upload(M->elemId, order)) || (rc = upload(M->emap, emap)) ||
-        (rc = upload(M->x, xv)) || (rc = upload(M->gPtr, gptr)) || (rc = upload(M->gSlot, gslot)) ||
-        (eNoN == 4 && (rc = upload(M->gSrc, gsrc))) ||
+        (rc = upload(M->x, xv)) || (rc = upload(M->gPtr, gptr)) || (rc = eNoN == 4 ? upload(M->gSrc, gsrc) : upload(M->gSlot, gslot)) ||
         (rc = upload(M->rPtr, rptr)) || (rc = upload(M->rSlot, rslot)) ||
         (!mids.empty() && (rc = upload(M->midNodes, mids)))) {
         delete M;

@@ -67,9 +67,35 @@ __device__ __forceinline__ void gnn_tet4(const double xl[4][3], double Nx[4][3],
     Jac = J;
 }
 
+typedef double d2_t __attribute__((ext_vector_type(2)));
+
+// v of the lane ^1 / ^2 in the same group of four lanes
+template <int X>
+__device__ __forceinline__ double quad_xor(double v)
+{
+    constexpr int ctrl = X == 1 ? 0xB1 : 0x4E; // quad_perm [1,0,3,2] / [2,3,0,1]
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// v of lane K of the group of four lanes
+template <int K>
+__device__ __forceinline__ double quad_get(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), K * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), K * 0x55, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double quad_sum(double v)
+{
+    v += quad_xor<2>(v);
+    v += quad_xor<1>(v);
+    return v;
+}
 // ---------------------------------------------------------------------------
 // LELAS3D (svFSI/LELAS.f:130-242) in CONSTRUCT_LELAS (LELAS.f:38-128), tet4.
 // ---------------------------------------------------------------------------
+// The coloured scatter path (SVFSI_ASM_GATHER=0).
 __global__ __launch_bounds__(256) void k_asm_lelas(int begin, int count, const int* __restrict__ ien,
                                                    const int* __restrict__ elemId,
                                                    const int* __restrict__ emap,
@@ -78,13 +104,11 @@ __global__ __launch_bounds__(256) void k_asm_lelas(int begin, int count, const i
                                                    const double* __restrict__ Dg,
                                                    const double* __restrict__ Eel, AsmParams P,
                                                    Tet4Rule rule, double* __restrict__ val,
-                                                   double* __restrict__ R, double* __restrict__ ke,
-                                                   double* __restrict__ re, const int* __restrict__ gslot,
-                                                   const int* __restrict__ rslot)
+                                                   double* __restrict__ R)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= count * 16) return;
-    const int p = ke ? t >> 4 : elemId[begin + (t >> 4)];
+    const int p = elemId[begin + (t >> 4)];
     const int ab = t & 15;
     const int a = ab >> 2, b = ab & 3;
     int nd[4];
@@ -120,15 +144,9 @@ __global__ __launch_bounds__(256) void k_asm_lelas(int begin, int count, const i
                 k[i * 3 + j] += wl * v;
             }
     }
-    if (ke) {
-        double* kb = ke + (size_t)gslot[(size_t)p * 16 + ab] * 9;
+    double* vb = val + (size_t)emap[(size_t)p * 16 + ab] * 9;
 #pragma unroll
-        for (int q = 0; q < 9; ++q) kb[q] = k[q];
-    } else {
-        double* vb = val + (size_t)emap[(size_t)p * 16 + ab] * 9;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) vb[q] += k[q];
-    }
+    for (int q = 0; q < 9; ++q) vb[q] += k[q];
 
     if (b != 0) return;
     // residual row a (LELAS.f:161-205 and 208-215)
@@ -167,17 +185,151 @@ __global__ __launch_bounds__(256) void k_asm_lelas(int begin, int count, const i
         r[1] += w * (rho * Na * ud[1] + Nx[a][0] * S[3] + Nx[a][1] * S[1] + Nx[a][2] * S[4]);
         r[2] += w * (rho * Na * ud[2] + Nx[a][0] * S[5] + Nx[a][1] * S[4] + Nx[a][2] * S[2]);
     }
-    if (re) {
-        double* rr = re + (size_t)rslot[(size_t)p * 4 + a] * 3;
-        rr[0] = r[0];
-        rr[1] = r[1];
-        rr[2] = r[2];
-        return;
-    }
     double* Rr = R + (size_t)ien[(size_t)p * 4 + a] * 3;
     Rr[0] += r[0];
     Rr[1] += r[1];
     Rr[2] += r[2];
+}
+
+// ---------------------------------------------------------------------------
+// LELAS gather assembly, two launches (the scheme of the fluid's records
+// below).  Summed over the Gauss points, the (a,b) block of an element is
+//   c0 Nx_a Nx_b^T + c1 Nx_b Nx_a^T + (c1 Nx_a.Nx_b + m_ab) I
+// with c0 = V af beta dt^2 lambda, c1 = V af beta dt^2 mu and the consistent
+// mass m_ab = am rho Jac sum_g w_g N_a N_b, which takes one value on the
+// diagonal (c2) and one off it (c3): 16 numbers, one 128-byte line, against
+// 1152 bytes of element blocks.  On the 215,622-tet cube the element kernel
+// takes 22 us and the gather 90, against 195 us for 16 lanes per element
+// storing their blocks and 81 + 8 us for summing those.
+// ---------------------------------------------------------------------------
+constexpr int LR_C = 12, LR_SZ = 16;
+
+// Four lanes per element: lane a reads node a and forms row a of the
+// residual (LELAS.f:161-215).
+__global__ __launch_bounds__(256) void k_lelas_rec(int nEl, const int* __restrict__ ien, const double* __restrict__ x,
+                                                   int tDof, const double* __restrict__ Ag,
+                                                   const double* __restrict__ Dg, const double* __restrict__ Eel,
+                                                   AsmParams P, Tet4Rule rule, double* __restrict__ rec,
+                                                   double* __restrict__ re, const int* __restrict__ rslot)
+{
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= nEl * 4) return; // whole quads
+    const int p = t >> 2, a = t & 3;
+    const int nd = ien[t];
+    double xa[3], Da[3], Aa[3], xl[4][3], D[4][3], As[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        xa[i] = x[(size_t)nd * 3 + i];
+        Da[i] = Dg[(size_t)nd * tDof + i];
+        Aa[i] = Ag[(size_t)nd * tDof + i];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        xl[0][i] = quad_get<0>(xa[i]);
+        xl[1][i] = quad_get<1>(xa[i]);
+        xl[2][i] = quad_get<2>(xa[i]);
+        xl[3][i] = quad_get<3>(xa[i]);
+        D[0][i] = quad_get<0>(Da[i]);
+        D[1][i] = quad_get<1>(Da[i]);
+        D[2][i] = quad_get<2>(Da[i]);
+        D[3][i] = quad_get<3>(Da[i]);
+        As[i] = quad_sum(Aa[i]);
+    }
+    double Nx[4][3], ks[3][3], Jac;
+    gnn_tet4(xl, Nx, Jac, ks);
+    double Nxa[3] = {0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (q == a) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) Nxa[i] = Nx[q][i];
+        }
+    const double E = Eel ? Eel[p] : P.E;
+    const double nu = P.nu, rho = P.rho;
+    const double lambda = E * nu / (1.0 + nu) / (1.0 - 2.0 * nu);
+    const double mu = E * 0.5 / (1.0 + nu);
+    const double T1 = P.af * P.beta * P.dt * P.dt;
+    // sum_g w_g, w_g N_a, w_g N_a^2 and w_g N_a N_b (a symmetric rule)
+    double w0 = 0.0, w1 = 0.0, md = 0.0, mo = 0.0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        w0 += rule.w[g];
+        w1 += rule.w[g] * rule.N[g][0];
+        md += rule.w[g] * rule.N[g][0] * rule.N[g][0];
+        mo += rule.w[g] * rule.N[g][0] * rule.N[g][1];
+    }
+    const double V = w0 * Jac;
+    const double c = a == 0 ? V * T1 * lambda : (a == 1 ? V * T1 * mu : P.am * rho * Jac * (a == 2 ? md : mo));
+    double* rc = rec + (size_t)p * LR_SZ;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rc[3 * a + i] = Nxa[i];
+    rc[LR_C + a] = c;
+    double ed[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        ed[0] += Nx[q][0] * D[q][0];
+        ed[1] += Nx[q][1] * D[q][1];
+        ed[2] += Nx[q][2] * D[q][2];
+        ed[3] += Nx[q][1] * D[q][0] + Nx[q][0] * D[q][1];
+        ed[4] += Nx[q][2] * D[q][1] + Nx[q][1] * D[q][2];
+        ed[5] += Nx[q][0] * D[q][2] + Nx[q][2] * D[q][0];
+    }
+    const double divD = lambda * (ed[0] + ed[1] + ed[2]);
+    const double S0 = divD + 2.0 * mu * ed[0], S1 = divD + 2.0 * mu * ed[1], S2 = divD + 2.0 * mu * ed[2];
+    const double S3 = mu * ed[3], S4 = mu * ed[4], S5 = mu * ed[5];
+    const double rJ = rho * Jac;
+    double* rr = re + (size_t)rslot[t] * 3;
+    rr[0] = rJ * (mo * As[0] + (md - mo) * Aa[0] - w1 * P.fb[0]) + V * (Nxa[0] * S0 + Nxa[1] * S3 + Nxa[2] * S5);
+    rr[1] = rJ * (mo * As[1] + (md - mo) * Aa[1] - w1 * P.fb[1]) + V * (Nxa[0] * S3 + Nxa[1] * S1 + Nxa[2] * S4);
+    rr[2] = rJ * (mo * As[2] + (md - mo) * Aa[2] - w1 * P.fb[2]) + V * (Nxa[0] * S5 + Nxa[1] * S4 + Nxa[2] * S2);
+}
+
+// Val(:, j) += the blocks of nnz entry j; lanes and order as k_fluid_gather
+// (lane (h, r): row r < 3 of every fourth contribution; the fourth lane of a
+// quad only loads).
+__global__ __launch_bounds__(256) void k_lelas_gather(int nnz, int nNo, unsigned nbVal, const int* __restrict__ gPtr,
+                                                      const int* __restrict__ gSrc, const double* __restrict__ rec,
+                                                      double* __restrict__ val, const int* __restrict__ rPtr,
+                                                      const double* __restrict__ re, double* __restrict__ R)
+{
+    if (blockIdx.x >= nbVal) {
+        const unsigned t = (blockIdx.x - nbVal) * 256 + threadIdx.x;
+        const int i = (int)(t / 3), c = (int)(t - 3 * (t / 3));
+        if (i >= nNo) return;
+        const int k1 = rPtr[i + 1];
+        double s = 0.0;
+#pragma unroll 4
+        for (int k = rPtr[i]; k < k1; ++k) s += re[(size_t)k * 3 + c];
+        R[(size_t)i * 3 + c] += s;
+        return;
+    }
+    const size_t t = (size_t)xcd_part(blockIdx.x, nbVal) * 256 + threadIdx.x;
+    const size_t j = t >> 4;
+    const int r = (int)(t & 3), h = (int)(t >> 2) & 3;
+    if (j >= (size_t)nnz) return; // whole groups of 16 lanes
+    const int k1 = gPtr[j + 1];
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    for (int k = gPtr[j] + h; k < k1; k += 4) {
+        const unsigned src = (unsigned)gSrc[k];
+        const int a = (int)(src >> 2) & 3, b = (int)src & 3;
+        const double* rc = rec + (size_t)(src >> 4) * LR_SZ;
+        const d2_a8 m = *reinterpret_cast<const d2_a8*>(rc + (r == 0 ? 3 * a : (r == 1 ? 3 * b : LR_C + 2 * (r - 2))));
+        const double n = rc[r == 0 ? 3 * a + 2 : (r == 1 ? 3 * b + 2 : 0)];
+        const double a0 = quad_get<0>(m.x), a1 = quad_get<0>(m.y), a2 = quad_get<0>(n);
+        const double b0 = quad_get<1>(m.x), b1 = quad_get<1>(m.y), b2 = quad_get<1>(n);
+        const double c0 = quad_get<2>(m.x), c1 = quad_get<2>(m.y), c2 = quad_get<3>(m.x), c3 = quad_get<3>(m.y);
+        const double d = c1 * (a0 * b0 + a1 * b1 + a2 * b2) + (a == b ? c2 : c3);
+        const double fb = c0 * (r == 0 ? a0 : (r == 1 ? a1 : a2)); // factor of Nx_b
+        const double fa = c1 * (r == 0 ? b0 : (r == 1 ? b1 : b2)); // factor of Nx_a
+        s0 += fb * b0 + fa * a0 + (r == 0 ? d : 0.0);
+        s1 += fb * b1 + fa * a1 + (r == 1 ? d : 0.0);
+        s2 += fb * b2 + fa * a2 + (r == 2 ? d : 0.0);
+    }
+    const bool hi = h & 2, lo = h & 1;
+    const double p0 = (hi ? s2 : s0) + __shfl_xor(hi ? s0 : s2, 8, 16);
+    const double p1 = (hi ? 0.0 : s1) + __shfl_xor(hi ? s1 : 0.0, 8, 16);
+    const double q = (lo ? p1 : p0) + __shfl_xor(lo ? p0 : p1, 4, 16);
+    if (r < 3 && h < 3) val[j * 9 + 3 * r + h] += q;
 }
 
 // ---------------------------------------------------------------------------
@@ -624,31 +776,6 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
 constexpr int FR_T = 0, FR_N = 16, FR_B = 32, FR_C = 36, FR_ES = 40;
 template <bool NN> struct FluidRec { static constexpr int SZ = NN ? 56 : 40; };
 
-typedef double d2_t __attribute__((ext_vector_type(2)));
-
-// v of the lane ^1 / ^2 in the same group of four lanes
-template <int X>
-__device__ __forceinline__ double quad_xor(double v)
-{
-    constexpr int ctrl = X == 1 ? 0xB1 : 0x4E; // quad_perm [1,0,3,2] / [2,3,0,1]
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-// v of lane K of the group of four lanes
-template <int K>
-__device__ __forceinline__ double quad_get(double v)
-{
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), K * 0x55, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), K * 0x55, 0xf, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double quad_sum(double v)
-{
-    v += quad_xor<2>(v);
-    v += quad_xor<1>(v);
-    return v;
-}
 // Sum over the four lanes of a quad of v[4][W], lane g keeping row g.
 template <int W>
 __device__ __forceinline__ void quad_rows(int g, const double (&v)[4][W], double (&o)[W])
@@ -1774,13 +1901,20 @@ int launch_asm_tet4(Mesh& M, int phys, const AsmParams& P, const Tet4Rule& rule,
     if (gather_enabled(M.eNoN)) {
         SV_TRY(M.re.ensure((size_t)M.nEl * 4 * dof * sizeof(double)));
         if (phys == SVFSI_PHYS_LELAS) {
-            SV_TRY(M.ke.ensure((size_t)M.nEl * 16 * dof * dof * sizeof(double)));
-            const unsigned grid = (unsigned)(((size_t)M.nEl * 16 + 255) / 256);
-            hipLaunchKernelGGL(k_asm_lelas, dim3(grid), dim3(256), 0, s, 0, M.nEl, M.ien.as<int>(),
-                               M.elemId.as<int>(), M.emap.as<int>(), M.x.as<double>(), tDof, Ag, Dg, prop, P, rule,
-                               val, R, M.ke.as<double>(), M.re.as<double>(), M.gSlot.as<int>(), M.rSlot.as<int>());
+            SV_TRY(M.ke.ensure((size_t)M.nEl * LR_SZ * sizeof(double)));
+            double* rec = M.ke.as<double>();
+            double* re = M.re.as<double>();
+            hipLaunchKernelGGL(k_lelas_rec, dim3((unsigned)(((size_t)M.nEl * 4 + 255) / 256)), dim3(256), 0, s, M.nEl,
+                               M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, prop, P, rule, rec, re,
+                               M.rSlot.as<int>());
+            const int nnz = M.lhs->nnz;
+            const unsigned nbVal = (unsigned)(((size_t)nnz * 16 + 255) / 256);
+            const unsigned nbR = (unsigned)(((size_t)M.nNo * 3 + 255) / 256);
+            hipLaunchKernelGGL(k_lelas_gather, dim3(nbVal + nbR), dim3(256), 0, s, nnz, M.nNo, nbVal,
+                               M.gPtr.as<int>(), M.gSrc.as<int>(), (const double*)rec, val, M.rPtr.as<int>(),
+                               (const double*)re, R);
             SV_HIP(hipGetLastError());
-            return launch_gather(M, dof, val, R, s);
+            return SVFSI_OK;
         }
         // mu_g is zero with the constant viscosity, whose record leaves esNx out
         if (P.viscType == SVFSI_VISC_CONST) return launch_fluid_rec<false>(M, P, rule, tDof, Ag, Yg, prop, val, R, s);
@@ -1794,7 +1928,7 @@ int launch_asm_tet4(Mesh& M, int phys, const AsmParams& P, const Tet4Rule& rule,
         if (phys == SVFSI_PHYS_LELAS)
             hipLaunchKernelGGL(k_asm_lelas, dim3(grid), dim3(256), 0, s, begin, count, M.ien.as<int>(),
                                M.elemId.as<int>(), M.emap.as<int>(), M.x.as<double>(), tDof, Ag, Dg, prop,
-                               P, rule, val, R, nullptr, nullptr, nullptr, nullptr);
+                               P, rule, val, R);
         else
             hipLaunchKernelGGL(k_asm_fluid, dim3(grid), dim3(256), 0, s, begin, count, M.ien.as<int>(),
                                M.elemId.as<int>(), M.emap.as<int>(), M.x.as<double>(), tDof, Ag, Yg, prop,

@@ -212,8 +212,8 @@ struct Mesh {
     // block j are ke positions gPtr[j] .. gPtr[j+1]-1, in element-id order
     // (the order of DOASSEM's element loop); likewise element row (p, a) at
     // rSlot[p*eNoN + a] of re, node i's rows at rPtr[i] .. rPtr[i+1]-1.
-    // gSrc is gSlot's inverse: position k of ke holds block gSrc[k] =
-    // p*eNoN^2 + a*eNoN + b (tet4: the gather forms the blocks from records).
+    // tet4, whose gather forms the blocks from records, has gSlot's inverse
+    // instead: contribution k is block gSrc[k] = p*16 + a*4 + b.
     DBuf gPtr, gSlot, gSrc, rPtr, rSlot;
     DBuf ke, re;     // element blocks or records / element residual rows, grown on demand
     ~Mesh() {

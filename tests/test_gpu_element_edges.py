@@ -129,3 +129,21 @@ def test_zero_sizes(gpu, nEl, shift):
         for t, n in ((V, nV), (R, nR)):
             assert t[shift:shift + n].abs().max().item() == 0.0
             assert t[:shift].eq(1).all() and t[shift + n:].eq(1).all()
+
+
+def lelas_case(nEl, tDof, uniform, seed=4):
+    prob = problems.lelas_cube(4)
+    rng = np.random.default_rng(seed)
+    prob.mesh.x = prob.mesh.x + rng.uniform(-0.03, 0.03, prob.mesh.x.shape)
+    prob.Ag, prob.Dg = (wide(rng.normal(size=(prob.nNo, 3)), tDof, rng) for _ in range(2))
+    prob.Yg = np.zeros_like(prob.Dg)
+    prob.prop_el = None if uniform else 1e3 * np.exp(0.3 * rng.normal(size=prob.mesh.nEl))
+    prob.eq = dict(prob.eq, E=1e3, fb=(0.3, -0.2, 0.1))
+    return first_elements(prob, nEl)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nEl,tDof,uniform", [(1, 3, True), (13, 7, False), (65, 3, False), (130, 4, True)])
+def test_lelas_assembly_sizes(gpu, orc, nEl, tDof, uniform):
+    for got, want in assembled(lelas_case(nEl, tDof, uniform), orc):
+        assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * np.abs(want).max()
