@@ -763,8 +763,16 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
             for (int a = 0; a < eNoN; ++a) rslot[(size_t)p * eNoN + a] = rpos[sien[(size_t)p * eNoN + a]]++;
         }
     }
-    std::vector<int> gsrc;
+    std::vector<int> gsrc, gtile;
     if (eNoN == 4) {
+        for (int j = 0; j < L.nnz;) {
+            gtile.push_back(j);
+            int j1 = j + 1;
+            while (j1 < L.nnz && j1 - j < kGatherTile && gptr[(size_t)j1 + 1] - gptr[j] <= kGatherTile) ++j1;
+            j = j1;
+        }
+        M->nGTile = (int)gtile.size();
+        gtile.push_back(L.nnz);
         gsrc.resize(gslot.size());
         for (size_t q = 0; q < gslot.size(); ++q) gsrc[gslot[q]] = (int)q;
     }
@@ -782,7 +790,7 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
     M->nMid = (int)mids.size();
     int rc = SVFSI_OK;
     if ((rc = upload(M->ien, sien)) || (rc = upload(M->elemId, order)) || (rc = upload(M->emap, emap)) ||
-        (rc = upload(M->x, xv)) || (rc = upload(M->gPtr, gptr)) || (rc = eNoN == 4 ? upload(M->gSrc, gsrc) : upload(M->gSlot, gslot)) ||
+        (rc = upload(M->x, xv)) || (rc = upload(M->gPtr, gptr)) || (rc = eNoN == 4 ? upload(M->gSrc, gsrc) : upload(M->gSlot, gslot)) || (rc = upload(M->gTile, gtile)) ||
         (rc = upload(M->rPtr, rptr)) || (rc = upload(M->rSlot, rslot)) ||
         (!mids.empty() && (rc = upload(M->midNodes, mids)))) {
         delete M;

@@ -93,6 +93,86 @@ __device__ __forceinline__ double quad_sum(double v)
     return v;
 }
 // ---------------------------------------------------------------------------
+// The record gathers: Val(:, j) += the element blocks of nnz entry j, in
+// element-id order (DOASSEM's element loop, LHSA.f:266-298), the blocks formed
+// from the elements' records.  gSrc[k] = 16 e + 4 a + b names contribution k,
+// gPtr the contributions of each entry.  One workgroup takes a tile of whole
+// entries with at most kGatherTile contributions (Mesh::gTile); four lanes
+// form a contribution, every lane kGatherTile / 64 of them with all loads
+// issued first (row(): the lane's row of the block), and leave its rows in
+// LDS; then DD lanes per entry add them in order.  An entry with more
+// contributions than a tile holds has a tile of its own and goes through it
+// in passes.
+//
+// Bound by latency: a contribution is the chain gPtr -> gSrc -> record ->
+// Val, so what counts is how many chains are in flight.  16 lanes per entry
+// walking its list, four chains at a time, took 94 us (fluid, 197,696 tets)
+// and 90 us (LELAS, 215,622), with most lanes waiting on short lists and the
+// 24 contributions of the diagonal entries; the tiles take 80 and 59
+// us (with multiply-adds contracted here, where no Jacobian is inverted).
+// Tiles go in XCD-contiguous order: the entries of neighbouring rows read the
+// same records.  Val may be only 8-byte aligned.
+// ---------------------------------------------------------------------------
+template <int DD, class ROW>
+__device__ __forceinline__ void gather_tile(unsigned b, const int* __restrict__ tile, const int* __restrict__ gPtr,
+                                            const int* __restrict__ gSrc, double* __restrict__ val, ROW&& row)
+{
+    constexpr int T = kGatherTile, U = T / 64, RW = DD == 16 ? 4 : 3, EPP = 256 / DD; // entries per pass of the sum
+    __shared__ double sB[T][DD];
+    __shared__ int sP[T + 1];
+    const int tid = threadIdx.x, r = tid & 3;
+    const int j0 = tile[b], nj = tile[b + 1] - j0;
+    for (int i = tid; i <= nj; i += 256) sP[i] = gPtr[j0 + i];
+    const int k0 = gPtr[j0], k1 = gPtr[j0 + nj];
+    // the old values of the entries this lane will write, loaded early
+    double old[U];
+    const int se = tid / DD, sq = tid - se * DD;
+#pragma unroll
+    for (int m = 0; m < U; ++m) {
+        const int e = se + m * EPP;
+        old[m] = (se < EPP && e < nj) ? val[(size_t)(j0 + e) * DD + sq] : 0.0;
+    }
+    double sum = 0.0; // an entry larger than the tile (nj = 1): the passes' running sum
+    for (int kb = k0; kb < k1; kb += T) {
+        unsigned src[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = kb + u * 64 + (tid >> 2);
+            src[u] = k < k1 ? (unsigned)gSrc[k] : 0u;
+        }
+        double v[U][RW];
+#pragma unroll
+        for (int u = 0; u < U; ++u) row(src[u], r, v[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (r < RW)
+#pragma unroll
+                for (int c = 0; c < RW; ++c) sB[u * 64 + (tid >> 2)][r * RW + c] = v[u][c];
+        __syncthreads();
+        if (se < EPP) {
+#pragma unroll
+            for (int m = 0; m < U; ++m) {
+                const int e = se + m * EPP;
+                if (e >= nj) break;
+                const int ke = min(sP[e + 1], kb + T);
+                double s = nj == 1 ? sum : 0.0;
+#pragma unroll 4
+                for (int k = max(sP[e], kb); k < ke; ++k) s += sB[k - kb][sq];
+                if (nj == 1) sum = s;
+                if (sP[e + 1] <= kb + T) val[(size_t)(j0 + e) * DD + sq] = old[m] + s;
+            }
+            for (int e = se + U * EPP; e < nj; e += EPP) { // many short entries
+                const int ke = sP[e + 1];
+                double s = 0.0;
+                for (int k = sP[e]; k < ke; ++k) s += sB[k - kb][sq];
+                val[(size_t)(j0 + e) * DD + sq] += s;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------------
 // LELAS3D (svFSI/LELAS.f:130-242) in CONSTRUCT_LELAS (LELAS.f:38-128), tet4.
 // ---------------------------------------------------------------------------
 // The coloured scatter path (SVFSI_ASM_GATHER=0).
@@ -199,7 +279,7 @@ __global__ __launch_bounds__(256) void k_asm_lelas(int begin, int count, const i
 // mass m_ab = am rho Jac sum_g w_g N_a N_b, which takes one value on the
 // diagonal (c2) and one off it (c3): 16 numbers, one 128-byte line, against
 // 1152 bytes of element blocks.  On the 215,622-tet cube the element kernel
-// takes 22 us and the gather 90, against 195 us for 16 lanes per element
+// takes 22 us and the gather 59, against 195 us for 16 lanes per element
 // storing their blocks and 81 + 8 us for summing those.
 // ---------------------------------------------------------------------------
 constexpr int LR_C = 12, LR_SZ = 16;
@@ -284,13 +364,13 @@ __global__ __launch_bounds__(256) void k_lelas_rec(int nEl, const int* __restric
     rr[2] = rJ * (mo * As[2] + (md - mo) * Aa[2] - w1 * P.fb[2]) + V * (Nxa[0] * S5 + Nxa[1] * S4 + Nxa[2] * S2);
 }
 
-// Val(:, j) += the blocks of nnz entry j; lanes and order as k_fluid_gather
-// (lane (h, r): row r < 3 of every fourth contribution; the fourth lane of a
-// quad only loads).
-__global__ __launch_bounds__(256) void k_lelas_gather(int nnz, int nNo, unsigned nbVal, const int* __restrict__ gPtr,
-                                                      const int* __restrict__ gSrc, const double* __restrict__ rec,
-                                                      double* __restrict__ val, const int* __restrict__ rPtr,
-                                                      const double* __restrict__ re, double* __restrict__ R)
+// Val from the records (gather_tile; the fourth lane of a quad only loads)
+// and, in the workgroups from nbVal on, the R rows.
+__global__ __launch_bounds__(256) void k_lelas_gather(int nNo, unsigned nbVal, const int* __restrict__ tile,
+                                                      const int* __restrict__ gPtr, const int* __restrict__ gSrc,
+                                                      const double* __restrict__ rec, double* __restrict__ val,
+                                                      const int* __restrict__ rPtr, const double* __restrict__ re,
+                                                      double* __restrict__ R)
 {
     if (blockIdx.x >= nbVal) {
         const unsigned t = (blockIdx.x - nbVal) * 256 + threadIdx.x;
@@ -303,14 +383,8 @@ __global__ __launch_bounds__(256) void k_lelas_gather(int nnz, int nNo, unsigned
         R[(size_t)i * 3 + c] += s;
         return;
     }
-    const size_t t = (size_t)xcd_part(blockIdx.x, nbVal) * 256 + threadIdx.x;
-    const size_t j = t >> 4;
-    const int r = (int)(t & 3), h = (int)(t >> 2) & 3;
-    if (j >= (size_t)nnz) return; // whole groups of 16 lanes
-    const int k1 = gPtr[j + 1];
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int k = gPtr[j] + h; k < k1; k += 4) {
-        const unsigned src = (unsigned)gSrc[k];
+    gather_tile<9>(xcd_part(blockIdx.x, nbVal), tile, gPtr, gSrc, val, [&](unsigned src, int r, double (&v)[3]) {
+#pragma clang fp contract(fast) // no Jacobian here: see the top of the file
         const int a = (int)(src >> 2) & 3, b = (int)src & 3;
         const double* rc = rec + (size_t)(src >> 4) * LR_SZ;
         const d2_a8 m = *reinterpret_cast<const d2_a8*>(rc + (r == 0 ? 3 * a : (r == 1 ? 3 * b : LR_C + 2 * (r - 2))));
@@ -321,15 +395,10 @@ __global__ __launch_bounds__(256) void k_lelas_gather(int nnz, int nNo, unsigned
         const double d = c1 * (a0 * b0 + a1 * b1 + a2 * b2) + (a == b ? c2 : c3);
         const double fb = c0 * (r == 0 ? a0 : (r == 1 ? a1 : a2)); // factor of Nx_b
         const double fa = c1 * (r == 0 ? b0 : (r == 1 ? b1 : b2)); // factor of Nx_a
-        s0 += fb * b0 + fa * a0 + (r == 0 ? d : 0.0);
-        s1 += fb * b1 + fa * a1 + (r == 1 ? d : 0.0);
-        s2 += fb * b2 + fa * a2 + (r == 2 ? d : 0.0);
-    }
-    const bool hi = h & 2, lo = h & 1;
-    const double p0 = (hi ? s2 : s0) + __shfl_xor(hi ? s0 : s2, 8, 16);
-    const double p1 = (hi ? 0.0 : s1) + __shfl_xor(hi ? s1 : 0.0, 8, 16);
-    const double q = (lo ? p1 : p0) + __shfl_xor(lo ? p0 : p1, 4, 16);
-    if (r < 3 && h < 3) val[j * 9 + 3 * r + h] += q;
+        v[0] = fb * b0 + fa * a0 + (r == 0 ? d : 0.0);
+        v[1] = fb * b1 + fa * a1 + (r == 1 ? d : 0.0);
+        v[2] = fb * b2 + fa * a2 + (r == 2 ? d : 0.0);
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -769,7 +838,7 @@ __global__ __launch_bounds__(256) void k_asm_fluid(int begin, int count, const i
 // element arithmetic: geometry and point quantities are evaluated 4 times
 // per element instead of 16, and the sum over g is taken once per element
 // instead of inside every entry.  FLUID assembly of that mesh: k_fluid_rec 45
-// us and k_fluid_gather 94 us, where the element blocks took 315 us (16 lanes
+// us and k_fluid_gather 80 us, where the element blocks took 315 us (16 lanes
 // per element, each its block with the geometry repeated) and their gather
 // 119 + 12 us.
 // ---------------------------------------------------------------------------
@@ -896,48 +965,33 @@ __global__ __launch_bounds__(256) void k_fluid_rec(int nEl, const int* __restric
     *reinterpret_cast<d2_t*>(rr + 2) = d2_t{ro[2], ro[3]};
 }
 
-// Val(:, j) += the blocks of nnz entry j, 16 lanes per entry: lane (h, r)
-// forms row r of the contributions gPtr[j] + h, + 4, ... (gSrc[k] = 16 e +
-// 4 a + b names the k-th, in element-id order) and the four partial sums meet
-// by shuffles, in a fixed order.  Each contribution is a chain of two
-// dependent loads (gSrc, then the record) and a diagonal entry has two dozen
-// of them, so four chains run side by side, and the workgroups go in
-// XCD-contiguous order (xcd_part), since the entries of neighbouring rows
-// read the same records, which otherwise every XCD's L2 fetches: 230 us with
-// one chain per entry, hardware order and the records in colour order, 122
-// us with these.  The workgroups from nbVal on sum the R rows.  Val may be
-// only 8-byte aligned.
+// Val from the records (gather_tile) and, in the workgroups from nbVal on, the
+// R rows.  The four lanes of a quad load a quarter of a contribution's 112 B
+// each and pass it on: two load instructions instead of eight (122 -> 94 us
+// before the tiles).
 template <bool NN>
-__global__ __launch_bounds__(256) void k_fluid_gather(int nnz, int nNo, unsigned nbVal, const int* __restrict__ gPtr,
-                                                      const int* __restrict__ gSrc, const double* __restrict__ rec,
-                                                      double* __restrict__ val, const int* __restrict__ rPtr,
-                                                      const double* __restrict__ re, double* __restrict__ R)
+__global__ __launch_bounds__(256) void k_fluid_gather(int nNo, unsigned nbVal, const int* __restrict__ tile,
+                                                      const int* __restrict__ gPtr, const int* __restrict__ gSrc,
+                                                      const double* __restrict__ rec, double* __restrict__ val,
+                                                      const int* __restrict__ rPtr, const double* __restrict__ re,
+                                                      double* __restrict__ R)
 {
     if (blockIdx.x >= nbVal) {
         const unsigned t = (blockIdx.x - nbVal) * 256 + threadIdx.x;
         const int i = (int)(t >> 2), c = (int)(t & 3);
         if (i >= nNo) return;
-        const double* src = re + (size_t)c;
         const int k1 = rPtr[i + 1];
         double s = 0.0;
 #pragma unroll 4
-        for (int k = rPtr[i]; k < k1; ++k) s += src[(size_t)k * 4];
+        for (int k = rPtr[i]; k < k1; ++k) s += re[(size_t)k * 4 + c];
         R[(size_t)i * 4 + c] += s;
         return;
     }
-    const size_t t = (size_t)xcd_part(blockIdx.x, nbVal) * 256 + threadIdx.x;
-    const size_t j = t >> 4;
-    const int r = (int)(t & 3), h = (int)(t >> 2) & 3;
-    if (j >= (size_t)nnz) return; // whole groups of 16 lanes
-    const int k1 = gPtr[j + 1];
-    const bool mom = r < 3;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    for (int k = gPtr[j] + h; k < k1; k += 4) {
-        const unsigned src = (unsigned)gSrc[k];
+    gather_tile<16>(xcd_part(blockIdx.x, nbVal), tile, gPtr, gSrc, val, [&](unsigned src, int r, double (&v)[4]) {
+#pragma clang fp contract(fast) // no Jacobian here: see the top of the file
+        const bool mom = r < 3;
         const int a = (int)(src >> 2) & 3, b = (int)src & 3;
         const double* rc = rec + (size_t)(src >> 4) * FluidRec<NN>::SZ;
-        // the four lanes of a quad load a quarter of the 112 B each and pass
-        // it on: two load instructions instead of eight (122 -> 94 us)
         const d2_t m = *reinterpret_cast<const d2_t*>(rc + FR_N + 4 * (r < 2 ? a : b) + 2 * (r & 1));
         const d2_a8 n = *reinterpret_cast<const d2_a8*>(
             rc + (r == 0 ? FR_C : (r == 1 ? FR_C + 2 : (r == 2 ? FR_T + 4 * a + b : FR_B + b))));
@@ -960,17 +1014,11 @@ __global__ __launch_bounds__(256) void k_fluid_gather(int nnz, int nNo, unsigned
             v1 += er * quad_get<1>(eb);
             v2 += er * quad_get<2>(eb);
         }
-        s0 += v0 + (r == 0 ? T : 0.0);
-        s1 += v1 + (r == 1 ? T : 0.0);
-        s2 += v2 + (r == 2 ? T : 0.0);
-        s3 += mom ? br * a1.y - c23.x * ar : c23.y * (a0.x * b0.x + a0.y * b0.y + a1.x * b1.x);
-    }
-    // the lanes h of a row: sum over h, lane h keeps column h
-    const bool hi = h & 2, lo = h & 1;
-    const double p0 = (hi ? s2 : s0) + __shfl_xor(hi ? s0 : s2, 8, 16);
-    const double p1 = (hi ? s3 : s1) + __shfl_xor(hi ? s1 : s3, 8, 16);
-    const double q = (lo ? p1 : p0) + __shfl_xor(lo ? p0 : p1, 4, 16);
-    val[j * 16 + 4 * r + h] += q;
+        v[0] = v0 + (r == 0 ? T : 0.0);
+        v[1] = v1 + (r == 1 ? T : 0.0);
+        v[2] = v2 + (r == 2 ? T : 0.0);
+        v[3] = mom ? br * a1.y - c23.x * ar : c23.y * (a0.x * b0.x + a0.y * b0.y + a1.x * b1.x);
+    });
 }
 
 // Viscosity sensitivity of the fluid element (no reference counterpart):
@@ -1885,11 +1933,11 @@ static int launch_fluid_rec(Mesh& M, const AsmParams& P, const Tet4Rule& rule, i
     hipLaunchKernelGGL(k_fluid_rec<NN>, dim3((unsigned)(((size_t)M.nEl * 4 + 255) / 256)), dim3(256), 0, s, M.nEl,
                        M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Yg, muEl, P, rule, rec, re,
                        M.rSlot.as<int>());
-    const int nnz = M.lhs->nnz;
-    const unsigned nbVal = (unsigned)(((size_t)nnz * 16 + 255) / 256);
+    const unsigned nbVal = (unsigned)M.nGTile;
     const unsigned nbR = (unsigned)(((size_t)M.nNo * 4 + 255) / 256);
-    hipLaunchKernelGGL(k_fluid_gather<NN>, dim3(nbVal + nbR), dim3(256), 0, s, nnz, M.nNo, nbVal, M.gPtr.as<int>(),
-                       M.gSrc.as<int>(), (const double*)rec, val, M.rPtr.as<int>(), (const double*)re, R);
+    hipLaunchKernelGGL(k_fluid_gather<NN>, dim3(nbVal + nbR), dim3(256), 0, s, M.nNo, nbVal, M.gTile.as<int>(),
+                       M.gPtr.as<int>(), M.gSrc.as<int>(), (const double*)rec, val, M.rPtr.as<int>(),
+                       (const double*)re, R);
     SV_HIP(hipGetLastError());
     return SVFSI_OK;
 }
@@ -1907,10 +1955,9 @@ int launch_asm_tet4(Mesh& M, int phys, const AsmParams& P, const Tet4Rule& rule,
             hipLaunchKernelGGL(k_lelas_rec, dim3((unsigned)(((size_t)M.nEl * 4 + 255) / 256)), dim3(256), 0, s, M.nEl,
                                M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, prop, P, rule, rec, re,
                                M.rSlot.as<int>());
-            const int nnz = M.lhs->nnz;
-            const unsigned nbVal = (unsigned)(((size_t)nnz * 16 + 255) / 256);
+            const unsigned nbVal = (unsigned)M.nGTile;
             const unsigned nbR = (unsigned)(((size_t)M.nNo * 3 + 255) / 256);
-            hipLaunchKernelGGL(k_lelas_gather, dim3(nbVal + nbR), dim3(256), 0, s, nnz, M.nNo, nbVal,
+            hipLaunchKernelGGL(k_lelas_gather, dim3(nbVal + nbR), dim3(256), 0, s, M.nNo, nbVal, M.gTile.as<int>(),
                                M.gPtr.as<int>(), M.gSrc.as<int>(), (const double*)rec, val, M.rPtr.as<int>(),
                                (const double*)re, R);
             SV_HIP(hipGetLastError());

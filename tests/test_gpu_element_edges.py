@@ -147,3 +147,26 @@ def lelas_case(nEl, tDof, uniform, seed=4):
 def test_lelas_assembly_sizes(gpu, orc, nEl, tDof, uniform):
     for got, want in assembled(lelas_case(nEl, tDof, uniform), orc):
         assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("points", [60, 200, 400])
+@pytest.mark.parametrize("kind", ["lelas", "fluid"])
+def test_assembly_hub_node(gpu, orc, kind, points):
+    """Tets that all share one node: its diagonal block sums fewer, more, and
+    several times more contributions than a gather tile holds (128)."""
+    from scipy.spatial import ConvexHull
+
+    rng = np.random.default_rng(points)
+    s = rng.normal(size=(points, 3))
+    s /= np.linalg.norm(s, axis=1, keepdims=True)
+    tri = ConvexHull(s).simplices
+    x = np.concatenate([s, np.zeros((1, 3))])
+    ien = np.concatenate([tri, np.full((len(tri), 1), points)], axis=1)
+    m = meshmod.TetMesh(x=x, ien=meshmod._orient(x, ien.astype(np.int32)).astype(np.int32))
+    prob = fluid_case(1, 4, True) if kind == "fluid" else lelas_case(1, 3, True)
+    prob.mesh = m
+    for k in ("Ag", "Yg", "Dg"):
+        setattr(prob, k, rng.normal(size=(m.nNo, prob.dof)))
+    for got, want in assembled(prob, orc):
+        assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * max(1.0, np.abs(want).max())
