@@ -903,15 +903,19 @@ __global__ __launch_bounds__(256) void k_fluid_rec(int nEl, const int* __restric
         uaN[a] = uN[a] + upN[a];
     }
     double v[4][6], o[6];
+    {
+#pragma clang fp contract(fast) // the Jacobian is behind: see the top of the file
+        const double ra = rho * amd;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const double adv = rho * tauM * uaN[a];
+        for (int a = 0; a < 4; ++a) {
+            const double adv = rho * tauM * uaN[a];
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-            v[a][b] = wl * (rho * amd * N[b] * (N[a] + adv) + rho * N[a] * uaN[b] + G.tauB * upN[a] * upN[b]
-                            + adv * (rho * uN[b]));
-        v[a][4] = wl * adv;
-        v[a][5] = wl * tauM * (rho * uN[a] + rho * amd * N[a]);
+            for (int b = 0; b < 4; ++b)
+                v[a][b] = wl * (ra * N[b] * (N[a] + adv) + rho * (N[a] * uaN[b] + adv * uN[b])
+                                + G.tauB * upN[a] * upN[b]);
+            v[a][4] = wl * adv;
+            v[a][5] = wl * tauM * (rho * uN[a] + ra * N[a]);
+        }
     }
     quad_rows<6>(g, v, o);
     const double W = quad_sum(wl);
