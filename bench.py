@@ -455,6 +455,11 @@ def main() -> int:
             what = ("the finest level of the multigrid V-cycle: FP32 CSR-stream block SpMVs over row tiles "
                     + ("with the residual (r = b - A x) or the Chebyshev step fused in" if fused else
                        "of the Chebyshev smoothing and the residuals"))
+        elif poly and os.environ.get("SVFSI_PERSIST", "") != "0" and n32 < lsprof[-1].RI.cM - n64m:
+            # fewer launches than products: the matrix-resident kernel, one launch per application
+            kname = f"k_ppoly<{dof}"
+            what = ("the polynomial preconditioner's factor steps in one matrix-resident launch per application, plus "
+                    "the setup Arnoldi SpMVs; bytes count the matrix once per launch")
         elif poly and os.environ.get("SVFSI_SPMV_STREAM", "") != "0":
             # the CSR-stream kernels over row tiles of 256 blocks (512 from 2M blocks on)
             tt = 512 if nnzb >= (2 << 20) else 256
@@ -474,7 +479,8 @@ def main() -> int:
             kname = "k_bspmv4<float, 4" if dof == 4 else f"k_bspmv<{dof}, float, float"
             what = "FP32 block SpMV, inner GMRES"
         roof = {"kernel": f"{kname}> ({what})",
-                "bound": "hbm", "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "bound": "latency" if kname.startswith("k_ppoly") else "hbm",
+                "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(gbs32 / HBM_PEAK_GBS, 4), "traffic": measured_traffic(nnzb, kname),
                 "bytes_per_launch": round(b32), "avg_launch_us": round(t32 / n32 * 1e3, 2), "launches": n32,
                 "full_work_launches": n32_full, "timing": "events attached to each dispatch (hipExtLaunchKernelGGL)"}

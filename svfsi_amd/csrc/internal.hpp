@@ -124,6 +124,7 @@ struct GraphCache {
     void clear();
 };
 
+struct Parts;   // row partition of the matrix-resident kernels (persist.hpp)
 struct AmgHier; // aggregation multigrid hierarchy (amg.hip)
 
 // Krylov workspace, grown on demand and reused across solves.
@@ -145,6 +146,7 @@ struct Work {
     DBuf valIn;  // FP64 nested solve: the block-Jacobi scaled inner matrix
     std::shared_ptr<AmgHier> amg; // inner multigrid of the nested solve (pattern part kept)
     DBuf polyCoef, polyVec; // polynomial preconditioner: factors, work vectors
+    DBuf polyOps;           // its matrix-resident form: step list
     int maskDof = -1;
     std::vector<int> maskInc;
     int maskVersion = -1;
@@ -180,6 +182,7 @@ struct Lhs {
     int nTiles[3] = {0, 0, 0};
     CplSet cpl;
     Work ws;
+    std::shared_ptr<Parts> parts; // built on first use
 };
 
 // Contributions per workgroup of the tet4 record gathers: 64, 128 and 256 take

@@ -12,6 +12,7 @@
 #include "internal.hpp"
 #include "devutil.hpp"
 #include "stream.hpp"
+#include "persist.hpp"
 
 #include <chrono>
 #include <cmath>
@@ -1035,7 +1036,7 @@ struct GmState {
     double fNorm;
     int stop, suc, iconv, iters;  // iters: Arnoldi steps run (accumulates)
     unsigned int counter;
-    int pad2;
+    int abort;  // a matrix-resident kernel gave up waiting (persist.hpp); stop is set too
 };
 
 struct GmArrays {
@@ -1077,6 +1078,7 @@ __global__ void k_gm_init(GmState* __restrict__ st, double eps)
     st->iconv = 0;
     st->iters = 0;
     st->counter = 0u;
+    st->abort = 0;
 }
 
 // u0 = R - u0 and |u0|; last block: err(1) = |u0|, cycle state reset.
@@ -2154,8 +2156,11 @@ static double env_dbl(const char* k, double d)
 // matrix: the FP32 copy of the scaled matrix written by the diagonal
 // preconditioner (IT = float), or nullptr (IT = double: the scaled FP64
 // matrix itself, or a copy in w.valIn when block Jacobi rescales it).
+// retry (may be null): set when a matrix-resident kernel gave up; R is then
+// untouched and the caller solves again without them.
 template <typename IT>
-static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, IT* Kin, double* R, hipStream_t s)
+static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, IT* Kin, double* R, hipStream_t s,
+                        bool* retry)
 {
     const size_t n = (size_t)L.nNo * dof;
     Work& w = L.ws;
@@ -2320,6 +2325,12 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
     IT *P0 = nullptr, *P1 = nullptr, *Wb = nullptr;
     const double* coefD = nullptr;
     bool usePoly = polyWanted;
+    // all factors in one matrix-resident launch where the matrix fits the
+    // chip's registers (ppoly.hip); ops: its SpMV steps
+    PersistLock plock;
+    Parts* parts = nullptr;
+    std::vector<int> ops;
+    int lastLin = -1;
     if (usePoly) {
         // degree 25 when the inner matrix fits half the Infinity Cache, else
         // 30 (measured, ms per Newton step: 200k-tet cylinder 6.7 at 25
@@ -2361,6 +2372,19 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
                 const bool last = f == nf - 1;
                 if (kinds[f] == 1) polySpmv += last ? 0 : 1;
                 else polySpmv += 1 + ((!last && coef[2 * f + 1] != 0.0) ? 1 : 0);
+                if (kinds[f] == 1 && last) lastLin = f;
+                else if (kinds[f] == 1) ops.insert(ops.end(), {0, f});
+                else {
+                    ops.insert(ops.end(), {1, f});
+                    if (!last) ops.insert(ops.end(), {2, f});
+                }
+            }
+            if (std::is_same<IT, float>::value && retry && plock.acquire()) parts = persist_parts(L);
+            if (parts) {
+                SV_TRY(w.polyOps.ensure(ops.size() * sizeof(int)));
+                SV_HIP(hipMemcpyAsync(w.polyOps.p, ops.data(), ops.size() * sizeof(int), hipMemcpyHostToDevice, s));
+            } else {
+                plock.release();
             }
         } else {
             usePoly = false; // no usable roots: the inner GMRES cycle
@@ -2423,6 +2447,12 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
                         hipLaunchKernelGGL((k_cvt<double, IT>), dim3(gv), dim3(256), 0, cs, n,
                                            (const double*)(Q + (size_t)(i - 1) * n), P0);
                         SV_TRY(amg_apply(L, dof, P0, zi, cs));
+                    }
+                } else if (parts) {
+                    if constexpr (std::is_same<IT, float>::value) {
+                        SV_TRY(ppoly_launch(L, *parts, dof, Kin, dinv, Q + (size_t)(i - 1) * n, zi, t64, coefD, w.polyOps.as<int>(), (int)ops.size() / 2,
+                                            lastLin, &st->stop, &st->abort, cs));
+                        t64Done = true;
                     }
                 } else if (usePoly) {
                     // z_i = p(B) D^-1 q_i, factor by factor
@@ -2508,6 +2538,12 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
                 if (hs.stop) break;
             }
         }
+        if (parts && hs.abort) {
+            SV_HIP(hipStreamSynchronize(s));
+            parts->off = true;
+            *retry = true;
+            return SVFSI_OK;
+        }
         {
             const size_t tri = (size_t)mo * (mo + 1) / 2;
             const size_t ldsB = (tri <= (size_t)kBackLds ? tri : 0) * sizeof(double);
@@ -2517,6 +2553,11 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
         SV_HIP(hipGetLastError());
         SV_HIP(hipMemcpyAsync(&hs, st, sizeof(GmState), hipMemcpyDeviceToHost, s));
         SV_HIP(hipStreamSynchronize(s));
+        if (parts && hs.abort) {
+            parts->off = true;
+            *retry = true;
+            return SVFSI_OK;
+        }
         ls.itr += hs.iconv;
         ls.fNorm = hs.fNorm;
         if (hs.suc) {
@@ -2544,12 +2585,15 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
 
 int mixed_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, float* K32, double* R, hipStream_t s)
 {
-    return nested_solve<float>(L, ls, dof, K, K32, R, s);
+    bool retry = false;
+    SV_TRY(nested_solve<float>(L, ls, dof, K, K32, R, s, &retry));
+    // with block Jacobi K32 already holds D^-1 K, formed again from K
+    return retry ? nested_solve<float>(L, ls, dof, K, K32, R, s, nullptr) : SVFSI_OK;
 }
 
 int nested_solve_fp64(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hipStream_t s)
 {
-    return nested_solve<double>(L, ls, dof, K, nullptr, R, s);
+    return nested_solve<double>(L, ls, dof, K, nullptr, R, s, nullptr);
 }
 
 } // namespace svfsi

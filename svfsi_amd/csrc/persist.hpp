@@ -1,0 +1,143 @@
+// persist.hpp -- matrix-resident kernels: a square block matrix cut into
+// parts of rows, one workgroup per part and at most one part per CU, all
+// parts resident at once, so that a sequence of products runs in one launch
+// with the matrix held in registers.
+//
+// The parts are balls of the node graph (grown breadth first on the host,
+// once per pattern): a part of 104 rows of the 200k-tet cylinder has a halo
+// of about 250 nodes, against 470 to 800 for 104 consecutive rows.  A row has
+// a group of 4 to 64 lanes, each holding U of its blocks.
+//
+// Between products the parts exchange the entries of the vector that their
+// neighbours' blocks touch (the halo) through global memory.  On eight XCDs
+// an ordinary store stays in the writer's L2, so the exchange uses agent-scope
+// relaxed atomics (write-through stores, loads that miss the L2s), and every
+// 8-byte word carries half a value and half a tag, the epoch it belongs to: a
+// reader polls the words it needs until their tags match, one trip through
+// memory, with no flag, no fence and no grid-wide barrier.  (Measured, 256
+// workgroups: a barrier on one counter 3.9 us, on eight counters under a
+// master 2.25 us; a product step with drained stores and per-part flags 6.0
+// us, with tagged words 3.6 us,
+// start and end of the kernel included.)
+//
+// Two buffers alternate.  A part writes step s + 2 over step s only after it
+// has read its neighbours' step s + 1, which they write after reading all of
+// step s: the pattern must be structurally symmetric, so that whoever reads a
+// part is also read by it.
+//
+// Every wait is bounded: a lane that has polled for kWaitTicks raises the
+// abort flag, its workgroup ends, and all others end at their next wait; the
+// caller then takes the path of one launch per product.  That happens only
+// when the parts are not resident together (another kernel that itself waits
+// holds CUs); PersistLock keeps two such kernels of one process apart.
+#pragma once
+
+#include "internal.hpp"
+
+namespace svfsi {
+
+// Device view of a partition.  Row r of part b (in lane order) is node
+// rowId[rowOff[b] + r], and rowOff[b] + r is its position in the exchange
+// buffer.  lane: per lane of the part its row | log2(lanes of the row) << 16,
+// -1 for none; a row's lanes are consecutive and aligned to their number.
+struct PartsDev {
+    const int* rowOff;          // G+1
+    const int* rowId;           // nNo
+    const int* laneOff;         // G+1
+    const int* lane;
+    const int* hOff;            // G+1 offsets into hPos
+    const int* hPos;            // halo: positions in the exchange buffer
+    const unsigned short* lcol; // per block: local index of its column, own rows first, then the halo
+    unsigned long long* xb;     // 2 x nNo x 4 tagged words
+    unsigned long long wait;    // ticks before a waiting lane gives up
+    int G;
+};
+
+constexpr unsigned long long kWaitTicks = 100000000ull; // 1 s of the 100 MHz wall clock
+
+template <typename T>
+__device__ __forceinline__ T ld_agent(const T* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void st_agent(T* p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// 32 bits of payload under a tag
+__device__ __forceinline__ void put_word(unsigned long long* p, unsigned v, unsigned tag)
+{
+    st_agent(p, ((unsigned long long)tag << 32) | v);
+}
+
+// Polls the N words p[m] (null: skipped) until each carries tag, payloads to
+// v.  false: gave up, or another workgroup has.
+template <int N>
+__device__ __forceinline__ bool get_words(const unsigned long long* const (&p)[N], unsigned tag, unsigned (&v)[N],
+                                          unsigned long long wait, int* abortFlag)
+{
+    unsigned long long t0 = 0;
+    for (int n = 1;; ++n) {
+        unsigned long long w[N];
+#pragma unroll
+        for (int m = 0; m < N; ++m) w[m] = p[m] ? ld_agent(p[m]) : ((unsigned long long)tag << 32);
+        bool all = true;
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            all = all && (unsigned)(w[m] >> 32) == tag;
+            v[m] = (unsigned)w[m];
+        }
+        if (all) return true;
+        if ((n & 63) == 0 || wait == 0) {
+            if (ld_agent(abortFlag)) return false;
+            const unsigned long long t = wall_clock64();
+            if (!t0) t0 = t;
+            if (t - t0 >= wait) {
+                st_agent(abortFlag, 1);
+                return false;
+            }
+        }
+    }
+}
+
+// A partition of a pattern for kernels that hold U blocks per lane.
+struct Parts {
+    int G = 0, U = 0, maxOwn = 0, maxHalo = 0, maxLanes = 0;
+    unsigned epoch = 0; // the last tag used; xb starts out with tag 0
+    bool tried = false, off = false;
+    unsigned long long wait = kWaitTicks;
+    DBuf rowOff, rowId, laneOff, lane, hOff, hPos, lcol, xb;
+    PartsDev dev() const
+    {
+        return {rowOff.as<int>(), rowId.as<int>(), laneOff.as<int>(), lane.as<int>(), hOff.as<int>(), hPos.as<int>(),
+                lcol.as<unsigned short>(), xb.as<unsigned long long>(), wait, G};
+    }
+};
+
+// The partition of L, built on the first call and kept with L; nullptr when
+// the pattern does not fit the chip or the path is off.
+Parts* persist_parts(Lhs& L);
+
+// One matrix-resident solve at a time per device and process: they would
+// wait for each other's CUs.
+struct PersistLock {
+    int dev = -1;
+    PersistLock() = default;
+    PersistLock(const PersistLock&) = delete;
+    PersistLock& operator=(const PersistLock&) = delete;
+    ~PersistLock() { release(); }
+    bool acquire();
+    void release();
+};
+
+// z = p(B) D^-1 q, all factors of the polynomial preconditioner in one
+// launch (ppoly.hip).  ops: nOps pairs (mode, factor) of SpMV steps as
+// launch_poly's; lastLin: the closing linear factor without a product, or -1.
+int ppoly_launch(Lhs& L, Parts& P, int dof, const float* B, const float* dinv, const double* q, float* z, double* z64,
+                 const double* coef, const int* ops, int nOps, int lastLin, int* stop, int* abortFlag,
+                 hipStream_t s);
+size_t ppoly_lds(const Parts& P); // its dynamic LDS
+
+} // namespace svfsi

@@ -1,0 +1,118 @@
+"""The matrix-resident polynomial preconditioner (one launch per application)
+against one launch per factor: the same polynomial with the products of long
+rows summed in another order, so the mixed solve makes the same outer steps
+(one more or less where the residual passes near the tolerance) and reaches
+the same solution to its own tolerance."""
+import threading
+
+import numpy as np
+import pytest
+
+from svfsi_amd import mesh as meshmod
+from svfsi_amd import problems
+
+
+def hub(points):
+    """Tets around one node: its block row holds points + 1 blocks."""
+    from scipy.spatial import ConvexHull
+
+    rng = np.random.default_rng(points)
+    s = rng.normal(size=(points, 3))
+    s /= np.linalg.norm(s, axis=1, keepdims=True)
+    tri = ConvexHull(s).simplices
+    x = np.concatenate([s, np.zeros((1, 3))])
+    ien = np.concatenate([tri, np.full((len(tri), 1), points)], axis=1)
+    prob = problems.lelas_cube(2)
+    prob.mesh = meshmod.TetMesh(x=x, ien=meshmod._orient(x, ien.astype(np.int32)).astype(np.int32))
+    for k in ("Ag", "Yg", "Dg"):
+        setattr(prob, k, np.zeros((points + 1, 3)))
+    prob.Dg = 1e-3 * rng.normal(size=(points + 1, 3))
+    prob.dir_faces, prob.trac_faces = [(np.arange(4, dtype=np.int32), 3)], []
+    return prob
+
+
+CASES = {
+    "lelas_1part": lambda: problems.lelas_cube(3),
+    "lelas_parts": lambda: problems.lelas_cube(13),
+    "lelas_all_cus": lambda: problems.lelas_cube(27),
+    "fluid_few": lambda: problems.fluid_cylinder(h=0.5),
+    "fluid_mid": lambda: problems.fluid_cylinder(h=0.22),
+    "hub_16_lanes": lambda: hub(40),
+    "hub_64_lanes": lambda: hub(150),
+    "hub_no_fit": lambda: hub(400),
+    "tet10": lambda: problems.struct_cube(3, Kpen=1e5),
+}
+
+
+def solve(prob, monkeypatch, persist, wait=None):
+    import torch
+
+    from svfsi_amd.step import NewtonStep
+
+    monkeypatch.setenv("SVFSI_PERSIST", persist)
+    if wait is None:
+        monkeypatch.delenv("SVFSI_PERSIST_WAIT", raising=False)
+    else:
+        monkeypatch.setenv("SVFSI_PERSIST_WAIT", wait)
+    st = NewtonStep(prob)
+    out = []
+    for _ in range(2):  # the second solve reuses the partition and its exchange buffer
+        ls = st.step(mixed=True)
+        torch.cuda.synchronize()
+        out.append((st.R.cpu().numpy().copy(), ls.RI.itr, ls.RI.suc))
+    assert np.array_equal(out[0][0], out[1][0])
+    return out[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(CASES))
+def test_matches_one_launch_per_factor(gpu, monkeypatch, name):
+    prob = CASES[name]()
+    x, itr, suc = solve(prob, monkeypatch, "1")
+    y, itr0, suc0 = solve(prob, monkeypatch, "0")
+    assert suc == suc0 == 1 and abs(itr - itr0) <= 1
+    # both solve to 1e-8 in the scaled residual
+    assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+
+
+@pytest.mark.gpu
+def test_gives_up_and_falls_back(gpu, monkeypatch):
+    """A wait of no ticks: the kernel ends at the first word not yet there and
+    the solve runs again with one launch per factor, to the same bits."""
+    prob = problems.lelas_cube(13)
+    x, itr, suc = solve(prob, monkeypatch, "1", wait="0")
+    y, itr0, suc0 = solve(prob, monkeypatch, "0")
+    assert suc == suc0 == 1 and itr == itr0
+    assert np.array_equal(x, y)
+
+
+@pytest.mark.gpu
+def test_two_threads(gpu, monkeypatch):
+    """Two solves at once on streams of their own, one of which finds the
+    matrix-resident path taken."""
+    import torch
+
+    from svfsi_amd.step import NewtonStep
+
+    monkeypatch.setenv("SVFSI_PERSIST", "1")
+    probs = [problems.lelas_cube(11), problems.fluid_cylinder(h=0.3)]
+    want = [solve(p, monkeypatch, "0") for p in probs]
+    monkeypatch.setenv("SVFSI_PERSIST", "1")
+    steps = [NewtonStep(p) for p in probs]
+    torch.cuda.synchronize()
+    got = [None, None]
+
+    def work(i):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(4):
+                ls = steps[i].step(mixed=True)
+            s.synchronize()
+            got[i] = (steps[i].R.cpu().numpy(), ls.RI.itr, ls.RI.suc)
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in (0, 1)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    for (x, itr, suc), (y, itr0, _) in zip(got, want):
+        assert suc == 1 and abs(itr - itr0) <= 1
+        assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
