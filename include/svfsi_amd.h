@@ -362,8 +362,10 @@ typedef struct {
 
 /* STRUCT (tet10) element kernel, ORed into svfsi_assemble_dev's quad.  No
  * counterpart in the reference (STRUCT3D is one FP64 code path there):
- *   VALU   -- FP64 vector units throughout;
- *   MFMA64 -- B^T Dm B on FP64 matrix cores (the default);
+ *   AUTO   -- the tangent as outer products on FP64 vector units and a row
+ *             gather (the default);
+ *   VALU   -- B^T Dm B on FP64 vector units throughout;
+ *   MFMA64 -- B^T Dm B on FP64 matrix cores;
  *   MFMA32 -- B^T Dm B on FP32 matrix cores with FP32 accumulation (the
  *             rest, and the accumulation into Val, stays FP64). */
 /* FLUID on a tet10 mesh: the Taylor-Hood (P2P1) basis of svFSI's nFs = 2
@@ -401,7 +403,7 @@ int svfsi_zero_dev(void* mesh, int dof, double* dVal, double* dR, void* stream);
  * device (tDof,nNo).  prop_el: optional per-element property (LELAS E_e,
  * FLUID mu_e, NULL = uniform).  quad: 0 = the reference rule (tet4 4-pt,
  * tet10 15-pt), 1 = tet10 4-point rule; for STRUCT, OR one of the
- * SVFSI_STRUCT_* kernel selectors above into quad (default: MFMA64); FLUID
+ * SVFSI_STRUCT_* kernel selectors above into quad (default: AUTO); FLUID
  * on a tet10 mesh takes quad = SVFSI_FLUID_P2P1 (the reference's rules). */
 int svfsi_assemble_dev(void* mesh, int phys, const svfsi_eq_params* p,
                        int tDof, const double* dAg, const double* dYg,

@@ -776,6 +776,12 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
         gsrc.resize(gslot.size());
         for (size_t q = 0; q < gslot.size(); ++q) gsrc[gslot[q]] = (int)q;
     }
+    std::vector<int> rsrc;
+    if (eNoN == 10) {
+        rsrc.resize(rslot.size());
+        for (size_t q = 0; q < rslot.size(); ++q) rsrc[rslot[q]] = (int)q;
+    }
+    for (int i = 0; i < nNo; ++i) M->maxRow = std::max(M->maxRow, L.hRowPtr[i + 1] - L.hRowPtr[i]);
     std::vector<double> xv(x, x + (size_t)3 * nNo);
     // mid-edge nodes (local 5..10 of a tet10), whose pressure rows
     // THOOD_ValRC resets in a Taylor-Hood FLUID assembly (FS.f:383-391)
@@ -791,6 +797,7 @@ int svfsi_mesh_create(void** mesh, void* lhs, int nNo, int nEl, int eNoN, const 
     int rc = SVFSI_OK;
     if ((rc = upload(M->ien, sien)) || (rc = upload(M->elemId, order)) || (rc = upload(M->emap, emap)) ||
         (rc = upload(M->x, xv)) || (rc = upload(M->gPtr, gptr)) || (rc = eNoN == 4 ? upload(M->gSrc, gsrc) : upload(M->gSlot, gslot)) || (rc = upload(M->gTile, gtile)) ||
+        (rc = upload(M->rSrc, rsrc)) ||
         (rc = upload(M->rPtr, rptr)) || (rc = upload(M->rSlot, rslot)) ||
         (!mids.empty() && (rc = upload(M->midNodes, mids)))) {
         delete M;

@@ -1861,6 +1861,267 @@ __global__ __launch_bounds__(256) void k_asm_struct_mfma(int begin, int count, c
 }
 
 // ---------------------------------------------------------------------------
+// STRUCT3D, the default kernels: the neo-Hookean tangent as outer products,
+// and a row gather.
+//
+// GETPK2CC's tangent is Dm = -2/3 (Ci x Sd + Sd x Ci) + 2 (r1 - p J) (Ci o Ci)
+// + (pl J - 2 r1/3) Ci x Ci with Sd = s I - r1 Ci (s = 2 C10 J^(-2/3), r1 = s
+// tr(C)/3), and the strain operator turns a symmetric tensor X into
+// B_a^T X = F X Nx_a.  With m_a = F Nx_a and n_a = F Ci Nx_a = F^-T Nx_a
+// (F Ci F^T = I) the material and geometric parts of block (a,b) are, at a
+// point,
+//   -2/3 s (n_a m_b^T + m_a n_b^T) + (pl J + 2 r1/3) n_a n_b^T
+//   + (r1 - p J) n_b n_a^T + s (Nx_a.Nx_b) I
+// (the (r1 - p J) n_a.n_b of the material part and of Nx_a.S.Nx_b cancel), and
+// the residual's F S Nx_a = s m_a - (r1 - p J) n_a.  That is 38 multiply-adds
+// per block and point, where the 6x6 contraction B_a^T Dm B_b takes 54 and
+// Dm B_b another 108 per node: the vector units need 30 us for the 82,944
+// elements of the 24^3 cube at the 4-point rule, less than staging the
+// operands for the matrix cores.
+//
+// k_struct_elem: a lane per (element, point) writes the point's node vectors
+// to LDS, then 50 lanes per element each sum two neighbouring blocks of a row
+// over the points and store them, element blocks contiguous (7.2 KB).
+// k_struct_rows: a wavefront per node adds the 720-byte strips of its
+// elements into the node's row of Val, in LDS, in element-id order.  The
+// scatter of the coloured kernels (30 launches, each a read-modify-write of
+// scattered 72-byte blocks) took 1.22 ms of the 1.41 ms there; these two
+// launches 837 us (4,374 elements, 15-point rule: 559 -> 67 us).
+// ---------------------------------------------------------------------------
+constexpr int SN_SZ = 10;                   // per node: Nx, n, m (scaled), pad
+constexpr int SQ_C = 10 * SN_SZ;            // then w s, w (pl J + 2 r1/3), w (r1 - p J), w
+constexpr int SQ_UD = SQ_C + 4, SQ_SZ = SQ_UD + 4;
+
+// One material point to LDS: node vectors Nx_a, n_a and w (-2/3 s) m_a, and
+// the scalars above (all without the factor af beta dt^2).
+__device__ __forceinline__ void struct_point_vec(int e, const int* __restrict__ ien, const double* __restrict__ x,
+                                                 int tDof, const double* __restrict__ Ag,
+                                                 const double* __restrict__ Dg, const AsmParams& P,
+                                                 const double* __restrict__ rg, double* rc)
+{
+    double A[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll 5
+    for (int a = 0; a < 10; ++a) {
+        const int na = ien[(size_t)e * 10 + a];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double xi = x[(size_t)na * 3 + i];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) A[i][j] += xi * rg[11 + a * 3 + j];
+        }
+    }
+    const double J = A[0][0] * A[1][1] * A[2][2] + A[0][1] * A[1][2] * A[2][0]
+                   + A[0][2] * A[1][0] * A[2][1] - A[0][0] * A[1][2] * A[2][1]
+                   - A[0][1] * A[1][0] * A[2][2] - A[0][2] * A[1][1] * A[2][0];
+    double B[3][3];
+    B[0][0] = (A[1][1] * A[2][2] - A[1][2] * A[2][1]) / J;
+    B[0][1] = (A[2][1] * A[0][2] - A[2][2] * A[0][1]) / J;
+    B[0][2] = (A[0][1] * A[1][2] - A[0][2] * A[1][1]) / J;
+    B[1][0] = (A[1][2] * A[2][0] - A[1][0] * A[2][2]) / J;
+    B[1][1] = (A[2][2] * A[0][0] - A[2][0] * A[0][2]) / J;
+    B[1][2] = (A[0][2] * A[1][0] - A[0][0] * A[1][2]) / J;
+    B[2][0] = (A[1][0] * A[2][1] - A[1][1] * A[2][0]) / J;
+    B[2][1] = (A[2][0] * A[0][1] - A[2][1] * A[0][0]) / J;
+    B[2][2] = (A[0][0] * A[1][1] - A[0][1] * A[1][0]) / J;
+    double F[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
+    double ud[3] = {-P.rho * P.fb[0], -P.rho * P.fb[1], -P.rho * P.fb[2]};
+#pragma unroll 5
+    for (int a = 0; a < 10; ++a) {
+        const int na = ien[(size_t)e * 10 + a];
+        double Nxa[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            Nxa[j] = rg[11 + a * 3] * B[0][j] + rg[11 + a * 3 + 1] * B[1][j] + rg[11 + a * 3 + 2] * B[2][j];
+            rc[a * SN_SZ + j] = Nxa[j];
+        }
+        const double Na = rg[1 + a];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double Dai = Dg[(size_t)na * tDof + i];
+            ud[i] += Na * (P.rho * Ag[(size_t)na * tDof + i]);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) F[i][j] += Nxa[j] * Dai;
+        }
+    }
+    const double Jf = det3d(F);
+    double Fi[3][3]; // F^-T
+    Fi[0][0] = (F[1][1] * F[2][2] - F[1][2] * F[2][1]) / Jf;
+    Fi[0][1] = (F[1][2] * F[2][0] - F[1][0] * F[2][2]) / Jf;
+    Fi[0][2] = (F[1][0] * F[2][1] - F[1][1] * F[2][0]) / Jf;
+    Fi[1][0] = (F[0][2] * F[2][1] - F[0][1] * F[2][2]) / Jf;
+    Fi[1][1] = (F[0][0] * F[2][2] - F[0][2] * F[2][0]) / Jf;
+    Fi[1][2] = (F[0][1] * F[2][0] - F[0][0] * F[2][1]) / Jf;
+    Fi[2][0] = (F[0][1] * F[1][2] - F[0][2] * F[1][1]) / Jf;
+    Fi[2][1] = (F[0][2] * F[1][0] - F[0][0] * F[1][2]) / Jf;
+    Fi[2][2] = (F[0][0] * F[1][1] - F[0][1] * F[1][0]) / Jf;
+    double p = 0.0, pl = 0.0, trC = 0.0;
+    const double Kp = P.Kpen;
+    if (!iszero_d(Kp)) {
+        if (P.volType == 1) { p = Kp * (Jf - 1.0); pl = Kp * (2.0 * Jf - 1.0); }
+        else if (P.volType == 3) { p = Kp * (1.0 - 1.0 / Jf); pl = Kp; }
+        else { p = 0.5 * Kp * (Jf - 1.0 / Jf); pl = Kp * Jf; }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) trC += F[i][j] * F[i][j];
+    const double w = rg[0] * J;
+    const double s = pow(Jf, -2.0 / 3.0) * (2.0 * P.C10);
+    const double r1 = s * trC / 3.0;
+    const double ws = w * s, cm = -2.0 / 3.0 * ws;
+    rc[SQ_C] = ws;
+    rc[SQ_C + 1] = w * (pl * Jf + 2.0 * r1 / 3.0);
+    rc[SQ_C + 2] = w * (r1 - p * Jf);
+    rc[SQ_C + 3] = w;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rc[SQ_UD + i] = ud[i];
+#pragma unroll 5
+    for (int a = 0; a < 10; ++a) {
+        double* na = rc + a * SN_SZ;
+        const double n0 = na[0], n1 = na[1], n2 = na[2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            na[3 + i] = Fi[i][0] * n0 + Fi[i][1] * n1 + Fi[i][2] * n2;
+            na[6 + i] = cm * (F[i][0] * n0 + F[i][1] * n1 + F[i][2] * n2);
+        }
+    }
+}
+
+template <int NG, int EPW, int NT>
+__global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restrict__ ien,
+                                                    const double* __restrict__ x, int tDof,
+                                                    const double* __restrict__ Ag, const double* __restrict__ Dg,
+                                                    AsmParams P, const double* __restrict__ rule,
+                                                    double* __restrict__ ke, double* __restrict__ re)
+{
+    static_assert(EPW * NG <= NT && EPW * 50 <= NT, "one pass of lanes per phase");
+    __shared__ __align__(16) double rec[EPW * NG][SQ_SZ];
+    __shared__ double sN[NG][10];
+    const int tid = threadIdx.x;
+    const int e0 = blockIdx.x * EPW;
+    for (int i = tid; i < NG * 10; i += NT) sN[i / 10][i % 10] = rule[(i / 10) * kTet10Rec + 1 + i % 10];
+    if (tid < EPW * NG) {
+        const int k = tid / NG, g = tid - k * NG;
+        if (e0 + k < nEl) struct_point_vec(e0 + k, ien, x, tDof, Ag, Dg, P, rule + g * kTet10Rec, rec[tid]);
+    }
+    __syncthreads();
+    const int k = tid / 50, r = tid - k * 50, e = e0 + k;
+    if (k >= EPW || e >= nEl) return;
+    {
+#pragma clang fp contract(fast) // the Jacobians are behind: see the top of the file
+        const int a = r / 5, b0 = 2 * (r - 5 * a);
+        double K[2][9], T[2] = {0, 0}, M[2] = {0, 0}, R[3] = {0, 0, 0};
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 9; ++q) K[h][q] = 0.0;
+#pragma unroll 1
+        for (int g = 0; g < NG; ++g) {
+            const double* rc = rec[k * NG + g];
+            double na[SN_SZ];
+#pragma unroll
+            for (int q = 0; q < SN_SZ / 2; ++q) {
+                const d2_t v = *reinterpret_cast<const d2_t*>(rc + a * SN_SZ + 2 * q);
+                na[2 * q] = v.x;
+                na[2 * q + 1] = v.y;
+            }
+            const double ws = rc[SQ_C], kap = rc[SQ_C + 1], gam = rc[SQ_C + 2], w = rc[SQ_C + 3];
+            const double Na = sN[g][a];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                double nb[SN_SZ];
+#pragma unroll
+                for (int q = 0; q < SN_SZ / 2; ++q) {
+                    const d2_t v = *reinterpret_cast<const d2_t*>(rc + (b0 + h) * SN_SZ + 2 * q);
+                    nb[2 * q] = v.x;
+                    nb[2 * q + 1] = v.y;
+                }
+                T[h] += ws * (na[0] * nb[0] + na[1] * nb[1] + na[2] * nb[2]);
+                M[h] += w * (Na * sN[g][b0 + h]);
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const double eb = kap * nb[3 + j] + nb[6 + j]; // n_a's partner
+                    const double ga = gam * na[3 + j];             // n_b's, transposed
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        K[h][i * 3 + j] += na[3 + i] * eb + na[6 + i] * nb[3 + j] + nb[3 + i] * ga;
+                }
+            }
+            if (b0 == 0) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) R[i] += w * (Na * rc[SQ_UD + i]) - 1.5 * na[6 + i] - gam * na[3 + i];
+            }
+        }
+        const double afu = P.af * P.beta * P.dt * P.dt, amd = P.am * P.rho;
+        double* o = ke + ((size_t)e * 100 + a * 10 + b0) * 9; // two blocks: 144 B, 16-byte aligned
+        double v[18];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 9; ++q) v[9 * h + q] = afu * K[h][q] + (q % 4 == 0 ? amd * M[h] + afu * T[h] : 0.0);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) *reinterpret_cast<d2_t*>(o + 2 * q) = d2_t{v[2 * q], v[2 * q + 1]};
+        if (b0 == 0) {
+            double* rr = re + ((size_t)e * 10 + a) * 3;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) rr[i] = R[i];
+        }
+    }
+}
+
+// Row of Val and of R of node i: a wavefront adds the strips ke[(e, a)][0..89]
+// of the node's elements (rSrc = 10 e + a, in element-id order) into LDS.  Its
+// LDS additions are issued strip by strip and complete in that order, and a
+// strip's 90 values go to 90 places, so the sums are in element order; four
+// strips' loads are in flight.
+__global__ __launch_bounds__(256) void k_struct_rows(int nNo, int maxRow, const int* __restrict__ rowPtr,
+                                                     const int* __restrict__ rPtr, const int* __restrict__ rSrc,
+                                                     const int* __restrict__ emap, const double* __restrict__ ke,
+                                                     const double* __restrict__ re, double* __restrict__ val,
+                                                     double* __restrict__ R)
+{
+    extern __shared__ double accs[];
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+    const int i = (int)xcd_part(blockIdx.x, gridDim.x) * 4 + wave;
+    if (i >= nNo) return;
+    double* acc = accs + (size_t)wave * maxRow * 9;
+    const int k0 = rowPtr[i], nv = (rowPtr[i + 1] - k0) * 9;
+    for (int q = l; q < nv; q += 64) acc[q] = 0.0;
+    const int b1 = l / 9, q1 = l - 9 * b1;               // value l of a strip
+    const int b2 = (l + 64) / 9, q2 = l + 64 - 9 * b2;   // value l + 64, l < 26
+    const int s1 = rPtr[i + 1];
+    double r = 0.0;
+    for (int s = rPtr[i]; s < s1; s += 4) {
+        double u[4], v[4], rv[4];
+        int m[4], n[4];
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+            if (s + h < s1) {
+                const size_t src = (size_t)rSrc[s + h];
+                m[h] = emap[src * 10 + b1];
+                u[h] = ke[src * 90 + l];
+                n[h] = l < 26 ? emap[src * 10 + b2] : 0;
+                v[h] = l < 26 ? ke[src * 90 + l + 64] : 0.0;
+                rv[h] = l < 3 ? re[src * 3 + l] : 0.0;
+            }
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+            if (s + h < s1) {
+                __hip_atomic_fetch_add(acc + (size_t)(m[h] - k0) * 9 + q1, u[h], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (l < 26)
+                    __hip_atomic_fetch_add(acc + (size_t)(n[h] - k0) * 9 + q2, v[h], __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                r += rv[h];
+            }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    double* o = val + (size_t)k0 * 9;
+    for (int q = l; q < nv; q += 64) o[q] += acc[q];
+    if (l < 3) R[(size_t)i * 3 + l] += r;
+}
+
+// ---------------------------------------------------------------------------
 // Gather assembly: Val(:, j) += the sum of the element blocks that land on
 // nnz block j, R(:, i) += the sum of node i's element residual rows.  The
 // element kernels stored those contributions contiguously, in element-id
@@ -2042,7 +2303,32 @@ int launch_asm_struct(Mesh& M, const AsmParams& P, int nG, const double* rule, i
         set_error("STRUCT: nG %d not supported", nG);
         return SVFSI_ERR_NOTSUP;
     }
-    if (kern == SVFSI_STRUCT_AUTO) kern = SVFSI_STRUCT_MFMA64;
+    if (kern == SVFSI_STRUCT_AUTO) {
+        // the outer-product kernels and their row gather, unless a row of Val
+        // is too long for four of them in LDS or the coloured scatter is asked
+        // for (SVFSI_ASM_GATHER=0)
+        const char* v = getenv("SVFSI_ASM_GATHER");
+        const size_t lds = (size_t)M.maxRow * 9 * 4 * sizeof(double);
+        if (lds <= ((size_t)64 << 10) && !(v && v[0] == '0')) {
+            SV_TRY(M.ke.ensure((size_t)M.nEl * 100 * 9 * sizeof(double)));
+            SV_TRY(M.re.ensure((size_t)M.nEl * 10 * 3 * sizeof(double)));
+            double* ke = M.ke.as<double>();
+            double* re = M.re.as<double>();
+            constexpr int E4 = 10, E15 = 5;
+            if (nG == 4)
+                hipLaunchKernelGGL((k_struct_elem<4, E4, 512>), dim3((unsigned)((M.nEl + E4 - 1) / E4)), dim3(512), 0,
+                                   s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule, ke, re);
+            else
+                hipLaunchKernelGGL((k_struct_elem<15, E15, 256>), dim3((unsigned)((M.nEl + E15 - 1) / E15)), dim3(256),
+                                   0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule, ke, re);
+            hipLaunchKernelGGL(k_struct_rows, dim3((unsigned)((M.nNo + 3) / 4)), dim3(256), lds, s, M.nNo, M.maxRow,
+                               M.lhs->rowPtr.as<int>(), M.rPtr.as<int>(), M.rSrc.as<int>(), M.emap.as<int>(),
+                               (const double*)ke, (const double*)re, val, R);
+            SV_HIP(hipGetLastError());
+            return SVFSI_OK;
+        }
+        kern = SVFSI_STRUCT_MFMA64;
+    }
     if (kern != SVFSI_STRUCT_VALU && kern != SVFSI_STRUCT_MFMA64 && kern != SVFSI_STRUCT_MFMA32) {
         set_error("STRUCT: unknown kernel selector %d", kern);
         return SVFSI_ERR_ARG;

@@ -224,8 +224,10 @@ struct Mesh {
     // instead: contribution k is block gSrc[k] = p*16 + a*4 + b.
     // The tet4 gather's tiles: tile b is nnz entries gTile[b] .. gTile[b+1]-1,
     // together at most kGatherTile contributions (or a single entry).
-    DBuf gPtr, gSlot, gSrc, gTile, rPtr, rSlot;
-    int nGTile = 0;
+    // tet10: rSrc is rSlot's inverse, node i's element rows p*10 + a at
+    // rPtr[i] .. rPtr[i+1]-1; maxRow the longest row of the pattern.
+    DBuf gPtr, gSlot, gSrc, gTile, rPtr, rSlot, rSrc;
+    int nGTile = 0, maxRow = 0;
     DBuf ke, re;     // element blocks or records / element residual rows, grown on demand
     ~Mesh() {
         for (auto* f : faceSets) delete f;

@@ -170,3 +170,24 @@ def test_assembly_hub_node(gpu, orc, kind, points):
         setattr(prob, k, rng.normal(size=(m.nNo, prob.dof)))
     for got, want in assembled(prob, orc):
         assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * max(1.0, np.abs(want).max())
+
+
+VOL = {"quad": dict(volType=1), "st91": dict(volType=2), "m94": dict(volType=3), "none": dict(Kpen=0.0)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vol", list(VOL))
+@pytest.mark.parametrize("nEl,tDof,quad", [(1, 3, 0), (5, 3, 0), (6, 4, 0), (162, 3, 0), (9, 3, 1), (10, 7, 1),
+                                           (11, 3, 1), (162, 4, 1)])
+def test_struct_assembly_sizes(gpu, orc, nEl, tDof, quad, vol):
+    prob = problems.struct_cube(n=3, quad=quad)
+    rng = np.random.default_rng(7)
+    prob.Ag = rng.normal(size=(prob.nNo, 3))
+    # |grad u| <= 0.004 * sum_a |grad N_a| <= 0.004 * (6 + 12) * 3 sqrt(2) < 1/3
+    # per entry: F is diagonally dominant, no element is inverted
+    prob.Dg = rng.uniform(-0.004, 0.004, size=(prob.nNo, 3))
+    prob.Ag, prob.Dg = wide(prob.Ag, tDof, rng), wide(prob.Dg, tDof, rng)
+    prob.Yg = np.zeros_like(prob.Dg)
+    prob.eq = dict(prob.eq, fb=(0.3, -0.2, 0.1), **VOL[vol])
+    for got, want in assembled(first_elements(prob, nEl), orc):
+        assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * np.abs(want).max()
