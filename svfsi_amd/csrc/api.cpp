@@ -1,5 +1,6 @@
 // api.cpp -- extern "C" entry points of libsvfsi_amd (see include/svfsi_amd.h).
 #include "internal.hpp"
+#include "persist.hpp"
 #include "assemble.hpp"
 
 #include <algorithm>
@@ -481,6 +482,7 @@ int fsils_gpu_lhs_create(void** lhs, int gnNo, int nNo, int nnz, const int* gNod
         delete L;
         return rc;
     }
+    persist_build(*L);
     *lhs = L;
     return SVFSI_OK;
 }

@@ -134,7 +134,7 @@ struct Work {
     GraphCache cgGraphs; // CG: one graph for a chunk of iterations
     GraphCache csGraphs; // NS solver's Schur-complement CG: likewise
     PinnedPoll poll;
-    DBuf W, X, R0, tmp, basis, basis32, Z32, val32, x32, y32;
+    DBuf W, X, tmp, basis, basis32, Z32, val32, x32, y32;
     DBuf partial, state, hess;
     DBuf zdir, opartial, ostate, ohess; // flexible GMRES: FP32 directions, outer state
     DBuf mask;

@@ -13,6 +13,7 @@
 #include "devutil.hpp"
 #include "stream.hpp"
 #include "persist.hpp"
+#include "cgstate.hpp"
 
 #include <chrono>
 #include <cmath>
@@ -31,14 +32,6 @@ double wall_seconds()
 // ===========================================================================
 // CGRADV (svFSILS/CGRAD.f:184-242)
 // ===========================================================================
-struct CgState {
-    double err, errO, alpha, eps;
-    int done, suc, itr, mItr;
-    unsigned int counter;
-    int pad;
-    double e[2]; // |R|^2 of the current and the next iteration, by iteration parity
-};
-
 // Every reduction ends at a kernel boundary (no last-block fences, which on
 // a multi-XCD part write back L2): a kernel writes per-block partials and
 // each block of the next kernel sums them in the same fixed order, so all
@@ -507,17 +500,33 @@ int cg_core(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hi
             w.cgGraphs.sig = sig;
         }
     }
+    // dof 3: chunks of iterations as one matrix-resident launch each where the
+    // matrix fits the chip (pcg.hip); KP, not used by them, keeps the
+    // right-hand side for the case that such a launch gives up
+    PersistLock plock;
+    Parts* parts = nullptr;
+    if (dof == 3 && !h0.done && plock.acquire()) {
+        parts = persist_parts(L);
+        if (parts && !pcg_fits(*parts)) parts = nullptr;
+        if (parts) {
+            SV_HIP(hipMemcpyAsync(KP, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+        } else {
+            plock.release();
+        }
+    }
     int posted = 0;
     CgState hs = h0;
     bool finished = h0.done != 0;
     int launched = 0;
     while (!finished) {
         const int q = posted & 1;
-        if (useGraphs)
+        if (parts)
+            SV_TRY(pcg3_launch(L, *parts, K, X, R, P, st, kPcgChunk, s));
+        else if (useGraphs)
             SV_TRY(graph_run(w.cgGraphs, 0, s, iters));
         else
             SV_TRY(iters(s));
-        launched += chunk;
+        launched += parts ? kPcgChunk : chunk;
         if (pinned) {
             SV_TRY(w.poll.post(q, st, sizeof(CgState), s));
             ++posted;
@@ -532,7 +541,21 @@ int cg_core(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hi
             SV_HIP(hipStreamSynchronize(s));
             if (hs.done) finished = true;
         }
-        if (launched > ls.mItr + 2 * chunk) break; // safety: flag must be set by now
+        if (parts && finished && hs.abort) {
+            SV_HIP(hipStreamSynchronize(s));
+            parts->off = true;
+            parts = nullptr;
+            plock.release();
+            SV_HIP(hipMemcpyAsync(R, KP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+            SV_HIP(hipMemcpyAsync(P, KP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+            SV_HIP(hipMemcpyAsync(st, &h0, sizeof(CgState), hipMemcpyHostToDevice, s));
+            SV_TRY(launch_fill(n, 0.0, X, s));
+            SV_HIP(hipStreamSynchronize(s));
+            finished = false;
+            posted = launched = 0;
+            continue;
+        }
+        if (launched > ls.mItr + 2 * (parts ? kPcgChunk : chunk)) break; // safety: flag must be set by now
     }
     SV_HIP(hipStreamSynchronize(s));
     SV_HIP(hipMemcpyAsync(&hs, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
@@ -991,6 +1014,18 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
             w.csGraphs.sig = sig;
         }
     }
+    // matrix-resident chunks as in cg_core
+    PersistLock plock;
+    Parts* parts = nullptr;
+    if (!cpl && !h0.done && !prof().on && plock.acquire()) {
+        parts = persist_parts(L);
+        if (parts && !pcg_fits(*parts)) parts = nullptr;
+        if (parts) {
+            SV_HIP(hipMemcpyAsync(SP, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+        } else {
+            plock.release();
+        }
+    }
     int posted = 0;
     CgState hs = h0;
     bool finished = h0.done != 0;
@@ -998,11 +1033,13 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
     while (!finished) {
         const int q = posted & 1;
         const bool firstChunk = launched == 0;
-        if (useGraphs)
+        if (parts)
+            SV_TRY(pcgs_launch(L, *parts, Lm, G, Gt, X, R, buf[1], st, kPcgChunk, s));
+        else if (useGraphs)
             SV_TRY(graph_run(w.csGraphs, firstChunk ? 0 : 1, s, [&](hipStream_t cs) { return iters(cs, firstChunk); }));
         else
             SV_TRY(iters(s, firstChunk));
-        launched += chunk;
+        launched += parts ? kPcgChunk : chunk;
         SV_TRY(poll.post(q, st, sizeof(CgState), s));
         ++posted;
         if (posted >= 2) {
@@ -1010,9 +1047,23 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
             std::memcpy(&hs, poll.h[q ^ 1], sizeof(CgState));
             if (hs.done) finished = true;
         }
+        if (parts && finished && hs.abort) {
+            SV_HIP(hipStreamSynchronize(s));
+            parts->off = true;
+            parts = nullptr;
+            plock.release();
+            SV_HIP(hipMemcpyAsync(R, SP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+            SV_HIP(hipMemcpyAsync(buf[1], SP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+            SV_HIP(hipMemcpyAsync(st, &h0, sizeof(CgState), hipMemcpyHostToDevice, s));
+            SV_TRY(launch_fill(n, 0.0, X, s));
+            SV_HIP(hipStreamSynchronize(s));
+            finished = false;
+            posted = launched = 0;
+            continue;
+        }
         // the last iteration's bookkeeping runs at the next chunk's start:
         // one chunk beyond mItr at most
-        if (launched > ls.mItr + 3 * chunk) break; // safety: the flag is set by now
+        if (launched > ls.mItr + 3 * (parts ? kPcgChunk : chunk)) break; // safety: the flag is set by now
     }
     SV_HIP(hipStreamSynchronize(s));
     SV_HIP(hipMemcpy(&hs, st, sizeof(CgState), hipMemcpyDeviceToHost));

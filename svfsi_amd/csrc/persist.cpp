@@ -5,25 +5,26 @@
 #include <atomic>
 #include <climits>
 #include <cstdlib>
+#include <cstring>
+#include <mutex>
 #include <thread>
 
 namespace svfsi {
 
-static std::atomic<int> g_busy[64];
+static std::mutex g_mu[64];
 
 bool PersistLock::acquire()
 {
     int d = 0;
     if (hipGetDevice(&d) != hipSuccess || d < 0 || d >= 64) return false;
-    int expected = 0;
-    if (!g_busy[d].compare_exchange_strong(expected, 1)) return false;
+    g_mu[d].lock();
     dev = d;
     return true;
 }
 
 void PersistLock::release()
 {
-    if (dev >= 0) g_busy[dev].store(0);
+    if (dev >= 0) g_mu[dev].unlock();
     dev = -1;
 }
 
@@ -31,14 +32,6 @@ void PersistLock::release()
 size_t ppoly_lds(const Parts& P)
 {
     return (size_t)(P.maxOwn + P.maxHalo) * 32 + (size_t)P.maxHalo * 4;
-}
-
-template <typename T>
-static int put(DBuf& b, const std::vector<T>& v)
-{
-    SV_TRY(b.ensure(v.size() * sizeof(T)));
-    if (!v.empty()) SV_HIP(hipMemcpy(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-    return SVFSI_OK;
 }
 
 // lanes of a row of n blocks: the smallest power of two from gMin on that
@@ -53,8 +46,9 @@ static int row_lanes(int n, int U, int gMin)
 // U blocks per lane and rows of at least gMin lanes; P.G stays 0 when the
 // pattern does not fit.
 //
-// The cost falls on the first solve of a pattern: about 3.5 ms for the 200k-tet
-// cylinder (8.5 with the halos found by one thread).
+// Part of FSILS_LHS_CREATE, so that every solve of a pattern takes the same
+// path: about 3.5 ms for the 200k-tet cylinder (8.5 with the halos found by one
+// thread).
 static int build(Lhs& L, Parts& P, int U, int gMin, int cus, size_t ldsMax)
 {
     const std::vector<int>& rp = L.hRowPtr;
@@ -198,15 +192,25 @@ static int build(Lhs& L, Parts& P, int U, int gMin, int cus, size_t ldsMax)
         P.maxHalo = std::max(P.maxHalo, (int)h.size());
     }
     if (ppoly_lds(P) + 64 > ldsMax) return SVFSI_OK;
-    SV_TRY(put(P.rowOff, rowOff));
-    SV_TRY(put(P.rowId, rowId));
-    SV_TRY(put(P.laneOff, laneOff));
-    SV_TRY(put(P.lane, lane));
-    SV_TRY(put(P.hOff, hOff));
-    SV_TRY(put(P.hPos, hPos));
-    SV_TRY(put(P.lcol, lcol));
-    SV_TRY(P.xb.ensure((size_t)n * 8 * sizeof(unsigned long long)));
-    SV_HIP(hipMemset(P.xb.p, 0, (size_t)n * 8 * sizeof(unsigned long long)));
+    // one array for all tables
+    const std::vector<int>* tabs[6] = {&rowOff, &rowId, &laneOff, &lane, &hOff, &hPos};
+    size_t ints = 0;
+    for (int i = 0; i < 6; ++i) {
+        P.at[i] = ints;
+        ints += tabs[i]->size();
+    }
+    P.at[6] = ints;
+    std::vector<int> all(ints + (lcol.size() + 1) / 2);
+    for (int i = 0; i < 6; ++i) std::copy(tabs[i]->begin(), tabs[i]->end(), all.begin() + P.at[i]);
+    std::memcpy(all.data() + ints, lcol.data(), lcol.size() * sizeof(unsigned short));
+    SV_TRY(P.tab.ensure(all.size() * sizeof(int)));
+    SV_HIP(hipMemcpy(P.tab.p, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice));
+    // the exchange buffer and the partials of two sums over all parts, tag 0
+    P.red = (size_t)n * 16;
+    const size_t words = P.red + (size_t)G * 4;
+    SV_TRY(P.xb.ensure(words * sizeof(unsigned long long)));
+    SV_HIP(hipMemset(P.xb.p, 0, words * sizeof(unsigned long long)));
+    P.ldsMax = ldsMax;
     P.U = U;
     P.G = (int)G;
     return SVFSI_OK;
@@ -225,31 +229,28 @@ static int choose(Lhs& L, Parts& P)
     return SVFSI_OK;
 }
 
+void persist_build(Lhs& L)
+{
+    // the exchange needs a structurally symmetric pattern (persist.hpp)
+    if (!L.symmetric) return;
+    try {
+        std::shared_ptr<Parts> P = std::make_shared<Parts>();
+        if (choose(L, *P) != SVFSI_OK) (void)hipGetLastError();
+        else if (P->G > 0) L.parts = P;
+    } catch (...) { // out of host memory: no parts
+    }
+}
+
 Parts* persist_parts(Lhs& L)
 {
     // SVFSI_PERSIST=0: one launch per product throughout (read at each call)
     const char* e = getenv("SVFSI_PERSIST");
-    if (e && e[0] == '0') return nullptr;
-    try {
-        if (!L.parts) L.parts = std::make_shared<Parts>();
-        Parts& P = *L.parts;
-        if (!P.tried) {
-            P.tried = true;
-            // the exchange needs a structurally symmetric pattern (persist.hpp)
-            if (L.symmetric && L.nNo > 0 && (int)L.hRowPtr.size() == L.nNo + 1 && choose(L, P) != SVFSI_OK) {
-                (void)hipGetLastError();
-                P.G = 0;
-            }
-        }
-    } catch (...) { // out of host memory: G is still 0
-        return nullptr;
-    }
-    Parts& P = *L.parts;
+    if (!L.parts || L.parts->off || (e && e[0] == '0')) return nullptr;
     // SVFSI_PERSIST_WAIT: ticks of 10 ns a lane waits before it gives up; 0:
     // at the first word that is not there yet (tests of that path)
     const char* w = getenv("SVFSI_PERSIST_WAIT");
-    P.wait = w ? strtoull(w, nullptr, 10) : kWaitTicks;
-    return P.G > 0 && !P.off ? &P : nullptr;
+    L.parts->wait = w ? strtoull(w, nullptr, 10) : kWaitTicks;
+    return L.parts.get();
 }
 
 } // namespace svfsi

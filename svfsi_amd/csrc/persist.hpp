@@ -48,7 +48,8 @@ struct PartsDev {
     const int* hOff;            // G+1 offsets into hPos
     const int* hPos;            // halo: positions in the exchange buffer
     const unsigned short* lcol; // per block: local index of its column, own rows first, then the halo
-    unsigned long long* xb;     // 2 x nNo x 4 tagged words
+    unsigned long long* xb;     // 16 tagged words per node
+    unsigned long long* red;    // partials of two sums over all parts, 2 G words each
     unsigned long long wait;    // ticks before a waiting lane gives up
     int G;
 };
@@ -106,22 +107,29 @@ __device__ __forceinline__ bool get_words(const unsigned long long* const (&p)[N
 struct Parts {
     int G = 0, U = 0, maxOwn = 0, maxHalo = 0, maxLanes = 0;
     unsigned epoch = 0; // the last tag used; xb starts out with tag 0
-    bool tried = false, off = false;
+    bool off = false;
     unsigned long long wait = kWaitTicks;
-    DBuf rowOff, rowId, laneOff, lane, hOff, hPos, lcol, xb;
+    size_t ldsMax = 0;
+    DBuf tab, xb;
+    size_t at[7] = {}; // of rowOff, rowId, laneOff, lane, hOff, hPos, lcol in tab
+    size_t red = 0;    // of the sums' words in xb, 2 G per sum
     PartsDev dev() const
     {
-        return {rowOff.as<int>(), rowId.as<int>(), laneOff.as<int>(), lane.as<int>(), hOff.as<int>(), hPos.as<int>(),
-                lcol.as<unsigned short>(), xb.as<unsigned long long>(), wait, G};
+        const int* t = tab.as<int>();
+        unsigned long long* x = xb.as<unsigned long long>();
+        return {t + at[0], t + at[1], t + at[2], t + at[3], t + at[4], t + at[5],
+                reinterpret_cast<const unsigned short*>(t + at[6]), x, x + red, wait, G};
     }
 };
 
-// The partition of L, built on the first call and kept with L; nullptr when
-// the pattern does not fit the chip or the path is off.
+// Partitions L if its pattern fits the chip (at the end of FSILS_LHS_CREATE).
+void persist_build(Lhs& L);
+// The partition of L; nullptr when there is none or the path is off.
 Parts* persist_parts(Lhs& L);
 
-// One matrix-resident solve at a time per device and process: they would
-// wait for each other's CUs.
+// One matrix-resident solve at a time per device and process, the others wait
+// on the host: their kernels would wait for each other's CUs, and a solve that
+// took the other path instead would differ in its last bits.
 struct PersistLock {
     int dev = -1;
     PersistLock() = default;
@@ -139,5 +147,20 @@ int ppoly_launch(Lhs& L, Parts& P, int dof, const float* B, const float* dinv, c
                  const double* coef, const int* ops, int nOps, int lastLin, int* stop, int* abortFlag,
                  hipStream_t s);
 size_t ppoly_lds(const Parts& P); // its dynamic LDS
+
+// `its` iterations of CGRADV (dof 3) and of CGRAD_SCHUR in one launch
+// (pcg.hip), from X, R, Pv and *st on to them; Parts with U = 3.
+struct CgState;
+int pcg3_launch(Lhs& L, Parts& P, const double* K, double* X, double* R, double* Pv, CgState* st, int its,
+                hipStream_t s);
+int pcgs_launch(Lhs& L, Parts& P, const double* Lm, const double* G, const double* Gt, double* X, double* R,
+                double* Pv, CgState* st, int its, hipStream_t s);
+size_t pcg_lds(const Parts& P); // their dynamic LDS
+inline bool pcg_fits(const Parts& P) // 16 groups of 16 parts share the sums
+{
+    return P.U == 3 && P.G <= 256 && pcg_lds(P) + 512 <= P.ldsMax;
+}
+// iterations per launch: about 2 ms, with the matrix read once
+constexpr int kPcgChunk = 256;
 
 } // namespace svfsi

@@ -8,8 +8,8 @@ import threading
 import numpy as np
 import pytest
 
+from svfsi_amd import fsils, problems
 from svfsi_amd import mesh as meshmod
-from svfsi_amd import problems
 
 
 def hub(points):
@@ -44,7 +44,7 @@ CASES = {
 }
 
 
-def solve(prob, monkeypatch, persist, wait=None):
+def solve(prob, monkeypatch, persist, wait=None, mixed=True):
     import torch
 
     from svfsi_amd.step import NewtonStep
@@ -57,7 +57,7 @@ def solve(prob, monkeypatch, persist, wait=None):
     st = NewtonStep(prob)
     out = []
     for _ in range(2):  # the second solve reuses the partition and its exchange buffer
-        ls = st.step(mixed=True)
+        ls = st.step(mixed=mixed)
         torch.cuda.synchronize()
         out.append((st.R.cpu().numpy().copy(), ls.RI.itr, ls.RI.suc))
     assert np.array_equal(out[0][0], out[1][0])
@@ -116,3 +116,52 @@ def test_two_threads(gpu, monkeypatch):
     for (x, itr, suc), (y, itr0, _) in zip(got, want):
         assert suc == 1 and abs(itr - itr0) <= 1
         assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+
+
+def with_ls(prob, **ls):
+    prob.ls = dict(prob.ls, **ls)
+    return prob
+
+
+FP64 = {
+    **{k: lambda k=k: with_ls(CASES[k](), LS_type=fsils.LS_TYPE_CG, relTol=1e-8, mItr=2000)
+       for k in ("lelas_1part", "lelas_parts", "lelas_all_cus", "hub_16_lanes", "hub_64_lanes", "hub_no_fit", "tet10")},
+    # the Schur complement is iterated to the NS solver's inner tolerances
+    **{f"ns_{k}": lambda k=k: with_ls(CASES[k](), LS_type=fsils.LS_TYPE_NS, relTol=1e-5, absTol=1e-30, mItr=20)
+       for k in ("fluid_few", "fluid_mid")},
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(FP64))
+def test_fp64_matches_one_launch_per_step(gpu, monkeypatch, name):
+    """CG and the Schur complement's CG: sums over the parts in another order,
+    so the same solution to the solver's tolerance."""
+    prob = FP64[name]()
+    x, itr, suc = solve(prob, monkeypatch, "1", mixed=False)
+    y, itr0, suc0 = solve(prob, monkeypatch, "0", mixed=False)
+    assert suc == suc0 == 1 and abs(itr - itr0) <= 2
+    tol = 1e-4 if name.startswith("ns_") else 1e-6  # relTol 1e-5 and 1e-8, times the conditioning
+    assert np.linalg.norm(x - y) <= tol * np.linalg.norm(y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mItr", [0, 1, 7, 256, 257, 600])
+def test_cg_iteration_limit(gpu, monkeypatch, mItr):
+    """The limit inside a launch, at its end, and beyond; X after mItr steps
+    agrees while the iteration has not lost its digits."""
+    prob = with_ls(CASES["lelas_parts"](), LS_type=fsils.LS_TYPE_CG, relTol=1e-300, absTol=1e-300, mItr=mItr)
+    x, itr, suc = solve(prob, monkeypatch, "1", mixed=False)
+    y, itr0, suc0 = solve(prob, monkeypatch, "0", mixed=False)
+    assert (itr, suc) == (itr0, suc0) == (mItr, 0)
+    assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["lelas_parts", "ns_fluid_mid"])
+def test_fp64_gives_up_and_falls_back(gpu, monkeypatch, name):
+    prob = FP64[name]()
+    x, itr, suc = solve(prob, monkeypatch, "1", wait="0", mixed=False)
+    y, itr0, suc0 = solve(prob, monkeypatch, "0", mixed=False)
+    assert (itr, suc) == (itr0, suc0)
+    assert np.array_equal(x, y)
