@@ -1879,25 +1879,34 @@ __global__ __launch_bounds__(256) void k_asm_struct_mfma(int begin, int count, c
 // elements of the 24^3 cube at the 4-point rule, less than staging the
 // operands for the matrix cores.
 //
-// k_struct_elem: a lane per (element, point) writes the point's node vectors
-// to LDS, then 50 lanes per element each sum two neighbouring blocks of a row
-// over the points and store them, element blocks contiguous (7.2 KB).
+// points: a lane per (element, point) writes the point's record, with the
+// Jacobian's inverse B (Nx_a = B^T xi_a, xi_a the reference gradients): F^-T
+// B^T, F B^T, B B^T and scalars, 30 doubles.
+// k_struct_elem: a lane per point and node writes C xi_a, n_a and m_a to LDS,
+// then 50 lanes per element each sum two neighbouring blocks of a row over
+// the points and store them, element blocks contiguous (7.2 KB).
 // k_struct_rows: a wavefront per node adds the 720-byte strips of its
-// elements into the node's row of Val, in LDS, in element-id order.  The
-// scatter of the coloured kernels (30 launches, each a read-modify-write of
-// scattered 72-byte blocks) took 1.22 ms of the 1.41 ms there; these two
-// launches 837 us (4,374 elements, 15-point rule: 559 -> 67 us).
+// elements into the node's row of Val, in LDS, in element-id order.
+//
+// What bounds it: the element blocks, 600 MB written and read on the 24^3
+// cube (82,944 elements), and the latency of the records' node gathers.  There
+// 661 us, against 1412 with B^T Dm B on the matrix cores and a coloured
+// scatter (30 launches, each a read-modify-write of scattered 72-byte blocks,
+// 1.22 ms); 4,374 elements with 15 points: 559 -> 78 us.  Strips formed in the
+// row kernel from the records, without the blocks' trip through memory, took
+// 660 and 130 us (two or three wavefronts per SIMD, a serial chain each).
 // ---------------------------------------------------------------------------
-constexpr int SN_SZ = 10;                   // per node: Nx, n, m (scaled), pad
-constexpr int SQ_C = 10 * SN_SZ;            // then w s, w (pl J + 2 r1/3), w (r1 - p J), w
-constexpr int SQ_UD = SQ_C + 4, SQ_SZ = SQ_UD + 4;
+constexpr int SP_N = 0, SP_M = 9, SP_C = 18, SP_K = 24, SP_UD = 27, SP_SZ = 30; // point record
+constexpr int SN_SZ = 10;        // per node: C xi, n, m (scaled), pad
+constexpr int SQ_C = 10 * SN_SZ; // then kap, gam, w, w times the inertia
+constexpr int SQ_SZ = SQ_C + 6;
 
-// One material point to LDS: node vectors Nx_a, n_a and w (-2/3 s) m_a, and
-// the scalars above (all without the factor af beta dt^2).
-__device__ __forceinline__ void struct_point_vec(int e, const int* __restrict__ ien, const double* __restrict__ x,
+// Record of point g of element e: F^-T B^T, w (-2/3 s) F B^T, w s B B^T (00, 11,
+// 22, 01, 02, 12), w (pl J + 2 r1/3), w (r1 - p J), w and w times the inertia.
+__device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ ien, const double* __restrict__ x,
                                                  int tDof, const double* __restrict__ Ag,
                                                  const double* __restrict__ Dg, const AsmParams& P,
-                                                 const double* __restrict__ rg, double* rc)
+                                                 const double* __restrict__ rg, double* out)
 {
     double A[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll 5
@@ -1932,7 +1941,6 @@ __device__ __forceinline__ void struct_point_vec(int e, const int* __restrict__ 
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             Nxa[j] = rg[11 + a * 3] * B[0][j] + rg[11 + a * 3 + 1] * B[1][j] + rg[11 + a * 3 + 2] * B[2][j];
-            rc[a * SN_SZ + j] = Nxa[j];
         }
         const double Na = rg[1 + a];
 #pragma unroll
@@ -1969,40 +1977,97 @@ __device__ __forceinline__ void struct_point_vec(int e, const int* __restrict__ 
     const double s = pow(Jf, -2.0 / 3.0) * (2.0 * P.C10);
     const double r1 = s * trC / 3.0;
     const double ws = w * s, cm = -2.0 / 3.0 * ws;
-    rc[SQ_C] = ws;
-    rc[SQ_C + 1] = w * (pl * Jf + 2.0 * r1 / 3.0);
-    rc[SQ_C + 2] = w * (r1 - p * Jf);
-    rc[SQ_C + 3] = w;
+    double o[SP_SZ];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) rc[SQ_UD + i] = ud[i];
-#pragma unroll 5
-    for (int a = 0; a < 10; ++a) {
-        double* na = rc + a * SN_SZ;
-        const double n0 = na[0], n1 = na[1], n2 = na[2];
+    for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            na[3 + i] = Fi[i][0] * n0 + Fi[i][1] * n1 + Fi[i][2] * n2;
-            na[6 + i] = cm * (F[i][0] * n0 + F[i][1] * n1 + F[i][2] * n2);
+        for (int k = 0; k < 3; ++k) {
+            o[SP_N + 3 * i + k] = Fi[i][0] * B[k][0] + Fi[i][1] * B[k][1] + Fi[i][2] * B[k][2];
+            o[SP_M + 3 * i + k] = cm * (F[i][0] * B[k][0] + F[i][1] * B[k][1] + F[i][2] * B[k][2]);
         }
-    }
+    auto bb = [&](int k, int m) { return ws * (B[k][0] * B[m][0] + B[k][1] * B[m][1] + B[k][2] * B[m][2]); };
+    o[SP_C] = bb(0, 0);
+    o[SP_C + 1] = bb(1, 1);
+    o[SP_C + 2] = bb(2, 2);
+    o[SP_C + 3] = bb(0, 1);
+    o[SP_C + 4] = bb(0, 2);
+    o[SP_C + 5] = bb(1, 2);
+    o[SP_K] = w * (pl * Jf + 2.0 * r1 / 3.0);
+    o[SP_K + 1] = w * (r1 - p * Jf);
+    o[SP_K + 2] = w;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) o[SP_UD + i] = w * ud[i];
+    // 240 bytes: 16-byte aligned
+#pragma unroll
+    for (int q = 0; q < SP_SZ / 2; ++q) *reinterpret_cast<d2_t*>(out + 2 * q) = d2_t{o[2 * q], o[2 * q + 1]};
 }
 
-template <int NG, int EPW, int NT>
+__global__ __launch_bounds__(256) void k_struct_rec(int nEl, int nG, const int* __restrict__ ien,
+                                                    const double* __restrict__ x, int tDof,
+                                                    const double* __restrict__ Ag, const double* __restrict__ Dg,
+                                                    AsmParams P, const double* __restrict__ rule,
+                                                    double* __restrict__ rec)
+{
+    const int id = blockIdx.x * 256 + threadIdx.x, e = id / nG;
+    if (e < nEl)
+        struct_point_rec(e, ien, x, tDof, Ag, Dg, P, rule + (id - e * nG) * kTet10Rec, rec + (size_t)id * SP_SZ);
+}
+
+// Element blocks from the point records.  With 15 points the workgroup forms
+// its records itself (a quarter of its lanes busy; a launch of its own takes
+// 18 us at 4,374 elements); with 4, where a tenth would be
+// busy, they come from k_struct_rec (REC; 82,944 elements: 62 + 281 us
+// against 430).
+template <int NG, int EPW, int NT, bool REC>
 __global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restrict__ ien,
                                                     const double* __restrict__ x, int tDof,
                                                     const double* __restrict__ Ag, const double* __restrict__ Dg,
                                                     AsmParams P, const double* __restrict__ rule,
-                                                    double* __restrict__ ke, double* __restrict__ re)
+                                                    const double* __restrict__ recs, double* __restrict__ ke,
+                                                    double* __restrict__ re)
 {
-    static_assert(EPW * NG <= NT && EPW * 50 <= NT, "one pass of lanes per phase");
-    __shared__ __align__(16) double rec[EPW * NG][SQ_SZ];
-    __shared__ double sN[NG][10];
+#pragma clang fp contract(fast) // the Jacobians are behind: see the top of the file
+    static_assert(EPW * 50 <= NT, "one pass of lanes in the second phase");
+    __shared__ __align__(16) double pt[EPW * NG][SQ_SZ];
+    __shared__ __align__(16) double sX[NG * 10][4]; // reference gradient and N
     const int tid = threadIdx.x;
     const int e0 = blockIdx.x * EPW;
-    for (int i = tid; i < NG * 10; i += NT) sN[i / 10][i % 10] = rule[(i / 10) * kTet10Rec + 1 + i % 10];
-    if (tid < EPW * NG) {
-        const int k = tid / NG, g = tid - k * NG;
-        if (e0 + k < nEl) struct_point_vec(e0 + k, ien, x, tDof, Ag, Dg, P, rule + g * kTet10Rec, rec[tid]);
+    for (int q = tid; q < NG * 40; q += NT) {
+        const int g = q / 40, a = (q - 40 * g) / 4, c = q & 3;
+        sX[g * 10 + a][c] = rule[g * kTet10Rec + (c < 3 ? 11 + 3 * a + c : 1 + a)];
+    }
+    const int nPt = min(EPW, nEl - e0) * NG;
+    const double* rec = recs + (size_t)e0 * NG * SP_SZ;
+    if constexpr (!REC) {
+        __shared__ __align__(16) double own[EPW * NG][SP_SZ];
+        for (int p = tid; p < nPt; p += NT)
+            struct_point_rec(e0 + p / NG, ien, x, tDof, Ag, Dg, P, rule + p % NG * kTet10Rec, own[p]);
+        __syncthreads();
+        rec = own[0];
+    }
+    for (int q = tid; q < nPt * 10; q += NT) {
+        const int p = q / 10, a = q - 10 * p, g = p % NG;
+        const d2_t* rc = reinterpret_cast<const d2_t*>(rec + (size_t)p * SP_SZ);
+        double o[SP_SZ];
+#pragma unroll
+        for (int u = 0; u < SP_SZ / 2; ++u) {
+            const d2_t v = rc[u];
+            o[2 * u] = v.x;
+            o[2 * u + 1] = v.y;
+        }
+        const double* xi = rule + g * kTet10Rec + 11 + 3 * a;
+        const double x0 = xi[0], x1 = xi[1], x2 = xi[2];
+        double* n = pt[p] + a * SN_SZ;
+        n[0] = o[SP_C] * x0 + o[SP_C + 3] * x1 + o[SP_C + 4] * x2;
+        n[1] = o[SP_C + 3] * x0 + o[SP_C + 1] * x1 + o[SP_C + 5] * x2;
+        n[2] = o[SP_C + 4] * x0 + o[SP_C + 5] * x1 + o[SP_C + 2] * x2;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            n[3 + c] = o[SP_N + 3 * c] * x0 + o[SP_N + 3 * c + 1] * x1 + o[SP_N + 3 * c + 2] * x2;
+            n[6 + c] = o[SP_M + 3 * c] * x0 + o[SP_M + 3 * c + 1] * x1 + o[SP_M + 3 * c + 2] * x2;
+        }
+        if (a < 6) pt[p][SQ_C + a] = a == 0 ? o[SP_K] : a == 1 ? o[SP_K + 1] : a == 2 ? o[SP_K + 2]
+                                     : a == 3 ? o[SP_UD] : a == 4 ? o[SP_UD + 1] : o[SP_UD + 2];
     }
     __syncthreads();
     const int k = tid / 50, r = tid - k * 50, e = e0 + k;
@@ -2017,7 +2082,7 @@ __global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restri
             for (int q = 0; q < 9; ++q) K[h][q] = 0.0;
 #pragma unroll 1
         for (int g = 0; g < NG; ++g) {
-            const double* rc = rec[k * NG + g];
+            const double* rc = pt[k * NG + g];
             double na[SN_SZ];
 #pragma unroll
             for (int q = 0; q < SN_SZ / 2; ++q) {
@@ -2025,19 +2090,20 @@ __global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restri
                 na[2 * q] = v.x;
                 na[2 * q + 1] = v.y;
             }
-            const double ws = rc[SQ_C], kap = rc[SQ_C + 1], gam = rc[SQ_C + 2], w = rc[SQ_C + 3];
-            const double Na = sN[g][a];
+            const double kap = rc[SQ_C], gam = rc[SQ_C + 1], w = rc[SQ_C + 2];
+            const double Na = sX[g * 10 + a][3];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 double nb[SN_SZ];
 #pragma unroll
-                for (int q = 0; q < SN_SZ / 2; ++q) {
+                for (int q = 1; q < SN_SZ / 2; ++q) {
                     const d2_t v = *reinterpret_cast<const d2_t*>(rc + (b0 + h) * SN_SZ + 2 * q);
                     nb[2 * q] = v.x;
                     nb[2 * q + 1] = v.y;
                 }
-                T[h] += ws * (na[0] * nb[0] + na[1] * nb[1] + na[2] * nb[2]);
-                M[h] += w * (Na * sN[g][b0 + h]);
+                const double* xb = sX[g * 10 + b0 + h];
+                T[h] += na[0] * xb[0] + na[1] * xb[1] + na[2] * xb[2];
+                M[h] += w * (Na * xb[3]);
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
                     const double eb = kap * nb[3 + j] + nb[6 + j]; // n_a's partner
@@ -2049,7 +2115,7 @@ __global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restri
             }
             if (b0 == 0) {
 #pragma unroll
-                for (int i = 0; i < 3; ++i) R[i] += w * (Na * rc[SQ_UD + i]) - 1.5 * na[6 + i] - gam * na[3 + i];
+                for (int i = 0; i < 3; ++i) R[i] += Na * rc[SQ_C + 3 + i] - 1.5 * na[6 + i] - gam * na[3 + i];
             }
         }
         const double afu = P.af * P.beta * P.dt * P.dt, amd = P.am * P.rho;
@@ -2314,13 +2380,21 @@ int launch_asm_struct(Mesh& M, const AsmParams& P, int nG, const double* rule, i
             SV_TRY(M.re.ensure((size_t)M.nEl * 10 * 3 * sizeof(double)));
             double* ke = M.ke.as<double>();
             double* re = M.re.as<double>();
-            constexpr int E4 = 10, E15 = 5;
-            if (nG == 4)
-                hipLaunchKernelGGL((k_struct_elem<4, E4, 512>), dim3((unsigned)((M.nEl + E4 - 1) / E4)), dim3(512), 0,
-                                   s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule, ke, re);
-            else
-                hipLaunchKernelGGL((k_struct_elem<15, E15, 256>), dim3((unsigned)((M.nEl + E15 - 1) / E15)), dim3(256),
-                                   0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule, ke, re);
+            constexpr int E4 = 5, E15 = 2;
+            if (nG == 4) {
+                const size_t nPts = (size_t)M.nEl * nG;
+                SV_TRY(M.srec.ensure(nPts * SP_SZ * sizeof(double)));
+                double* rec = M.srec.as<double>();
+                hipLaunchKernelGGL(k_struct_rec, dim3((unsigned)((nPts + 255) / 256)), dim3(256), 0, s, M.nEl, nG,
+                                   M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule, rec);
+                hipLaunchKernelGGL((k_struct_elem<4, E4, 256, true>), dim3((unsigned)((M.nEl + E4 - 1) / E4)),
+                                   dim3(256), 0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule,
+                                   (const double*)rec, ke, re);
+            } else {
+                hipLaunchKernelGGL((k_struct_elem<15, E15, 128, false>), dim3((unsigned)((M.nEl + E15 - 1) / E15)),
+                                   dim3(128), 0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule,
+                                   (const double*)nullptr, ke, re);
+            }
             hipLaunchKernelGGL(k_struct_rows, dim3((unsigned)((M.nNo + 3) / 4)), dim3(256), lds, s, M.nNo, M.maxRow,
                                M.lhs->rowPtr.as<int>(), M.rPtr.as<int>(), M.rSrc.as<int>(), M.emap.as<int>(),
                                (const double*)ke, (const double*)re, val, R);
