@@ -1277,6 +1277,13 @@ __global__ __launch_bounds__(256) void k_gm_fold(int nb, double* __restrict__ pa
 // (SVFSI_FOLD_CHUNKS overrides, read at each solve).
 constexpr int kFoldChunks = 1024;
 
+// Row chunks (512 unknowns each) up to which GMRESV ends a step with
+// k_gm_rotupdate: ms per solve with it / with k_gm_givens and k_gm_update at
+// 21 chunks 22.7 / 25.6 (1230 steps), at 39 74.6 / 84.5, at 70 123.9 / 137.0,
+// at 130 232.6 / 249.6; the partials that every block reads grow with the
+// chunks, and beyond this the gain is within the spread of the step count.
+constexpr size_t kOneEnd = 160;
+
 // The serial part of an Arnoldi step (one thread): h(i+1,i) (Pythagorean
 // for passes 0-2, hsh[i] = |w|^2 for pass 3), the previous rotations, the
 // new Givens rotation, the Hessenberg column, the residual estimate and the
@@ -1505,7 +1512,10 @@ __global__ __launch_bounds__(256) void k_gm_scale(size_t n, int i, int sD, BT* _
 // block that starts later skips its rows: u_{i+1} is not used after a stop.
 // PRE: the coefficients were already summed into A.hraw by k_gm_hsum (the
 // fused SpMV + dot path); otherwise every block sums the multi-dot partials.
-template <typename BT, bool PRE = false>
+// SERIAL: that rule's sum by one thread in the order of givens_tail, so that the
+// step has the bits of k_gm_givens and k_gm_update (GMRESV: on stiff systems
+// the count of steps follows them).
+template <typename BT, bool PRE = false, bool SERIAL = false>
 __global__ __launch_bounds__(256) void k_gm_rotupdate(size_t n, int i, int sD, int nb,
                                                       const double* __restrict__ partial, BT* __restrict__ basis,
                                                       GmState* __restrict__ st, GmArrays A)
@@ -1558,7 +1568,7 @@ __global__ __launch_bounds__(256) void k_gm_rotupdate(size_t n, int i, int sD, i
             cs_s[0][jj] = A.c[jj];
             cs_s[1][jj] = A.sn[jj];
         }
-    if (threadIdx.x < kWave) {
+    if (!SERIAL && threadIdx.x < kWave) {
         double q = 0.0;
         for (int jj = threadIdx.x; jj < i; jj += kWave) q += hsh[jj] * hsh[jj];
         for (int o = kWave >> 1; o > 0; o >>= 1) q += __shfl_xor(q, o, kWave);
@@ -1566,7 +1576,12 @@ __global__ __launch_bounds__(256) void k_gm_rotupdate(size_t n, int i, int sD, i
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        const double hii = sqrt(fabs(hsh[i] - inv_s));
+        double hii = hsh[i];
+        if constexpr (SERIAL)
+            for (int jj = 0; jj < i; ++jj) hii = hii - hsh[jj] * hsh[jj];
+        else
+            hii = hii - inv_s;
+        hii = sqrt(fabs(hii));
         hsh[i] = hii;
         inv_s = 1.0 / hii;
     }
@@ -1885,12 +1900,16 @@ static int gmres_core(Lhs& L, const GmOp<BT>& op, int dof, BT* R, DBuf& basisBuf
     SV_TRY(poll.ensure(256));
     GmState hs{};
     const int chunk = 8;
+    // up to kOneEnd row chunks the step ends in one launch (k_gm_rotupdate:
+    // every block sums the partials itself) instead of two
+    const bool oneEnd = nbr <= kOneEnd;
     const bool useGraphs = graphs_enabled();
     if (useGraphs) {
         std::vector<uintptr_t> sig = {
             (uintptr_t)n, (uintptr_t)dof, (uintptr_t)sD, (uintptr_t)op.K, (uintptr_t)sizeof(BT),
             (uintptr_t)op_transposed(op), (uintptr_t)basis, (uintptr_t)part, (uintptr_t)st, (uintptr_t)w.hess.p,
-            (uintptr_t)L.rowPtr.p, (uintptr_t)L.colPtr.p, (uintptr_t)L.trans.p, (uintptr_t)op_cpl(op), (uintptr_t)((long long)nbr > foldAt)};
+            (uintptr_t)L.rowPtr.p, (uintptr_t)L.colPtr.p, (uintptr_t)L.trans.p, (uintptr_t)op_cpl(op), (uintptr_t)((long long)nbr > foldAt),
+            (uintptr_t)oneEnd};
         if (op_cpl(op)) cpl_sig(L, sig);
         if (sig != w.gmGraphs.sig) {
             w.gmGraphs.clear();
@@ -1916,6 +1935,11 @@ static int gmres_core(Lhs& L, const GmOp<BT>& op, int dof, BT* R, DBuf& basisBuf
                     SV_TRY(op.apply(basis + (size_t)(i - 1) * n, basis + (size_t)i * n, cs, stopFlag));
                     hipLaunchKernelGGL(k_gm_mdot<BT>, dim3((unsigned)nbr, (unsigned)((i + 8) / 8)), dim3(256), 0, cs,
                                        n, i, (const BT*)basis, part, (const GmState*)st);
+                    if (oneEnd) {
+                        hipLaunchKernelGGL((k_gm_rotupdate<BT, false, true>), dim3((unsigned)((n + 255) / 256)),
+                                           dim3(256), 0, cs, n, i, sD, (int)nbr, (const double*)part, basis, st, A);
+                        continue;
+                    }
                     if ((long long)nbr > foldAt) {
                         hipLaunchKernelGGL(k_gm_fold, dim3((unsigned)(i + 1)), dim3(256), 0, cs, (int)nbr, part,
                                            (const GmState*)st);
