@@ -1902,7 +1902,7 @@ static int gmres_core(Lhs& L, const GmOp<BT>& op, int dof, BT* R, DBuf& basisBuf
     const int chunk = 8;
     // up to kOneEnd row chunks the step ends in one launch (k_gm_rotupdate:
     // every block sums the partials itself) instead of two
-    const bool oneEnd = nbr <= kOneEnd;
+    const bool oneEnd = nbr <= kOneEnd && (long long)nbr <= foldAt;
     const bool useGraphs = graphs_enabled();
     if (useGraphs) {
         std::vector<uintptr_t> sig = {
