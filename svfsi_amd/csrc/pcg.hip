@@ -205,12 +205,12 @@ __global__ __launch_bounds__(1024) void k_pcg3(PartsDev P, int tabN, int maxHalo
                                                double* __restrict__ R, double* __restrict__ Pv, CgState* st,
                                                int its, unsigned base)
 {
-    if (st->done) return; // set by an earlier launch only
+    __shared__ ReduceLds L;
+    if (leave_at_start(&st->done, &L.bad)) return;
     extern __shared__ double ldsd[];
     double* tp = ldsd;                // P: own rows, then the halo, 4 per node
     double* tr = tp + 4 * tabN;       // R of the halo, 3 per node
     int* sH = reinterpret_cast<int*>(tr + 3 * maxHalo);
-    __shared__ ReduceLds L;
     const int tid = threadIdx.x, NT = blockDim.x, b = blockIdx.x;
     const int w1 = NT > 64 * sum_waves(P) ? 64 * sum_waves(P) : 0; // the others fetch the halo
     const Lane t = lane_of(P, b);
@@ -240,7 +240,6 @@ __global__ __launch_bounds__(1024) void k_pcg3(PartsDev P, int tabN, int maxHalo
         tp[4 * t.lr + t.l] = p;
     }
     for (int i = tid; i < nh; i += NT) sH[i] = P.hPos[P.hOff[b] + i];
-    if (tid == 0) L.bad = 0;
     __syncthreads();
     for (int q = tid; q < 3 * nh; q += NT) {
         const int h = q / 3, c = q - 3 * h;
@@ -295,7 +294,7 @@ __global__ __launch_bounds__(1024) void k_pcg3(PartsDev P, int tabN, int maxHalo
         __syncthreads();
     }
     if (L.bad) { // some part gave up: the caller starts over
-        if (tid == 0) st->done = 1;
+        if (tid == 0) st_agent(&st->done, 1);
         return;
     }
     if (own) {
@@ -323,13 +322,13 @@ __global__ __launch_bounds__(1024) void k_pcgs(PartsDev P, int tabN, int maxHalo
                                                double* __restrict__ R, double* __restrict__ Pv, CgState* st,
                                                int its, unsigned base)
 {
-    if (st->done) return;
+    __shared__ ReduceLds L;
+    if (leave_at_start(&st->done, &L.bad)) return;
     extern __shared__ double ldsd[];
     double* tg = ldsd;                // G P: own rows, then the halo, 4 per node
     double* tp = tg + 4 * tabN;       // P: own rows, then the halo
     double* tr = tp + tabN;           // R of the halo
     int* sH = reinterpret_cast<int*>(tr + maxHalo);
-    __shared__ ReduceLds L;
     const int tid = threadIdx.x, NT = blockDim.x, b = blockIdx.x;
     const int w1 = NT > 64 * sum_waves(P) ? 64 * sum_waves(P) : 0; // the others fetch the halo
     const Lane t = lane_of(P, b);
@@ -360,7 +359,6 @@ __global__ __launch_bounds__(1024) void k_pcgs(PartsDev P, int tabN, int maxHalo
         tp[t.lr] = p;
     }
     for (int i = tid; i < nh; i += NT) sH[i] = P.hPos[P.hOff[b] + i];
-    if (tid == 0) L.bad = 0;
     __syncthreads();
     for (int h = tid; h < nh; h += NT) tp[nr + h] = Pv[P.rowId[sH[h]]];
     double err = st->err, errO = st->errO, alpha = st->alpha;
@@ -427,7 +425,7 @@ __global__ __launch_bounds__(1024) void k_pcgs(PartsDev P, int tabN, int maxHalo
         __syncthreads();
     }
     if (L.bad) {
-        if (tid == 0) st->done = 1;
+        if (tid == 0) st_agent(&st->done, 1);
         return;
     }
     if (own) {

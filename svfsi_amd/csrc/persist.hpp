@@ -27,7 +27,11 @@
 //
 // Every wait is bounded: a lane that has polled for kWaitTicks raises the
 // abort flag, its workgroup ends, and all others end at their next wait; the
-// caller then takes the path of one launch per product.  That happens only
+// caller then takes the path of one launch per product.  A workgroup that
+// gives up also sets the solver's own flag (stop, done) for the launches
+// already queued, and leaving frees its CU for one that had to wait: a
+// workgroup may start while the flags change, so one lane reads them for all
+// (leave_at_start).  Giving up happens only
 // when the parts are not resident together (another kernel that itself waits
 // holds CUs); PersistLock keeps two such kernels of one process apart.
 #pragma once
@@ -65,6 +69,21 @@ template <typename T>
 __device__ __forceinline__ void st_agent(T* p, T v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// At a kernel's entry, by all lanes: whether the workgroup leaves, the flag set
+// by an earlier launch or, when parts give up, by this one.  The lanes must
+// agree, since those that stay index with LDS that all of them fill.  Clears
+// *bad, the workgroup's own give-up flag.
+__device__ __forceinline__ bool leave_at_start(const int* flag, int* bad)
+{
+    __shared__ int leave;
+    if (threadIdx.x == 0) {
+        leave = ld_agent(flag);
+        *bad = 0;
+    }
+    __syncthreads();
+    return leave != 0;
 }
 
 // 32 bits of payload under a tag

@@ -43,12 +43,13 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
                                                 const int* __restrict__ ops, int nOps, int lastLin, unsigned base,
                                                 int* stop, int* abortFlag)
 {
-    if (*stop) return; // set by an earlier kernel only: the same for the whole grid
+    __shared__ int bad[2]; // by step parity: a wave may give up at a step while another still reads the last one's
+    if (threadIdx.x == 0) bad[1] = 0;
+    if (leave_at_start(stop, &bad[0])) return;
     constexpr int DD = DOF * DOF;
     extern __shared__ float lds[];
     float* tab[2] = {lds, lds + 4 * tabN};   // the current vector, own rows then halo, by step parity
     int* sH = reinterpret_cast<int*>(lds + 8 * tabN);
-    __shared__ int bad;
     const int tid = threadIdx.x, NT = blockDim.x;
     const int b = blockIdx.x;
     const int o0 = P.rowOff[b], nr = P.rowOff[b + 1] - o0;
@@ -78,7 +79,6 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
         }
     }
     for (int i = tid; i < nh; i += NT) sH[i] = P.hPos[h0 + i];
-    if (tid == 0) bad = 0;
     // the row's entry c = l of the vectors: x the current one, y the result,
     // o the one before a quadratic factor's first half
     const bool own = has && l < DOF;
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
                 src[m] = t < nw ? xin + (size_t)sH[h] * 4 + (t - h * DOF) : nullptr;
             }
             if (!get_words<4>(src, base + s, v, P.wait, abortFlag)) {
-                bad = 1;
+                bad[s & 1] = 1;
                 break;
             }
 #pragma unroll
@@ -126,8 +126,8 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
             }
         }
         __syncthreads();
-        if (bad) {
-            if (tid == 0) *stop = 1;
+        if (bad[s & 1]) {
+            if (tid == 0) st_agent(stop, 1);
             return;
         }
         float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;

@@ -76,10 +76,12 @@ def test_matches_one_launch_per_factor(gpu, monkeypatch, name):
 
 
 @pytest.mark.gpu
-def test_gives_up_and_falls_back(gpu, monkeypatch):
-    """A wait of no ticks: the kernel ends at the first word not yet there and
-    the solve runs again with one launch per factor, to the same bits."""
-    prob = problems.lelas_cube(13)
+@pytest.mark.parametrize("name", ["lelas_parts", "lelas_all_cus", "fluid_mid", "tet10"])
+def test_gives_up_and_falls_back(gpu, monkeypatch, name):
+    """A wait of no ticks: the kernel ends at the first word not yet there,
+    some workgroups before others have started, and the solve runs again with
+    one launch per factor, to the same bits."""
+    prob = CASES[name]()
     x, itr, suc = solve(prob, monkeypatch, "1", wait="0")
     y, itr0, suc0 = solve(prob, monkeypatch, "0")
     assert suc == suc0 == 1 and itr == itr0
@@ -158,7 +160,7 @@ def test_cg_iteration_limit(gpu, monkeypatch, mItr):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["lelas_parts", "ns_fluid_mid"])
+@pytest.mark.parametrize("name", ["lelas_parts", "lelas_all_cus", "ns_fluid_few", "ns_fluid_mid"])
 def test_fp64_gives_up_and_falls_back(gpu, monkeypatch, name):
     prob = FP64[name]()
     x, itr, suc = solve(prob, monkeypatch, "1", wait="0", mixed=False)
