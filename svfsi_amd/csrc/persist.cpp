@@ -205,11 +205,15 @@ static int build(Lhs& L, Parts& P, int U, int gMin, int cus, size_t ldsMax)
     std::memcpy(all.data() + ints, lcol.data(), lcol.size() * sizeof(unsigned short));
     SV_TRY(P.tab.ensure(all.size() * sizeof(int)));
     SV_HIP(hipMemcpy(P.tab.p, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice));
-    // the exchange buffer and the partials of two sums over all parts, tag 0
+    // the exchange buffer and the partials of two sums over all parts, tag 0;
+    // cleared before this returns: the first solve may be on a stream that does
+    // not wait for the null stream, and what a freed pattern left in the memory
+    // may carry the tags that it starts with
     P.red = (size_t)n * 16;
     const size_t words = P.red + (size_t)G * 4;
     SV_TRY(P.xb.ensure(words * sizeof(unsigned long long)));
     SV_HIP(hipMemset(P.xb.p, 0, words * sizeof(unsigned long long)));
+    SV_HIP(hipStreamSynchronize(nullptr));
     P.ldsMax = ldsMax;
     P.U = U;
     P.G = (int)G;

@@ -89,6 +89,32 @@ def test_gives_up_and_falls_back(gpu, monkeypatch, name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mixed", [True, False])
+def test_first_solve_on_recycled_memory(gpu, monkeypatch, mixed):
+    """Patterns of one size made and freed in turn, each solved at once on a
+    stream that does not wait for the null stream: a buffer that still held
+    the freed pattern's words, with the tags the new one starts with, would
+    be read as its neighbours' values."""
+    import torch
+
+    from svfsi_amd.step import NewtonStep
+
+    monkeypatch.setenv("SVFSI_PERSIST", "1")
+    monkeypatch.delenv("SVFSI_PERSIST_WAIT", raising=False)
+    first = {}
+    with torch.cuda.stream(torch.cuda.Stream()):
+        for k in range(8):
+            prob = problems.lelas_cube(13)
+            prob.prop_el = 1e6 * (1.0 + 0.5 * (k % 2)) * np.ones(prob.mesh.nEl)
+            st = NewtonStep(prob)
+            st.step(mixed=mixed)
+            torch.cuda.current_stream().synchronize()
+            x = st.R.cpu().numpy()
+            assert np.array_equal(x, first.setdefault(k % 2, x))
+            st.lhs.free()
+
+
+@pytest.mark.gpu
 def test_two_threads(gpu, monkeypatch):
     """Two solves at once on streams of their own, one of which finds the
     matrix-resident path taken."""
