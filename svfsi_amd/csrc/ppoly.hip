@@ -14,9 +14,13 @@
 // here a step is one trip of the halo through memory and a few hundred ns of
 // LDS gathers, shuffles and FP64 updates, and the matrix is read once per
 // application: 97 us, the mixed step of that mesh 6.05 -> 4.06 ms (LELAS 20^3
-// 2.95 -> 2.21 ms, 4,918-node cylinder 2.50 -> 1.98 ms).  Tried before: parts
-// of consecutive rows (160 us: twice the halo), products through LDS with a
-// second barrier (3.2 us of the 6.5 us per step).
+// 2.95 -> 2.21 ms, 4,918-node cylinder 2.50 -> 1.98 ms).  The table is 16-byte
+// aligned and indexed from its own name, so that a gather is one ds_read_b128;
+// through a pointer array it was a flat load (mixed step 4.04 against 3.77 ms).
+// With dof 4 and five blocks a lane 4 of the 128 registers spill (20 bytes of
+// scratch a lane).  Tried before: parts of consecutive rows (160 us: twice the
+// halo), products through LDS with a second barrier (3.2 us of the 6.5 us per
+// step).
 #include "persist.hpp"
 #include "devutil.hpp"
 #include "stream.hpp"
@@ -47,8 +51,8 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
     if (threadIdx.x == 0) bad[1] = 0;
     if (leave_at_start(stop, &bad[0])) return;
     constexpr int DD = DOF * DOF;
-    extern __shared__ float lds[];
-    float* tab[2] = {lds, lds + 4 * tabN};   // the current vector, own rows then halo, by step parity
+    extern __shared__ __align__(16) float lds[]; // read as f4_t
+    auto tab = [&](int s) { return lds + (s & 1) * 4 * tabN; }; // the current vector, own rows then halo
     int* sH = reinterpret_cast<int*>(lds + 8 * tabN);
     const int tid = threadIdx.x, NT = blockDim.x;
     const int b = blockIdx.x;
@@ -94,7 +98,7 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
         } else {
             x = (float)qi[l];
         }
-        tab[0][4 * lr + l] = x;
+        tab(0)[4 * lr + l] = x;
         put_word(P.xb + (size_t)(o0 + lr) * 4 + l, __float_as_uint(x), base);
     }
     __syncthreads(); // sH
@@ -104,7 +108,7 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
     for (int s = 0; s < nOps; ++s) {
         const int mode = ops[2 * s], f = ops[2 * s + 1];
         const double c1 = coef[2 * f], c2 = coef[2 * f + 1];
-        float* xt = tab[s & 1];
+        float* xt = tab(s);
         // the halo of the current vector, up to four words a lane at a time
         const unsigned long long* xin = P.xb + (size_t)(s & 1) * xbN;
         for (int t0 = tid; t0 < nw; t0 += 4 * NT) {
@@ -185,7 +189,7 @@ __global__ __launch_bounds__(1024) void k_ppoly(PartsDev P, int nNo, int tabN, c
             if (s + 1 < nOps) {
                 put_word(P.xb + (size_t)((s + 1) & 1) * xbN + (size_t)(o0 + lr) * 4 + l, __float_as_uint(x),
                          base + s + 1);
-                tab[(s + 1) & 1][4 * lr + l] = x;
+                tab(s + 1)[4 * lr + l] = x;
             }
         }
     }
