@@ -2153,6 +2153,8 @@ __global__ __launch_bounds__(256) void k_struct_rows(int nNo, int maxRow, const 
     double* acc = accs + (size_t)wave * maxRow * 9;
     const int k0 = rowPtr[i], nv = (rowPtr[i + 1] - k0) * 9;
     for (int q = l; q < nv; q += 64) acc[q] = 0.0;
+    // the additions below are by other lanes than the zeroing
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const int b1 = l / 9, q1 = l - 9 * b1;               // value l of a strip
     const int b2 = (l + 64) / 9, q2 = l + 64 - 9 * b2;   // value l + 64, l < 26
     const int s1 = rPtr[i + 1];
