@@ -2364,6 +2364,26 @@ int launch_lelas_dkde(const Mesh& M, const AsmParams& P, const Tet4Rule& rule, c
     return SVFSI_OK;
 }
 
+// Scratch of the outer-product kernels: 7.44 KB per element, and 960 B of point
+// records with four points.  false: not to be had, or more than
+// SVFSI_ASM_SCRATCH_MB allows; what was taken is given back to the coloured
+// kernels that run instead, whose points take 3.1 KB per element with four
+// points (11.6 KB with 15).
+static bool struct_scratch(Mesh& M, int nG)
+{
+    const size_t ke = (size_t)M.nEl * 100 * 9 * sizeof(double), re = (size_t)M.nEl * 10 * 3 * sizeof(double);
+    const size_t rec = nG == 4 ? (size_t)M.nEl * nG * SP_SZ * sizeof(double) : 0;
+    const char* v = getenv("SVFSI_ASM_SCRATCH_MB");
+    if (v && ke + re + rec > (size_t)strtoull(v, nullptr, 10) << 20) return false;
+    if (M.ke.ensure(ke) == SVFSI_OK && M.re.ensure(re) == SVFSI_OK && (!rec || M.srec.ensure(rec) == SVFSI_OK))
+        return true;
+    (void)hipGetLastError();
+    M.ke.release();
+    M.re.release();
+    M.srec.release();
+    return false;
+}
+
 int launch_asm_struct(Mesh& M, const AsmParams& P, int nG, const double* rule, int tDof, const double* Ag,
                       const double* Dg, double* val, double* R, int kern, hipStream_t s)
 {
@@ -2373,19 +2393,16 @@ int launch_asm_struct(Mesh& M, const AsmParams& P, int nG, const double* rule, i
     }
     if (kern == SVFSI_STRUCT_AUTO) {
         // the outer-product kernels and their row gather, unless a row of Val
-        // is too long for four of them in LDS or the coloured scatter is asked
-        // for (SVFSI_ASM_GATHER=0)
+        // is too long for four of them in LDS, the coloured scatter is asked
+        // for (SVFSI_ASM_GATHER=0) or the scratch cannot be had
         const char* v = getenv("SVFSI_ASM_GATHER");
         const size_t lds = (size_t)M.maxRow * 9 * 4 * sizeof(double);
-        if (lds <= ((size_t)64 << 10) && !(v && v[0] == '0')) {
-            SV_TRY(M.ke.ensure((size_t)M.nEl * 100 * 9 * sizeof(double)));
-            SV_TRY(M.re.ensure((size_t)M.nEl * 10 * 3 * sizeof(double)));
+        if (lds <= ((size_t)64 << 10) && !(v && v[0] == '0') && struct_scratch(M, nG)) {
             double* ke = M.ke.as<double>();
             double* re = M.re.as<double>();
             constexpr int E4 = 5, E15 = 2;
             if (nG == 4) {
                 const size_t nPts = (size_t)M.nEl * nG;
-                SV_TRY(M.srec.ensure(nPts * SP_SZ * sizeof(double)));
                 double* rec = M.srec.as<double>();
                 hipLaunchKernelGGL(k_struct_rec, dim3((unsigned)((nPts + 255) / 256)), dim3(256), 0, s, M.nEl, nG,
                                    M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule, rec);

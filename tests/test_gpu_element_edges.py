@@ -191,3 +191,32 @@ def test_struct_assembly_sizes(gpu, orc, nEl, tDof, quad, vol):
     prob.eq = dict(prob.eq, fb=(0.3, -0.2, 0.1), **VOL[vol])
     for got, want in assembled(first_elements(prob, nEl), orc):
         assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quad", [0, 1])
+def test_struct_without_scratch(gpu, orc, monkeypatch, quad):
+    """162 elements of 7.4 or 8.4 KB do not fit 1 MB: the coloured kernels run,
+    to the bits of the call that asks for them."""
+    prob = first_elements(problems.struct_cube(n=3, quad=quad), 162)
+    rng = np.random.default_rng(11)
+    prob.Dg = rng.uniform(-0.004, 0.004, size=(prob.nNo, 3))
+
+    def run():  # on the same random Val and R each time
+        import torch
+
+        torch.manual_seed(11)
+        return assembled(prob, orc)
+
+    monkeypatch.setenv("SVFSI_ASM_SCRATCH_MB", "1")
+    capped = run()
+    monkeypatch.setenv("SVFSI_ASM_SCRATCH_MB", "2")
+    monkeypatch.setenv("SVFSI_ASM_GATHER", "0")
+    coloured = run()
+    monkeypatch.delenv("SVFSI_ASM_GATHER")
+    roomy = run()
+    for (got, want), (col, _), (out, _) in zip(capped, coloured, roomy):
+        assert np.abs(got - want.reshape(got.shape)).max() <= 1e-12 * np.abs(want).max()
+        assert np.array_equal(got, col)
+        assert np.abs(out - got).max() <= 1e-12 * np.abs(want).max()
+    assert not np.array_equal(capped[0][0], roomy[0][0])  # the two paths round differently
