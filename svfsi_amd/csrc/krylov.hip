@@ -503,17 +503,10 @@ int cg_core(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hi
     // dof 3: chunks of iterations as one matrix-resident launch each where the
     // matrix fits the chip (pcg.hip); KP, not used by them, keeps the
     // right-hand side for the case that such a launch gives up
-    PersistLock plock;
-    Parts* parts = nullptr;
-    if (dof == 3 && !h0.done && plock.acquire()) {
-        parts = persist_parts(L);
-        if (parts && !pcg_fits(*parts)) parts = nullptr;
-        if (parts) {
-            SV_HIP(hipMemcpyAsync(KP, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-        } else {
-            plock.release();
-        }
-    }
+    ResidentTurn turn;
+    Parts* parts = dof == 3 && !h0.done ? persist_parts(L, true) : nullptr;
+    if (parts && !turn.enter(s)) parts = nullptr;
+    if (parts) SV_HIP(hipMemcpyAsync(KP, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
     int posted = 0;
     CgState hs = h0;
     bool finished = h0.done != 0;
@@ -521,7 +514,7 @@ int cg_core(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hi
     while (!finished) {
         const int q = posted & 1;
         if (parts)
-            SV_TRY(pcg3_launch(L, *parts, K, X, R, P, st, kPcgChunk, s));
+            SV_TRY(turn.launch([&] { return pcg3_launch(L, *parts, K, X, R, P, st, kPcgChunk, s); }));
         else if (useGraphs)
             SV_TRY(graph_run(w.cgGraphs, 0, s, iters));
         else
@@ -545,7 +538,7 @@ int cg_core(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hi
             SV_HIP(hipStreamSynchronize(s));
             parts->off = true;
             parts = nullptr;
-            plock.release();
+            turn.leave();
             SV_HIP(hipMemcpyAsync(R, KP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
             SV_HIP(hipMemcpyAsync(P, KP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
             SV_HIP(hipMemcpyAsync(st, &h0, sizeof(CgState), hipMemcpyHostToDevice, s));
@@ -1015,17 +1008,10 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
         }
     }
     // matrix-resident chunks as in cg_core
-    PersistLock plock;
-    Parts* parts = nullptr;
-    if (!cpl && !h0.done && !prof().on && plock.acquire()) {
-        parts = persist_parts(L);
-        if (parts && !pcg_fits(*parts)) parts = nullptr;
-        if (parts) {
-            SV_HIP(hipMemcpyAsync(SP, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-        } else {
-            plock.release();
-        }
-    }
+    ResidentTurn turn;
+    Parts* parts = !cpl && !h0.done && !prof().on ? persist_parts(L, true) : nullptr;
+    if (parts && !turn.enter(s)) parts = nullptr;
+    if (parts) SV_HIP(hipMemcpyAsync(SP, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
     int posted = 0;
     CgState hs = h0;
     bool finished = h0.done != 0;
@@ -1034,7 +1020,7 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
         const int q = posted & 1;
         const bool firstChunk = launched == 0;
         if (parts)
-            SV_TRY(pcgs_launch(L, *parts, Lm, G, Gt, X, R, buf[1], st, kPcgChunk, s));
+            SV_TRY(turn.launch([&] { return pcgs_launch(L, *parts, Lm, G, Gt, X, R, buf[1], st, kPcgChunk, s); }));
         else if (useGraphs)
             SV_TRY(graph_run(w.csGraphs, firstChunk ? 0 : 1, s, [&](hipStream_t cs) { return iters(cs, firstChunk); }));
         else
@@ -1051,7 +1037,7 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
             SV_HIP(hipStreamSynchronize(s));
             parts->off = true;
             parts = nullptr;
-            plock.release();
+            turn.leave();
             SV_HIP(hipMemcpyAsync(R, SP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
             SV_HIP(hipMemcpyAsync(buf[1], SP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
             SV_HIP(hipMemcpyAsync(st, &h0, sizeof(CgState), hipMemcpyHostToDevice, s));
@@ -2402,7 +2388,7 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
     bool usePoly = polyWanted;
     // all factors in one matrix-resident launch where the matrix fits the
     // chip's registers (ppoly.hip); ops: its SpMV steps
-    PersistLock plock;
+    ResidentTurn turn;
     Parts* parts = nullptr;
     std::vector<int> ops;
     int lastLin = -1;
@@ -2454,12 +2440,11 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
                     if (!last) ops.insert(ops.end(), {2, f});
                 }
             }
-            if (std::is_same<IT, float>::value && retry && plock.acquire()) parts = persist_parts(L);
+            if (std::is_same<IT, float>::value && retry) parts = persist_parts(L, false);
+            if (parts && !turn.enter(s)) parts = nullptr;
             if (parts) {
                 SV_TRY(w.polyOps.ensure(ops.size() * sizeof(int)));
                 SV_HIP(hipMemcpyAsync(w.polyOps.p, ops.data(), ops.size() * sizeof(int), hipMemcpyHostToDevice, s));
-            } else {
-                plock.release();
             }
         } else {
             usePoly = false; // no usable roots: the inner GMRES cycle
@@ -2525,8 +2510,11 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
                     }
                 } else if (parts) {
                     if constexpr (std::is_same<IT, float>::value) {
-                        SV_TRY(ppoly_launch(L, *parts, dof, Kin, dinv, Q + (size_t)(i - 1) * n, zi, t64, coefD, w.polyOps.as<int>(), (int)ops.size() / 2,
-                                            lastLin, &st->stop, &st->abort, cs));
+                        SV_TRY(turn.launch([&] {
+                            return ppoly_launch(L, *parts, dof, Kin, dinv, Q + (size_t)(i - 1) * n, zi, t64, coefD,
+                                                w.polyOps.as<int>(), (int)ops.size() / 2, lastLin, &st->stop,
+                                                &st->abort, cs);
+                        }));
                         t64Done = true;
                     }
                 } else if (usePoly) {

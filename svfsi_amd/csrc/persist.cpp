@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <atomic>
 #include <climits>
+#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -11,21 +12,65 @@
 
 namespace svfsi {
 
-static std::mutex g_mu[64];
+namespace {
+struct Device {
+    std::mutex mu;
+    std::condition_variable cv;   // a solve has left
+    ResidentTurn* turns = nullptr; // the solves between enter and leave
+    hipEvent_t ev = nullptr;
+};
+constexpr int kDevices = 64;
+Device g_dev[kDevices];
+} // namespace
 
-bool PersistLock::acquire()
+std::mutex& ResidentTurn::mutex() const { return g_dev[dev].mu; }
+
+bool ResidentTurn::enter(hipStream_t stream)
 {
     int d = 0;
-    if (hipGetDevice(&d) != hipSuccess || d < 0 || d >= 64) return false;
-    g_mu[d].lock();
+    if (hipGetDevice(&d) != hipSuccess || d < 0 || d >= kDevices) return false;
+    Device& D = g_dev[d];
+    std::unique_lock<std::mutex> g(D.mu);
+    // nobody inside waits for anybody here, so this ends with their solves
+    D.cv.wait(g, [&] {
+        for (ResidentTurn* t = D.turns; t; t = t->next)
+            if (stream == hipStreamPerThread || t->s == hipStreamPerThread) return false;
+        return true;
+    });
     dev = d;
+    s = stream;
+    prev = nullptr;
+    next = D.turns;
+    if (next) next->prev = this;
+    D.turns = this;
     return true;
 }
 
-void PersistLock::release()
+void ResidentTurn::leave()
 {
-    if (dev >= 0) g_mu[dev].unlock();
+    if (dev < 0) return;
+    Device& D = g_dev[dev];
+    {
+        std::lock_guard<std::mutex> g(D.mu);
+        (prev ? prev->next : D.turns) = next;
+        if (next) next->prev = prev;
+    }
+    D.cv.notify_all();
     dev = -1;
+}
+
+// The streams of the others are alive: their solves are inside.  An event may be
+// recorded again once a stream was told to wait for it.
+int ResidentTurn::follow_others()
+{
+    Device& D = g_dev[dev];
+    for (ResidentTurn* t = D.turns; t; t = t->next) {
+        if (t == this || t->s == s) continue;
+        if (!D.ev) SV_HIP(hipEventCreateWithFlags(&D.ev, hipEventDisableTiming));
+        SV_HIP(hipEventRecord(D.ev, t->s));
+        SV_HIP(hipStreamWaitEvent(s, D.ev, 0));
+    }
+    return SVFSI_OK;
 }
 
 // LDS of k_ppoly: two exchange tables, halo positions
@@ -245,11 +290,11 @@ void persist_build(Lhs& L)
     }
 }
 
-Parts* persist_parts(Lhs& L)
+Parts* persist_parts(Lhs& L, bool pcg)
 {
     // SVFSI_PERSIST=0: one launch per product throughout (read at each call)
     const char* e = getenv("SVFSI_PERSIST");
-    if (!L.parts || L.parts->off || (e && e[0] == '0')) return nullptr;
+    if (!L.parts || L.parts->off || (pcg && !pcg_fits(*L.parts)) || (e && e[0] == '0')) return nullptr;
     // SVFSI_PERSIST_WAIT: ticks of 10 ns a lane waits before it gives up; 0:
     // at the first word that is not there yet (tests of that path)
     const char* w = getenv("SVFSI_PERSIST_WAIT");

@@ -33,10 +33,12 @@
 // workgroup may start while the flags change, so one lane reads them for all
 // (leave_at_start).  Giving up happens only
 // when the parts are not resident together (another kernel that itself waits
-// holds CUs); PersistLock keeps two such kernels of one process apart.
+// holds CUs); ResidentTurn keeps two such kernels of one process apart.
 #pragma once
 
 #include "internal.hpp"
+
+#include <mutex>
 
 namespace svfsi {
 
@@ -143,20 +145,40 @@ struct Parts {
 
 // Partitions L if its pattern fits the chip (at the end of FSILS_LHS_CREATE).
 void persist_build(Lhs& L);
-// The partition of L; nullptr when there is none or the path is off.
-Parts* persist_parts(Lhs& L);
+// The partition of L for a solve; nullptr when there is none, the path is off,
+// or (pcg) the kernels of pcg.hip do not fit it.
+Parts* persist_parts(Lhs& L, bool pcg);
 
-// One matrix-resident solve at a time per device and process, the others wait
-// on the host: their kernels would wait for each other's CUs, and a solve that
-// took the other path instead would differ in its last bits.
-struct PersistLock {
+// A solve that launches matrix-resident kernels, from enter to leave (or its
+// end).  Kernels of two such solves on different streams would wait for each
+// other's CUs, so each launch is put behind what the other solves of the device
+// and process have queued so far, by events on the device: the solves' other
+// kernels overlap, no host thread waits, and a solve that is alone pays a
+// mutex.  Streams named by hipStreamPerThread, which another thread cannot
+// name, take turns solve by solve instead.
+struct ResidentTurn {
     int dev = -1;
-    PersistLock() = default;
-    PersistLock(const PersistLock&) = delete;
-    PersistLock& operator=(const PersistLock&) = delete;
-    ~PersistLock() { release(); }
-    bool acquire();
-    void release();
+    hipStream_t s = nullptr;
+    ResidentTurn *prev = nullptr, *next = nullptr;
+    ResidentTurn() = default;
+    ResidentTurn(const ResidentTurn&) = delete;
+    ResidentTurn& operator=(const ResidentTurn&) = delete;
+    ~ResidentTurn() { leave(); }
+    bool enter(hipStream_t stream);
+    void leave();
+    // launch() with no other resident launch of the device between the events
+    // and it
+    template <class F>
+    int launch(F&& f)
+    {
+        std::lock_guard<std::mutex> g(mutex());
+        SV_TRY(follow_others());
+        return f();
+    }
+
+private:
+    std::mutex& mutex() const;
+    int follow_others();
 };
 
 // z = p(B) D^-1 q, all factors of the polynomial preconditioner in one

@@ -4,6 +4,7 @@ rows summed in another order, so the mixed solve makes the same outer steps
 (one more or less where the residual passes near the tolerance) and reaches
 the same solution to its own tolerance."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -116,8 +117,8 @@ def test_first_solve_on_recycled_memory(gpu, monkeypatch, mixed):
 
 @pytest.mark.gpu
 def test_two_threads(gpu, monkeypatch):
-    """Two solves at once on streams of their own, one of which finds the
-    matrix-resident path taken."""
+    """Two mixed solves at once on streams of their own: their matrix-resident
+    launches take turns, and both solve as they do alone."""
     import torch
 
     from svfsi_amd.step import NewtonStep
@@ -144,6 +145,44 @@ def test_two_threads(gpu, monkeypatch):
     for (x, itr, suc), (y, itr0, _) in zip(got, want):
         assert suc == 1 and abs(itr - itr0) <= 1
         assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,persist", [("hub_no_fit", "1"), ("lelas_1part", "0"), ("lelas_1part", "1")])
+def test_does_not_wait_for_another_solve(gpu, monkeypatch, name, persist):
+    """A solve without a partition, with the path off, or matrix-resident
+    itself, beside a matrix-resident one of half a million iterations (2 s or
+    more): it ends while that one runs."""
+    import torch
+
+    from svfsi_amd.step import NewtonStep
+
+    monkeypatch.setenv("SVFSI_PERSIST", "1")
+    monkeypatch.delenv("SVFSI_PERSIST_WAIT", raising=False)
+    cg = dict(LS_type=fsils.LS_TYPE_CG, absTol=1e-300)
+    slow = NewtonStep(with_ls(CASES["lelas_parts"](), relTol=1e-300, mItr=100, **cg))
+    fast = NewtonStep(with_ls(CASES[name](), relTol=1e-8, mItr=2000, **cg))
+    slow.step(), fast.step()  # workspaces
+    slow.assemble(), fast.assemble()
+    torch.cuda.synchronize()
+    slow.prob.ls["mItr"] = 500000
+    began = threading.Event()
+
+    def work():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            began.set()
+            slow.solve()
+
+    t = threading.Thread(target=work)
+    t.start()
+    began.wait()
+    time.sleep(0.1)
+    monkeypatch.setenv("SVFSI_PERSIST", persist)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        ls = fast.solve()
+        running = t.is_alive()
+    t.join()
+    assert ls.RI.suc == 1 and running
 
 
 def with_ls(prob, **ls):
