@@ -291,6 +291,11 @@ int svfsi_spmv_t_dev(void* lhs, int dof, const double* dK, const double* dU,
  * number of levels (0: none). */
 int svfsi_amg_aggregate(int nNo, const int* rowPtr, const int* colPtr, int cap, int* agg);
 int svfsi_amg_levels(void* lhs, int* nodes, int maxLevels);
+/* The matrix-resident kernels of lhs (no reference counterpart): stats[0..3]
+ * receive the parts of its pattern (0: none, every solve makes one launch per
+ * step), the blocks a lane holds, the launches made so far, and the solves
+ * that gave them up after a wait and ran again with one launch per step. */
+int svfsi_resident_stats(void* lhs, long long* stats);
 
 /* Residual dR = dB - K dU (transpose != 0: dB - K^T dU) with every row's sum
  * carried in double-double (FMA-split products, TwoSum accumulation) and

@@ -112,6 +112,7 @@ SIGNATURES = {
     "svfsi_resid_dd_dev": [_P, _I, _P, _P, _P, _P, _I, _P],
     "svfsi_amg_aggregate": [_I, _P, _P, _I, _P],
     "svfsi_amg_levels": [_P, _P, _I],
+    "svfsi_resident_stats": [_P, C.POINTER(C.c_longlong)],
     "svfsi_dot_dev": [_I, _P, _P, _DP, _P],
     "svfsi_precond_diag_dev": [_P, _I, _P, _P, _P, _IP, _P],
     "svfsi_precond_rcs_dev": [_P, _I, _P, _P, _P, _P, _IP, _P],

@@ -661,6 +661,17 @@ int svfsi_amg_levels(void* lhs, int* nodes, int maxLevels)
     return n;
 }
 
+int svfsi_resident_stats(void* lhs, long long* stats)
+{
+    SV_ARG(lhs && stats, "NULL argument");
+    const Parts* P = static_cast<Lhs*>(lhs)->parts.get();
+    stats[0] = P ? P->G : 0;
+    stats[1] = P ? P->U : 0;
+    stats[2] = P ? P->launches : 0;
+    stats[3] = P ? P->giveUps : 0;
+    return SVFSI_OK;
+}
+
 int svfsi_resid_dd_dev(void* lhs, int dof, const double* dK, const double* dU, const double* dB, double* dR,
                        int transpose, void* stream)
 {

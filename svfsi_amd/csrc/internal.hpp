@@ -182,7 +182,7 @@ struct Lhs {
     int nTiles[3] = {0, 0, 0};
     CplSet cpl;
     Work ws;
-    std::shared_ptr<Parts> parts; // built on first use
+    std::shared_ptr<Parts> parts; // built in FSILS_LHS_CREATE; null: the pattern has none
 };
 
 // Contributions per workgroup of the tet4 record gathers: 64, 128 and 256 take

@@ -536,7 +536,7 @@ int cg_core(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hi
         }
         if (parts && finished && hs.abort) {
             SV_HIP(hipStreamSynchronize(s));
-            parts->off = true;
+            parts->gave_up();
             parts = nullptr;
             turn.leave();
             SV_HIP(hipMemcpyAsync(R, KP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -1035,7 +1035,7 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
         }
         if (parts && finished && hs.abort) {
             SV_HIP(hipStreamSynchronize(s));
-            parts->off = true;
+            parts->gave_up();
             parts = nullptr;
             turn.leave();
             SV_HIP(hipMemcpyAsync(R, SP, n * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -2603,7 +2603,7 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
         }
         if (parts && hs.abort) {
             SV_HIP(hipStreamSynchronize(s));
-            parts->off = true;
+            parts->gave_up();
             *retry = true;
             return SVFSI_OK;
         }
@@ -2617,7 +2617,7 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
         SV_HIP(hipMemcpyAsync(&hs, st, sizeof(GmState), hipMemcpyDeviceToHost, s));
         SV_HIP(hipStreamSynchronize(s));
         if (parts && hs.abort) {
-            parts->off = true;
+            parts->gave_up();
             *retry = true;
             return SVFSI_OK;
         }

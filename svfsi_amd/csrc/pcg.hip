@@ -471,6 +471,7 @@ int pcg3_launch(Lhs& L, Parts& P, const double* K, double* X, double* R, double*
                        P.epoch + 1);
     SV_HIP(hipGetLastError());
     P.epoch += (unsigned)its + 1u;
+    ++P.launches;
     return SVFSI_OK;
 }
 
@@ -484,6 +485,7 @@ int pcgs_launch(Lhs& L, Parts& P, const double* Lm, const double* G, const doubl
                        its, P.epoch + 1);
     SV_HIP(hipGetLastError());
     P.epoch += (unsigned)its + 1u;
+    ++P.launches;
     return SVFSI_OK;
 }
 

@@ -59,6 +59,17 @@ void ResidentTurn::leave()
     dev = -1;
 }
 
+// The device's event, made with its first partition: solves allocate nothing.
+static int make_event()
+{
+    int d = 0;
+    SV_HIP(hipGetDevice(&d));
+    if (d < 0 || d >= kDevices) return SVFSI_OK; // no solve enters there
+    std::lock_guard<std::mutex> g(g_dev[d].mu);
+    if (!g_dev[d].ev) SV_HIP(hipEventCreateWithFlags(&g_dev[d].ev, hipEventDisableTiming));
+    return SVFSI_OK;
+}
+
 // The streams of the others are alive: their solves are inside.  An event may be
 // recorded again once a stream was told to wait for it.
 int ResidentTurn::follow_others()
@@ -66,7 +77,6 @@ int ResidentTurn::follow_others()
     Device& D = g_dev[dev];
     for (ResidentTurn* t = D.turns; t; t = t->next) {
         if (t == this || t->s == s) continue;
-        if (!D.ev) SV_HIP(hipEventCreateWithFlags(&D.ev, hipEventDisableTiming));
         SV_HIP(hipEventRecord(D.ev, t->s));
         SV_HIP(hipStreamWaitEvent(s, D.ev, 0));
     }
@@ -272,7 +282,11 @@ static int choose(Lhs& L, Parts& P)
     SV_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, d));
     SV_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, d));
     // 8 lanes and 3 blocks a lane suit tet4 rows (15 to 24 blocks); where
-    // that needs more lanes than the chip has, 4 lanes and 5 blocks
+    // that needs more lanes than the chip has, 4 lanes and 5 blocks.  Mixed
+    // solve, with them / with one launch per factor, ms: 3 blocks, elasticity
+    // cube 28^3 2.99 / 4.47; 5 blocks, cubes 32^3 3.75 / 5.86 and 37^3 5.14 /
+    // 9.68, fluid cylinders of 35,306, 40,381 and 47,392 nodes 4.69 / 8.66,
+    // 4.72 / 9.09 and 5.72 / 11.2.  CG has no form with 5 blocks.
     SV_TRY(build(L, P, 3, 8, cus, (size_t)lds));
     if (!P.G) SV_TRY(build(L, P, 5, 4, cus, (size_t)lds));
     return SVFSI_OK;
@@ -284,7 +298,7 @@ void persist_build(Lhs& L)
     if (!L.symmetric) return;
     try {
         std::shared_ptr<Parts> P = std::make_shared<Parts>();
-        if (choose(L, *P) != SVFSI_OK) (void)hipGetLastError();
+        if (choose(L, *P) != SVFSI_OK || (P->G > 0 && make_event() != SVFSI_OK)) (void)hipGetLastError();
         else if (P->G > 0) L.parts = P;
     } catch (...) { // out of host memory: no parts
     }

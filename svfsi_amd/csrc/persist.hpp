@@ -129,6 +129,12 @@ struct Parts {
     int G = 0, U = 0, maxOwn = 0, maxHalo = 0, maxLanes = 0;
     unsigned epoch = 0; // the last tag used; xb starts out with tag 0
     bool off = false;
+    long long launches = 0, giveUps = 0; // svfsi_resident_stats
+    void gave_up()
+    {
+        ++giveUps;
+        off = true;
+    }
     unsigned long long wait = kWaitTicks;
     size_t ldsMax = 0;
     DBuf tab, xb;
@@ -197,7 +203,9 @@ int pcg3_launch(Lhs& L, Parts& P, const double* K, double* X, double* R, double*
 int pcgs_launch(Lhs& L, Parts& P, const double* Lm, const double* G, const double* Gt, double* X, double* R,
                 double* Pv, CgState* st, int its, hipStream_t s);
 size_t pcg_lds(const Parts& P); // their dynamic LDS
-inline bool pcg_fits(const Parts& P) // 16 groups of 16 parts share the sums
+// whether they fit: their static LDS is below 512 bytes, and the sums were
+// measured with at most 256 partials
+inline bool pcg_fits(const Parts& P)
 {
     return P.U == 3 && P.G <= 256 && pcg_lds(P) + 512 <= P.ldsMax;
 }

@@ -219,6 +219,7 @@ static int launch(Lhs& L, Parts& P, const float* B, const float* dinv, const dou
               abortFlag);
     SV_HIP(hipGetLastError());
     P.epoch += (unsigned)nOps + 1u;
+    ++P.launches;
     return SVFSI_OK;
 }
 

@@ -84,6 +84,13 @@ class Lhs:
         self.rowPtr = rowPtr
         self.colPtr = colPtr
 
+    def resident_stats(self) -> dict:
+        """Parts and blocks a lane of the matrix-resident kernels (0: none),
+        their launches so far, and the solves that gave them up."""
+        v = (C.c_longlong * 4)()
+        call("svfsi_resident_stats", self.handle, v)
+        return dict(parts=v[0], blocks=v[1], launches=v[2], give_ups=v[3])
+
     def free(self) -> None:
         if self.handle:
             call("fsils_gpu_lhs_free", self.handle)

@@ -41,11 +41,20 @@ CASES = {
     "hub_16_lanes": lambda: hub(40),
     "hub_64_lanes": lambda: hub(150),
     "hub_no_fit": lambda: hub(400),
+    "lelas_5_blocks": lambda: problems.lelas_cube(32),
+    "fluid_5_blocks": lambda: problems.fluid_cylinder(h=0.095),
     "tet10": lambda: problems.struct_cube(3, Kpen=1e5),
 }
 
 
-def solve(prob, monkeypatch, persist, wait=None, mixed=True):
+# blocks a lane of the patterns that get other than three; 0: no partition
+BLOCKS = {"hub_no_fit": 0, "lelas_5_blocks": 5, "fluid_5_blocks": 5}
+
+
+def solve(prob, monkeypatch, persist, wait=None, mixed=True, blocks=None):
+    """The second of two equal solves, after checking which kernels ran: those
+    of a partition with `blocks` blocks a lane (None: as PERSIST says; 0: none),
+    given up once if the wait is 0."""
     import torch
 
     from svfsi_amd.step import NewtonStep
@@ -61,6 +70,11 @@ def solve(prob, monkeypatch, persist, wait=None, mixed=True):
         ls = st.step(mixed=mixed)
         torch.cuda.synchronize()
         out.append((st.R.cpu().numpy().copy(), ls.RI.itr, ls.RI.suc))
+    r = st.lhs.resident_stats()
+    if blocks is not None:
+        assert r["blocks"] == blocks and (r["parts"] > 0) == (blocks > 0)
+    used = persist == "1" and r["parts"] > 0 and (mixed or r["blocks"] == 3) and prob.ls["mItr"] > 0
+    assert (r["launches"] > 0) == used and r["give_ups"] == (1 if used and wait == "0" else 0), r
     assert np.array_equal(out[0][0], out[1][0])
     return out[0]
 
@@ -69,7 +83,7 @@ def solve(prob, monkeypatch, persist, wait=None, mixed=True):
 @pytest.mark.parametrize("name", list(CASES))
 def test_matches_one_launch_per_factor(gpu, monkeypatch, name):
     prob = CASES[name]()
-    x, itr, suc = solve(prob, monkeypatch, "1")
+    x, itr, suc = solve(prob, monkeypatch, "1", blocks=BLOCKS.get(name, 3))
     y, itr0, suc0 = solve(prob, monkeypatch, "0")
     assert suc == suc0 == 1 and abs(itr - itr0) <= 1
     # both solve to 1e-8 in the scaled residual
@@ -77,13 +91,13 @@ def test_matches_one_launch_per_factor(gpu, monkeypatch, name):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["lelas_parts", "lelas_all_cus", "fluid_mid", "tet10"])
+@pytest.mark.parametrize("name", ["lelas_parts", "lelas_all_cus", "fluid_mid", "tet10", "lelas_5_blocks", "fluid_5_blocks"])
 def test_gives_up_and_falls_back(gpu, monkeypatch, name):
     """A wait of no ticks: the kernel ends at the first word not yet there,
     some workgroups before others have started, and the solve runs again with
     one launch per factor, to the same bits."""
     prob = CASES[name]()
-    x, itr, suc = solve(prob, monkeypatch, "1", wait="0")
+    x, itr, suc = solve(prob, monkeypatch, "1", wait="0", blocks=BLOCKS.get(name, 3))
     y, itr0, suc0 = solve(prob, monkeypatch, "0")
     assert suc == suc0 == 1 and itr == itr0
     assert np.array_equal(x, y)
@@ -145,6 +159,9 @@ def test_two_threads(gpu, monkeypatch):
     for (x, itr, suc), (y, itr0, _) in zip(got, want):
         assert suc == 1 and abs(itr - itr0) <= 1
         assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y)
+    for st in steps:
+        r = st.lhs.resident_stats()
+        assert r["launches"] > 0 and r["give_ups"] == 0
 
 
 @pytest.mark.gpu
@@ -183,6 +200,9 @@ def test_does_not_wait_for_another_solve(gpu, monkeypatch, name, persist):
         running = t.is_alive()
     t.join()
     assert ls.RI.suc == 1 and running
+    r, q = fast.lhs.resident_stats(), slow.lhs.resident_stats()
+    assert (r["launches"] > 0) == (name == "lelas_1part") and r["give_ups"] == q["give_ups"] == 0
+    assert q["launches"] >= 500000 // 256
 
 
 def with_ls(prob, **ls):
@@ -205,7 +225,7 @@ def test_fp64_matches_one_launch_per_step(gpu, monkeypatch, name):
     """CG and the Schur complement's CG: sums over the parts in another order,
     so the same solution to the solver's tolerance."""
     prob = FP64[name]()
-    x, itr, suc = solve(prob, monkeypatch, "1", mixed=False)
+    x, itr, suc = solve(prob, monkeypatch, "1", mixed=False, blocks=BLOCKS.get(name, 3))
     y, itr0, suc0 = solve(prob, monkeypatch, "0", mixed=False)
     assert suc == suc0 == 1 and abs(itr - itr0) <= 2
     tol = 1e-4 if name.startswith("ns_") else 1e-6  # relTol 1e-5 and 1e-8, times the conditioning
@@ -228,7 +248,7 @@ def test_cg_iteration_limit(gpu, monkeypatch, mItr):
 @pytest.mark.parametrize("name", ["lelas_parts", "lelas_all_cus", "ns_fluid_few", "ns_fluid_mid"])
 def test_fp64_gives_up_and_falls_back(gpu, monkeypatch, name):
     prob = FP64[name]()
-    x, itr, suc = solve(prob, monkeypatch, "1", wait="0", mixed=False)
+    x, itr, suc = solve(prob, monkeypatch, "1", wait="0", mixed=False, blocks=3)
     y, itr0, suc0 = solve(prob, monkeypatch, "0", mixed=False)
     assert (itr, suc) == (itr0, suc0)
     assert np.array_equal(x, y)
