@@ -554,6 +554,7 @@ int cg_core(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, double* R, hi
     SV_HIP(hipMemcpyAsync(&hs, st, sizeof(CgState), hipMemcpyDeviceToHost, s));
     SV_HIP(hipMemcpyAsync(R, X, n * sizeof(double), hipMemcpyDeviceToDevice, s));
     SV_HIP(hipStreamSynchronize(s));
+    if (parts) parts->solved();
     ls.suc = hs.suc;
     ls.itr = hs.itr;
     ls.cM = hs.itr;
@@ -1055,6 +1056,7 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
     SV_HIP(hipMemcpy(&hs, st, sizeof(CgState), hipMemcpyDeviceToHost));
     SV_HIP(hipMemcpyAsync(R, X, n * sizeof(double), hipMemcpyDeviceToDevice, s));
     SV_HIP(hipStreamSynchronize(s));
+    if (parts) parts->solved();
     ls.suc = hs.suc;
     ls.fNorm = std::sqrt(hs.err);
     ls.callD = wall_seconds() - time + ls.callD;
@@ -2641,6 +2643,7 @@ static int nested_solve(Lhs& L, FSILS_subLsType& ls, int dof, const double* K, I
     }
     SV_HIP(hipMemcpyAsync(R, x, n * sizeof(double), hipMemcpyDeviceToDevice, s));
     SV_HIP(hipStreamSynchronize(s));
+    if (parts) parts->solved();
     ls.callD = wall_seconds() - ls.callD;
     ls.dB = 10.0 * std::log(ls.fNorm / ls.dB);
     return SVFSI_OK;

@@ -308,7 +308,11 @@ Parts* persist_parts(Lhs& L, bool pcg)
 {
     // SVFSI_PERSIST=0: one launch per product throughout (read at each call)
     const char* e = getenv("SVFSI_PERSIST");
-    if (!L.parts || L.parts->off || (pcg && !pcg_fits(*L.parts)) || (e && e[0] == '0')) return nullptr;
+    if (!L.parts || (pcg && !pcg_fits(*L.parts)) || (e && e[0] == '0')) return nullptr;
+    if (L.parts->rest > 0) {
+        --L.parts->rest;
+        return nullptr;
+    }
     // SVFSI_PERSIST_WAIT: ticks of 10 ns a lane waits before it gives up; 0:
     // at the first word that is not there yet (tests of that path)
     const char* w = getenv("SVFSI_PERSIST_WAIT");

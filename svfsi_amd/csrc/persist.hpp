@@ -27,7 +27,8 @@
 //
 // Every wait is bounded: a lane that has polled for kWaitTicks raises the
 // abort flag, its workgroup ends, and all others end at their next wait; the
-// caller then takes the path of one launch per product.  A workgroup that
+// caller then takes the path of one launch per product, and so do some solves
+// after it (Parts::rest).  A workgroup that
 // gives up also sets the solver's own flag (stop, done) for the launches
 // already queued, and leaving frees its CU for one that had to wait: a
 // workgroup may start while the flags change, so one lane reads them for all
@@ -128,13 +129,18 @@ __device__ __forceinline__ bool get_words(const unsigned long long* const (&p)[N
 struct Parts {
     int G = 0, U = 0, maxOwn = 0, maxHalo = 0, maxLanes = 0;
     unsigned epoch = 0; // the last tag used; xb starts out with tag 0
-    bool off = false;
     long long launches = 0, giveUps = 0; // svfsi_resident_stats
+    // After a give-up the next `rest` solves go without; 16, and four times as
+    // many after each give-up in a row, up to 65,536: a passing contention costs
+    // a second and 16 slower solves, a lasting one a few seconds in an hour
+    int rest = 0, row = 0;
     void gave_up()
     {
         ++giveUps;
-        off = true;
+        rest = 16 << 2 * row;
+        if (row < 6) ++row;
     }
+    void solved() { row = 0; }
     unsigned long long wait = kWaitTicks;
     size_t ldsMax = 0;
     DBuf tab, xb;
@@ -151,8 +157,9 @@ struct Parts {
 
 // Partitions L if its pattern fits the chip (at the end of FSILS_LHS_CREATE).
 void persist_build(Lhs& L);
-// The partition of L for a solve; nullptr when there is none, the path is off,
-// or (pcg) the kernels of pcg.hip do not fit it.
+// The partition of L for a solve, asked for once by it; nullptr when there is
+// none, the path is off or resting after a give-up, or (pcg) the kernels of
+// pcg.hip do not fit it.
 Parts* persist_parts(Lhs& L, bool pcg);
 
 // A solve that launches matrix-resident kernels, from enter to leave (or its
