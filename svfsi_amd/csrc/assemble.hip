@@ -1879,11 +1879,11 @@ __global__ __launch_bounds__(256) void k_asm_struct_mfma(int begin, int count, c
 // elements of the 24^3 cube at the 4-point rule, less than staging the
 // operands for the matrix cores.
 //
-// points: a lane per (element, point) writes the point's record, with the
-// Jacobian's inverse B (Nx_a = B^T xi_a, xi_a the reference gradients): F^-T
-// B^T, F B^T, B B^T and scalars, 30 doubles.
-// k_struct_elem: a lane per point and node writes C xi_a, n_a and m_a to LDS,
-// then 50 lanes per element each sum two neighbouring blocks of a row over
+// k_struct_rec (4 points): a lane per (element, point) writes the point's
+// record, with the Jacobian's inverse B (Nx_a = B^T xi_a, xi_a the reference
+// gradients): F^-T B^T, F B^T, B B^T and scalars, 30 doubles.
+// k_struct_elem: a lane per point and node writes C xi_a, n_a and m_a to LDS
+// (15 points: a lane per point, from the mesh), then 50 lanes per element each sum two neighbouring blocks of a row over
 // the points and store them, element blocks contiguous (7.2 KB).
 // k_struct_rows: a wavefront per node adds the 720-byte strips of its
 // elements into the node's row of Val, in LDS, in element-id order.
@@ -1892,22 +1892,32 @@ __global__ __launch_bounds__(256) void k_asm_struct_mfma(int begin, int count, c
 // cube (82,944 elements), and the latency of the records' node gathers.  There
 // 661 us, against 1412 with B^T Dm B on the matrix cores and a coloured
 // scatter (30 launches, each a read-modify-write of scattered 72-byte blocks,
-// 1.22 ms); 4,374 elements with 15 points: 559 -> 78 us.  Strips formed in the
+// 1.22 ms); 4,374 elements with 15 points: 559 -> 67 us.  Strips formed in the
 // row kernel from the records, without the blocks' trip through memory, took
 // 660 and 130 us (two or three wavefronts per SIMD, a serial chain each).
 // ---------------------------------------------------------------------------
 constexpr int SP_N = 0, SP_M = 9, SP_C = 18, SP_K = 24, SP_UD = 27, SP_SZ = 30; // point record
-constexpr int SN_SZ = 10;        // per node: C xi, n, m (scaled), pad
+constexpr int SN_SZ = 10;        // per node: C xi (without records Nx), n, m (scaled), pad
 constexpr int SQ_C = 10 * SN_SZ; // then kap, gam, w, w times the inertia
-constexpr int SQ_SZ = SQ_C + 6;
+constexpr int SQ_WS = SQ_C + 6;  // then, without records, w s
+template <bool REC> struct StructLds { static constexpr int SZ = REC ? SQ_WS : SQ_WS + 2; };
 
-// Record of point g of element e: F^-T B^T, w (-2/3 s) F B^T, w s B B^T (00, 11,
-// 22, 01, 02, 12), w (pl J + 2 r1/3), w (r1 - p J), w and w times the inertia.
-__device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ ien, const double* __restrict__ x,
-                                                 int tDof, const double* __restrict__ Ag,
-                                                 const double* __restrict__ Dg, const AsmParams& P,
-                                                 const double* __restrict__ rg, double* out)
+// Kinematics and neo-Hookean scalars of a point: the Jacobian's inverse B, F,
+// F^-T, the inertia ud, w, w s, -2/3 w s, w (pl J + 2 r1/3) and w (r1 - p J).
+struct StructPoint {
+    double B[3][3], F[3][3], Fi[3][3], ud[3], w, ws, cm, kap, gam;
+};
+
+// nx(a, Nx_a) is called for each node on the way.
+template <class NX>
+__device__ __forceinline__ void struct_point(int e, const int* __restrict__ ien, const double* __restrict__ x, int tDof,
+                                             const double* __restrict__ Ag, const double* __restrict__ Dg,
+                                             const AsmParams& P, const double* __restrict__ rg, StructPoint& S, NX&& nx)
 {
+    double (&B)[3][3] = S.B;
+    double (&F)[3][3] = S.F;
+    double (&Fi)[3][3] = S.Fi;
+    double (&ud)[3] = S.ud;
     double A[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll 5
     for (int a = 0; a < 10; ++a) {
@@ -1922,7 +1932,6 @@ __device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ 
     const double J = A[0][0] * A[1][1] * A[2][2] + A[0][1] * A[1][2] * A[2][0]
                    + A[0][2] * A[1][0] * A[2][1] - A[0][0] * A[1][2] * A[2][1]
                    - A[0][1] * A[1][0] * A[2][2] - A[0][2] * A[1][1] * A[2][0];
-    double B[3][3];
     B[0][0] = (A[1][1] * A[2][2] - A[1][2] * A[2][1]) / J;
     B[0][1] = (A[2][1] * A[0][2] - A[2][2] * A[0][1]) / J;
     B[0][2] = (A[0][1] * A[1][2] - A[0][2] * A[1][1]) / J;
@@ -1932,8 +1941,12 @@ __device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ 
     B[2][0] = (A[1][0] * A[2][1] - A[1][1] * A[2][0]) / J;
     B[2][1] = (A[2][0] * A[0][1] - A[2][1] * A[0][0]) / J;
     B[2][2] = (A[0][0] * A[1][1] - A[0][1] * A[1][0]) / J;
-    double F[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
-    double ud[3] = {-P.rho * P.fb[0], -P.rho * P.fb[1], -P.rho * P.fb[2]};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        ud[i] = -P.rho * P.fb[i];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) F[i][j] = i == j ? 1.0 : 0.0;
+    }
 #pragma unroll 5
     for (int a = 0; a < 10; ++a) {
         const int na = ien[(size_t)e * 10 + a];
@@ -1942,6 +1955,7 @@ __device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ 
         for (int j = 0; j < 3; ++j) {
             Nxa[j] = rg[11 + a * 3] * B[0][j] + rg[11 + a * 3 + 1] * B[1][j] + rg[11 + a * 3 + 2] * B[2][j];
         }
+        nx(a, Nxa);
         const double Na = rg[1 + a];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
@@ -1952,7 +1966,6 @@ __device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ 
         }
     }
     const double Jf = det3d(F);
-    double Fi[3][3]; // F^-T
     Fi[0][0] = (F[1][1] * F[2][2] - F[1][2] * F[2][1]) / Jf;
     Fi[0][1] = (F[1][2] * F[2][0] - F[1][0] * F[2][2]) / Jf;
     Fi[0][2] = (F[1][0] * F[2][1] - F[1][1] * F[2][0]) / Jf;
@@ -1973,10 +1986,28 @@ __device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ 
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) trC += F[i][j] * F[i][j];
-    const double w = rg[0] * J;
     const double s = pow(Jf, -2.0 / 3.0) * (2.0 * P.C10);
     const double r1 = s * trC / 3.0;
-    const double ws = w * s, cm = -2.0 / 3.0 * ws;
+    S.w = rg[0] * J;
+    S.ws = S.w * s;
+    S.cm = -2.0 / 3.0 * S.ws;
+    S.kap = S.w * (pl * Jf + 2.0 * r1 / 3.0);
+    S.gam = S.w * (r1 - p * Jf);
+}
+
+// Record of point g of element e: F^-T B^T, w (-2/3 s) F B^T, w s B B^T (00, 11,
+// 22, 01, 02, 12), w (pl J + 2 r1/3), w (r1 - p J), w and w times the inertia.
+__device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ ien, const double* __restrict__ x,
+                                                 int tDof, const double* __restrict__ Ag,
+                                                 const double* __restrict__ Dg, const AsmParams& P,
+                                                 const double* __restrict__ rg, double* out)
+{
+    StructPoint S;
+    struct_point(e, ien, x, tDof, Ag, Dg, P, rg, S, [](int, const double (&)[3]) {});
+    const double (&B)[3][3] = S.B;
+    const double (&F)[3][3] = S.F;
+    const double (&Fi)[3][3] = S.Fi;
+    const double ws = S.ws, cm = S.cm;
     double o[SP_SZ];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -1992,14 +2023,44 @@ __device__ __forceinline__ void struct_point_rec(int e, const int* __restrict__ 
     o[SP_C + 3] = bb(0, 1);
     o[SP_C + 4] = bb(0, 2);
     o[SP_C + 5] = bb(1, 2);
-    o[SP_K] = w * (pl * Jf + 2.0 * r1 / 3.0);
-    o[SP_K + 1] = w * (r1 - p * Jf);
-    o[SP_K + 2] = w;
+    o[SP_K] = S.kap;
+    o[SP_K + 1] = S.gam;
+    o[SP_K + 2] = S.w;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) o[SP_UD + i] = w * ud[i];
+    for (int i = 0; i < 3; ++i) o[SP_UD + i] = S.w * S.ud[i];
     // 240 bytes: 16-byte aligned
 #pragma unroll
     for (int q = 0; q < SP_SZ / 2; ++q) *reinterpret_cast<d2_t*>(out + 2 * q) = d2_t{o[2 * q], o[2 * q + 1]};
+}
+
+// The same point's node vectors, straight to LDS (SN_SZ doubles a node): Nx_a,
+// n_a and w (-2/3 s) m_a; then the scalars of SQ_C and w s.
+__device__ __forceinline__ void struct_point_vec(int e, const int* __restrict__ ien, const double* __restrict__ x,
+                                                 int tDof, const double* __restrict__ Ag,
+                                                 const double* __restrict__ Dg, const AsmParams& P,
+                                                 const double* __restrict__ rg, double* rc)
+{
+    StructPoint S;
+    struct_point(e, ien, x, tDof, Ag, Dg, P, rg, S, [rc](int a, const double (&Nxa)[3]) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) rc[a * SN_SZ + j] = Nxa[j];
+    });
+    rc[SQ_C] = S.kap;
+    rc[SQ_C + 1] = S.gam;
+    rc[SQ_C + 2] = S.w;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) rc[SQ_C + 3 + i] = S.w * S.ud[i];
+    rc[SQ_WS] = S.ws;
+#pragma unroll 5
+    for (int a = 0; a < 10; ++a) {
+        double* na = rc + a * SN_SZ;
+        const double n0 = na[0], n1 = na[1], n2 = na[2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            na[3 + i] = S.Fi[i][0] * n0 + S.Fi[i][1] * n1 + S.Fi[i][2] * n2;
+            na[6 + i] = S.cm * (S.F[i][0] * n0 + S.F[i][1] * n1 + S.F[i][2] * n2);
+        }
+    }
 }
 
 __global__ __launch_bounds__(256) void k_struct_rec(int nEl, int nG, const int* __restrict__ ien,
@@ -2013,11 +2074,12 @@ __global__ __launch_bounds__(256) void k_struct_rec(int nEl, int nG, const int* 
         struct_point_rec(e, ien, x, tDof, Ag, Dg, P, rule + (id - e * nG) * kTet10Rec, rec + (size_t)id * SP_SZ);
 }
 
-// Element blocks from the point records.  With 15 points the workgroup forms
-// its records itself (a quarter of its lanes busy; a launch of its own takes
-// 18 us at 4,374 elements); with 4, where a tenth would be
-// busy, they come from k_struct_rec (REC; 82,944 elements: 62 + 281 us
-// against 430).
+// Element blocks.  With 15 points 75 lanes of a workgroup take a point each,
+// from the mesh to its node vectors, for five elements: 67 us per call at 4,374
+// elements and 183 at 16,464, against 79 and 214 for two elements in 128 lanes
+// that left point records in LDS first (a launch of its own for the records
+// takes 18 us alone).  With 4 points, where 20 lanes would be busy, the records
+// come from k_struct_rec (REC; 82,944 elements: 62 + 281 us against 430).
 template <int NG, int EPW, int NT, bool REC>
 __global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restrict__ ien,
                                                     const double* __restrict__ x, int tDof,
@@ -2028,46 +2090,45 @@ __global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restri
 {
 #pragma clang fp contract(fast) // the Jacobians are behind: see the top of the file
     static_assert(EPW * 50 <= NT, "one pass of lanes in the second phase");
-    __shared__ __align__(16) double pt[EPW * NG][SQ_SZ];
-    __shared__ __align__(16) double sX[NG * 10][4]; // reference gradient and N
+    __shared__ __align__(16) double pt[EPW * NG][StructLds<REC>::SZ];
+    constexpr int XN = REC ? 3 : 0;
+    __shared__ __align__(16) double sX[NG * 10][XN + 1]; // reference gradient (with records) and N
     const int tid = threadIdx.x;
     const int e0 = blockIdx.x * EPW;
-    for (int q = tid; q < NG * 40; q += NT) {
-        const int g = q / 40, a = (q - 40 * g) / 4, c = q & 3;
-        sX[g * 10 + a][c] = rule[g * kTet10Rec + (c < 3 ? 11 + 3 * a + c : 1 + a)];
+    for (int q = tid; q < NG * 10 * (XN + 1); q += NT) {
+        const int n = q / (XN + 1), c = q - n * (XN + 1), g = n / 10, a = n - 10 * g;
+        sX[n][c] = rule[g * kTet10Rec + (c < XN ? 11 + 3 * a + c : 1 + a)];
     }
     const int nPt = min(EPW, nEl - e0) * NG;
-    const double* rec = recs + (size_t)e0 * NG * SP_SZ;
-    if constexpr (!REC) {
-        __shared__ __align__(16) double own[EPW * NG][SP_SZ];
-        for (int p = tid; p < nPt; p += NT)
-            struct_point_rec(e0 + p / NG, ien, x, tDof, Ag, Dg, P, rule + p % NG * kTet10Rec, own[p]);
-        __syncthreads();
-        rec = own[0];
-    }
-    for (int q = tid; q < nPt * 10; q += NT) {
-        const int p = q / 10, a = q - 10 * p, g = p % NG;
-        const d2_t* rc = reinterpret_cast<const d2_t*>(rec + (size_t)p * SP_SZ);
-        double o[SP_SZ];
+    if constexpr (REC) {
+        for (int q = tid; q < nPt * 10; q += NT) {
+            const int p = q / 10, a = q - 10 * p, g = p % NG;
+            const d2_t* rc = reinterpret_cast<const d2_t*>(recs + ((size_t)e0 * NG + p) * SP_SZ);
+            double o[SP_SZ];
 #pragma unroll
-        for (int u = 0; u < SP_SZ / 2; ++u) {
-            const d2_t v = rc[u];
-            o[2 * u] = v.x;
-            o[2 * u + 1] = v.y;
-        }
-        const double* xi = rule + g * kTet10Rec + 11 + 3 * a;
-        const double x0 = xi[0], x1 = xi[1], x2 = xi[2];
-        double* n = pt[p] + a * SN_SZ;
-        n[0] = o[SP_C] * x0 + o[SP_C + 3] * x1 + o[SP_C + 4] * x2;
-        n[1] = o[SP_C + 3] * x0 + o[SP_C + 1] * x1 + o[SP_C + 5] * x2;
-        n[2] = o[SP_C + 4] * x0 + o[SP_C + 5] * x1 + o[SP_C + 2] * x2;
+            for (int u = 0; u < SP_SZ / 2; ++u) {
+                const d2_t v = rc[u];
+                o[2 * u] = v.x;
+                o[2 * u + 1] = v.y;
+            }
+            const double* xi = rule + g * kTet10Rec + 11 + 3 * a;
+            const double x0 = xi[0], x1 = xi[1], x2 = xi[2];
+            double* n = pt[p] + a * SN_SZ;
+            n[0] = o[SP_C] * x0 + o[SP_C + 3] * x1 + o[SP_C + 4] * x2;
+            n[1] = o[SP_C + 3] * x0 + o[SP_C + 1] * x1 + o[SP_C + 5] * x2;
+            n[2] = o[SP_C + 4] * x0 + o[SP_C + 5] * x1 + o[SP_C + 2] * x2;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            n[3 + c] = o[SP_N + 3 * c] * x0 + o[SP_N + 3 * c + 1] * x1 + o[SP_N + 3 * c + 2] * x2;
-            n[6 + c] = o[SP_M + 3 * c] * x0 + o[SP_M + 3 * c + 1] * x1 + o[SP_M + 3 * c + 2] * x2;
+            for (int c = 0; c < 3; ++c) {
+                n[3 + c] = o[SP_N + 3 * c] * x0 + o[SP_N + 3 * c + 1] * x1 + o[SP_N + 3 * c + 2] * x2;
+                n[6 + c] = o[SP_M + 3 * c] * x0 + o[SP_M + 3 * c + 1] * x1 + o[SP_M + 3 * c + 2] * x2;
+            }
+            if (a < 6) pt[p][SQ_C + a] = a == 0 ? o[SP_K] : a == 1 ? o[SP_K + 1] : a == 2 ? o[SP_K + 2]
+                                         : a == 3 ? o[SP_UD] : a == 4 ? o[SP_UD + 1] : o[SP_UD + 2];
         }
-        if (a < 6) pt[p][SQ_C + a] = a == 0 ? o[SP_K] : a == 1 ? o[SP_K + 1] : a == 2 ? o[SP_K + 2]
-                                     : a == 3 ? o[SP_UD] : a == 4 ? o[SP_UD + 1] : o[SP_UD + 2];
+    } else {
+        static_assert(EPW * NG <= NT, "a lane per point");
+        if (tid < nPt)
+            struct_point_vec(e0 + tid / NG, ien, x, tDof, Ag, Dg, P, rule + tid % NG * kTet10Rec, pt[tid]);
     }
     __syncthreads();
     const int k = tid / 50, r = tid - k * 50, e = e0 + k;
@@ -2091,19 +2152,20 @@ __global__ __launch_bounds__(NT) void k_struct_elem(int nEl, const int* __restri
                 na[2 * q + 1] = v.y;
             }
             const double kap = rc[SQ_C], gam = rc[SQ_C + 1], w = rc[SQ_C + 2];
-            const double Na = sX[g * 10 + a][3];
+            const double Na = sX[g * 10 + a][XN];
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 double nb[SN_SZ];
 #pragma unroll
-                for (int q = 1; q < SN_SZ / 2; ++q) {
+                for (int q = REC ? 1 : 0; q < SN_SZ / 2; ++q) {
                     const d2_t v = *reinterpret_cast<const d2_t*>(rc + (b0 + h) * SN_SZ + 2 * q);
                     nb[2 * q] = v.x;
                     nb[2 * q + 1] = v.y;
                 }
                 const double* xb = sX[g * 10 + b0 + h];
-                T[h] += na[0] * xb[0] + na[1] * xb[1] + na[2] * xb[2];
-                M[h] += w * (Na * xb[3]);
+                if constexpr (REC) T[h] += na[0] * xb[0] + na[1] * xb[1] + na[2] * xb[2];
+                else T[h] += rc[SQ_WS] * (na[0] * nb[0] + na[1] * nb[1] + na[2] * nb[2]);
+                M[h] += w * (Na * xb[XN]);
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
                     const double eb = kap * nb[3 + j] + nb[6 + j]; // n_a's partner
@@ -2400,7 +2462,7 @@ int launch_asm_struct(Mesh& M, const AsmParams& P, int nG, const double* rule, i
         if (lds <= ((size_t)64 << 10) && !(v && v[0] == '0') && struct_scratch(M, nG)) {
             double* ke = M.ke.as<double>();
             double* re = M.re.as<double>();
-            constexpr int E4 = 5, E15 = 2;
+            constexpr int E4 = 5, E15 = 5;
             if (nG == 4) {
                 const size_t nPts = (size_t)M.nEl * nG;
                 double* rec = M.srec.as<double>();
@@ -2410,8 +2472,8 @@ int launch_asm_struct(Mesh& M, const AsmParams& P, int nG, const double* rule, i
                                    dim3(256), 0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule,
                                    (const double*)rec, ke, re);
             } else {
-                hipLaunchKernelGGL((k_struct_elem<15, E15, 128, false>), dim3((unsigned)((M.nEl + E15 - 1) / E15)),
-                                   dim3(128), 0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule,
+                hipLaunchKernelGGL((k_struct_elem<15, E15, 256, false>), dim3((unsigned)((M.nEl + E15 - 1) / E15)),
+                                   dim3(256), 0, s, M.nEl, M.ien.as<int>(), M.x.as<double>(), tDof, Ag, Dg, P, rule,
                                    (const double*)nullptr, ke, re);
             }
             hipLaunchKernelGGL(k_struct_rows, dim3((unsigned)((M.nNo + 3) / 4)), dim3(256), lds, s, M.nNo, M.maxRow,
