@@ -1889,8 +1889,9 @@ static int gmres_core(Lhs& L, const GmOp<BT>& op, int dof, BT* R, DBuf& basisBuf
     GmState hs{};
     const int chunk = 8;
     // up to kOneEnd row chunks the step ends in one launch (k_gm_rotupdate:
-    // every block sums the partials itself) instead of two
-    const bool oneEnd = nbr <= kOneEnd && (long long)nbr <= foldAt;
+    // every block sums the partials itself) instead of two, to the same bits
+    // (SVFSI_GM_ONE_END=0: two)
+    const bool oneEnd = nbr <= kOneEnd && (long long)nbr <= foldAt && env_int("SVFSI_GM_ONE_END", 1) != 0;
     const bool useGraphs = graphs_enabled();
     if (useGraphs) {
         std::vector<uintptr_t> sig = {
