@@ -99,7 +99,7 @@ def main() -> int:
     import torch
 
     from svfsi_amd import problems
-    from svfsi_amd._lib import SVFSI_STRUCT_MFMA32, SVFSI_STRUCT_MFMA64, SVFSI_STRUCT_VALU, lib
+    from svfsi_amd._lib import SVFSI_STRUCT_AUTO, SVFSI_STRUCT_MFMA32, SVFSI_STRUCT_MFMA64, SVFSI_STRUCT_VALU, lib
     from svfsi_amd.step import NewtonStep
 
     if not torch.cuda.is_available():
@@ -182,13 +182,13 @@ def main() -> int:
         torch.cuda.synchronize()
         b = time.perf_counter()
         L.svfsi_prof_enable(0)
-        cnt = [C.c_longlong(), C.c_longlong()]
-        tot = [C.c_double(), C.c_double()]
-        byt = [C.c_double(), C.c_double()]
-        for kk in (0, 1):
-            L.svfsi_prof_get(kk, C.byref(cnt[kk]), C.byref(tot[kk]))
-            L.svfsi_prof_get_bytes(kk, C.byref(byt[kk]))
-        return (b - a) * 1e3 / k, lss, [(cnt[q].value, tot[q].value, byt[q].value) for q in (0, 1)]
+        prof = []
+        for kk in (0, 1, 6):  # FP64 SpMV, FP32 SpMV, matrix-resident polynomial
+            cnt, tot, byt = C.c_longlong(), C.c_double(), C.c_double()
+            L.svfsi_prof_get(kk, C.byref(cnt), C.byref(tot))
+            L.svfsi_prof_get_bytes(kk, C.byref(byt))
+            prof.append((cnt.value, tot.value, byt.value))
+        return (b - a) * 1e3 / k, lss, prof
 
     # phase split (outside the timed loops): assembly alone
     torch.cuda.synchronize()
@@ -199,10 +199,11 @@ def main() -> int:
     asm_ms = (time.perf_counter() - a) * 1e3 / max(1, args.steps)
 
     log(f"assembly {asm_ms:.3f} ms")
-    # STRUCT: each element kernel on its own (vector units, FP64 MFMA, FP32
-    # MFMA), with the contraction kernels' event timing and MFMA rate
+    # STRUCT: each element kernel on its own (the default's outer products,
+    # vector units, FP64 MFMA, FP32 MFMA), with the contraction kernels' event
+    # timing and MFMA rate
     asm_kern = {}
-    struct_kernels = (("valu", SVFSI_STRUCT_VALU), ("mfma64", SVFSI_STRUCT_MFMA64),
+    struct_kernels = (("auto", SVFSI_STRUCT_AUTO), ("valu", SVFSI_STRUCT_VALU), ("mfma64", SVFSI_STRUCT_MFMA64),
                       ("mfma32", SVFSI_STRUCT_MFMA32))
     base_quad = prob.quad
     if args.workload == "struct":
@@ -218,6 +219,10 @@ def main() -> int:
                 st.assemble()
             torch.cuda.synchronize()
             ms = (time.perf_counter() - a) * 1e3 / max(1, args.steps)
+            if name == "auto":
+                asm_kern[name] = {"ms": round(ms, 3)}
+                log(f"assembly[{name}] {ms:.3f} ms")
+                continue
             L.svfsi_prof_reset()
             L.svfsi_prof_enable(1)
             st.assemble()
@@ -455,11 +460,12 @@ def main() -> int:
             what = ("the finest level of the multigrid V-cycle: FP32 CSR-stream block SpMVs over row tiles "
                     + ("with the residual (r = b - A x) or the Chebyshev step fused in" if fused else
                        "of the Chebyshev smoothing and the residuals"))
-        elif poly and os.environ.get("SVFSI_PERSIST", "") != "0" and n32 < lsprof[-1].RI.cM - n64m:
-            # fewer launches than products: the matrix-resident kernel, one launch per application
-            kname = f"k_ppoly<{dof}"
-            what = ("the polynomial preconditioner's factor steps in one matrix-resident launch per application, plus "
-                    "the setup Arnoldi SpMVs; bytes count the matrix once per launch")
+        elif profmx[2][0]:
+            # the matrix-resident kernel, one launch per application; launches
+            # queued after convergence exit at once, as the outer steps' do
+            kname = f"k_ppoly<{dof}, {st.lhs.resident_stats()['blocks']}"
+            what = ("the polynomial preconditioner's factor steps in one matrix-resident launch per application; "
+                    "bytes count the matrix once per launch")
         elif poly and os.environ.get("SVFSI_SPMV_STREAM", "") != "0":
             # the CSR-stream kernels over row tiles of 256 blocks (512 from 2M blocks on)
             tt = 512 if nnzb >= (2 << 20) else 256
@@ -478,19 +484,25 @@ def main() -> int:
         else:
             kname = "k_bspmv4<float, 4" if dof == 4 else f"k_bspmv<{dof}, float, float"
             what = "FP32 block SpMV, inner GMRES"
+        # launches, those that did the work, time and bytes of the kernel named
+        nL, nF, tL, bL = n32, n32_full, t32, b32
+        if kname.startswith("k_ppoly"):
+            nL, tL = profmx[2][:2]
+            nF, bL = min(nL, lsprof[-1].RI.itr), profmx[2][2] / nL
+        gbsL = bL * nF / (tL * 1e-3) / 1e9
         roof = {"kernel": f"{kname}> ({what})",
                 "bound": "latency" if kname.startswith("k_ppoly") else "hbm",
-                "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(gbs32 / HBM_PEAK_GBS, 4), "traffic": measured_traffic(nnzb, kname),
-                "bytes_per_launch": round(b32), "avg_launch_us": round(t32 / n32 * 1e3, 2), "launches": n32,
-                "full_work_launches": n32_full, "timing": "events attached to each dispatch (hipExtLaunchKernelGGL)"}
+                "achieved": round(gbsL, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(gbsL / HBM_PEAK_GBS, 4), "traffic": measured_traffic(nnzb, kname),
+                "bytes_per_launch": round(bL), "avg_launch_us": round(tL / nL * 1e3, 2), "launches": nL,
+                "full_work_launches": nF, "timing": "events attached to each dispatch (hipExtLaunchKernelGGL)"}
         # the 256 MiB Infinity Cache (MALL) sits between L2 and HBM: a launch whose bytes fit it streams
         # partly from there, so its rate is an effective one and the FETCH/WRITE counters bound the HBM bytes
         # from above rather than measuring them
         mall = 256 << 20
-        roof["working_set_bytes"] = round(b32)
+        roof["working_set_bytes"] = round(bL)
         roof["residency"] = ("fits the 256 MiB Infinity Cache: rate against the HBM peak is an effective "
-                             "rate, part of the bytes come from MALL" if b32 < mall else
+                             "rate, part of the bytes come from MALL" if bL < mall else
                              "larger than the 256 MiB Infinity Cache: streams from HBM")
     out = {
         "metric": "Assembly+GMRES time per Newton step at 1e-8 residual; FP64 vs mixed; SpMV GB/s",
@@ -547,8 +559,9 @@ def bench_ns(args, prob, t0) -> int:
     """Assembly + FSILS_SOLVE with the NS solver (NSSOLVER.f, LS.f:69-95
     defaults: RI 0.4 / 10, GM 1e-2 / 2 restarts of 100, CG 0.2 / 500) per
     Newton step, FP64 on the GPU, beside the oracle's NSSOLVER on the host
-    cores.  Roofline: the Schur-complement product (k_cgs_sp), the kernel
-    that dominates the solve."""
+    cores.  Roofline: the kernel that dominates the solve, the
+    matrix-resident Schur-complement CG (k_pcgs), or its product (k_cgs_sp)
+    where every step is a launch."""
     import ctypes as C
 
     import torch
@@ -579,7 +592,8 @@ def bench_ns(args, prob, t0) -> int:
     asm_ms = (time.perf_counter() - a) * 1e3 / args.steps
     log(f"ns step {ns_ms:.3f} ms (assembly {asm_ms:.3f} ms): RI.itr {ls.RI.itr} GM.itr {ls.GM.itr} "
         f"CG.itr {ls.CG.itr}")
-    # profiled step: dispatch-attached events on the Schur product
+    # profiled step: dispatch-attached events on the matrix-resident Schur CG,
+    # or on the Schur product where the solve makes one launch per step
     L.svfsi_prof_reset()
     L.svfsi_prof_enable(1)
     lsp = st.step()
@@ -595,12 +609,25 @@ def bench_ns(args, prob, t0) -> int:
     ct = os.environ.get("SVFSI_CGS_TILE")
     ct = int(ct) if ct in ("0", "512", "1024") else (512 if nnzb >= (2 << 20) else 0)
     kname = f"k_cgs_sp_t<{ct}>" if ct else "k_cgs_sp<8>"
-    roof = None if gbs is None else {
-        "kernel": f"{kname} (Schur-complement product SP = L P - Gt GP with its partial dot)", "bound": "hbm",
-        "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
-        "traffic": measured_traffic(nnzb, kname), "bytes_per_launch": round(bpl),
-        "avg_launch_us": round(tot.value / full * 1e3, 2), "launches": cnt.value, "full_work_launches": full,
-        "timing": "events attached to each dispatch (hipExtLaunchKernelGGL)"}
+    rc, rt, rb = C.c_longlong(), C.c_double(), C.c_double()
+    L.svfsi_prof_get(7, C.byref(rc), C.byref(rt))
+    L.svfsi_prof_get_bytes(7, C.byref(rb))
+    if rc.value:
+        gbs = rb.value / (rt.value * 1e-3) / 1e9
+        roof = {
+            "kernel": "k_pcgs<3> (up to 256 Schur-complement CG iterations in one matrix-resident launch; bytes count "
+                      "the matrix once per launch)", "bound": "latency",
+            "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
+            "traffic": measured_traffic(nnzb, "k_pcgs<3>"), "bytes_per_launch": round(rb.value / rc.value),
+            "us_per_iteration": round(rt.value / max(lsp.CG.itr, 1) * 1e3, 2), "launches": rc.value,
+            "timing": "events attached to each dispatch (hipExtLaunchKernelGGL)"}
+    else:
+        roof = None if gbs is None else {
+            "kernel": f"{kname} (Schur-complement product SP = L P - Gt GP with its partial dot)", "bound": "hbm",
+            "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
+            "traffic": measured_traffic(nnzb, kname), "bytes_per_launch": round(bpl),
+            "avg_launch_us": round(tot.value / full * 1e3, 2), "launches": cnt.value, "full_work_launches": full,
+            "timing": "events attached to each dispatch (hipExtLaunchKernelGGL)"}
     cpu = None
     acc = {}
     if not args.no_cpu:

@@ -478,12 +478,15 @@ int svfsi_poly_factors(int d, int ld, const double* Hu, double* coef,
 /* ---------------------------------------------------------------------- */
 int svfsi_prof_enable(int on);
 /* kernel: 0 = FP64 SpMV, 1 = FP32 SpMV (including the inner solver's SpMV
- * fused with its multi-dot, and the polynomial preconditioner's steps),
+ * fused with its multi-dot, and the polynomial preconditioner's steps where
+ * each is a launch),
  * 2 = STRUCT element kernels (one per colour), 3 = STRUCT material-point
  * kernel, 4 = the NS solver's Schur-complement product SP = L P - Gt GP
  * (with its partial dot), 5 = FP32 SpMV of the multigrid inner
- * preconditioner's coarse levels (its finest level counts as 1).  Returns
- * launches and total ms. */
+ * preconditioner's coarse levels (its finest level counts as 1), 6 =
+ * matrix-resident applications of the polynomial preconditioner, 7 =
+ * matrix-resident launches of CG and the Schur-complement CG (up to 256
+ * iterations each).  Returns launches and total ms. */
 int svfsi_prof_get(int kernel, long long* count, double* total_ms);
 /* Algorithmic bytes of the profiled launches of `kernel` (values, indices,
  * row pointers, x and y once; for the fused inner step also the basis

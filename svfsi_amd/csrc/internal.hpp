@@ -244,8 +244,10 @@ struct Prof {
     bool on = false;
     // slots: 0 FP64 SpMV, 1 FP32 SpMV (inner solver), 2 STRUCT element
     // kernels, 3 STRUCT material-point kernel, 4 NS Schur-complement product,
-    // 5 FP32 SpMV of the multigrid's coarse levels
-    static constexpr int kSlots = 6;
+    // 5 FP32 SpMV of the multigrid's coarse levels, 6 matrix-resident
+    // polynomial applications, 7 matrix-resident CG and Schur-complement CG
+    // launches
+    static constexpr int kSlots = 8;
     long long count[kSlots] = {};
     double ms[kSlots] = {};
     double bytes[kSlots] = {}; // algorithmic bytes (slot 2: MFMA flops) of the timed launches

@@ -1010,7 +1010,7 @@ int cg_schur_solve(Lhs& L, FSILS_subLsType& ls, const double* Gt, const double* 
     }
     // matrix-resident chunks as in cg_core
     ResidentTurn turn;
-    Parts* parts = !cpl && !h0.done && !prof().on ? persist_parts(L, true) : nullptr;
+    Parts* parts = !cpl && !h0.done ? persist_parts(L, true) : nullptr;
     if (parts && !turn.enter(s)) parts = nullptr;
     if (parts) SV_HIP(hipMemcpyAsync(SP, R, n * sizeof(double), hipMemcpyDeviceToDevice, s));
     int posted = 0;

@@ -466,9 +466,10 @@ int pcg3_launch(Lhs& L, Parts& P, const double* K, double* X, double* R, double*
 {
     const size_t lds = pcg_lds(P);
     SV_TRY(lds_limit(&k_pcg3<3>, lds));
-    hipLaunchKernelGGL(k_pcg3<3>, dim3((unsigned)P.G), dim3((unsigned)P.maxLanes), lds, s, P.dev(),
-                       P.maxOwn + P.maxHalo, P.maxHalo, L.rowPtr.as<int>(), K, X, R, Pv, st, its,
-                       P.epoch + 1);
+    // algorithmic bytes: the matrix and its indices once, X, R and P in and out
+    ProfScope ps(7, (double)L.nnz * (9.0 * 8.0 + 2.0) + 6.0 * 24.0 * L.nNo);
+    SV_LAUNCH(ps, k_pcg3<3>, dim3((unsigned)P.G), dim3((unsigned)P.maxLanes), lds, s, P.dev(),
+              P.maxOwn + P.maxHalo, P.maxHalo, L.rowPtr.as<int>(), K, X, R, Pv, st, its, P.epoch + 1);
     SV_HIP(hipGetLastError());
     P.epoch += (unsigned)its + 1u;
     ++P.launches;
@@ -480,9 +481,9 @@ int pcgs_launch(Lhs& L, Parts& P, const double* Lm, const double* G, const doubl
 {
     const size_t lds = pcg_lds(P);
     SV_TRY(lds_limit(&k_pcgs<3>, lds));
-    hipLaunchKernelGGL(k_pcgs<3>, dim3((unsigned)P.G), dim3((unsigned)P.maxLanes), lds, s, P.dev(),
-                       P.maxOwn + P.maxHalo, P.maxHalo, L.rowPtr.as<int>(), Lm, G, Gt, X, R, Pv, st,
-                       its, P.epoch + 1);
+    ProfScope ps(7, (double)L.nnz * (7.0 * 8.0 + 2.0) + 6.0 * 8.0 * L.nNo);
+    SV_LAUNCH(ps, k_pcgs<3>, dim3((unsigned)P.G), dim3((unsigned)P.maxLanes), lds, s, P.dev(),
+              P.maxOwn + P.maxHalo, P.maxHalo, L.rowPtr.as<int>(), Lm, G, Gt, X, R, Pv, st, its, P.epoch + 1);
     SV_HIP(hipGetLastError());
     P.epoch += (unsigned)its + 1u;
     ++P.launches;

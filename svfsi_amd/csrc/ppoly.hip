@@ -213,7 +213,7 @@ static int launch(Lhs& L, Parts& P, const float* B, const float* dinv, const dou
     // algorithmic bytes: the matrix and its indices once, q, z and z64, per
     // step one vector written and read
     const double vec = (double)L.nNo * DOF * 4.0;
-    ProfScope ps(1, (double)L.nnz * DOF * DOF * 4.0 + 2.0 * L.nnz + 5.0 * vec + 2.0 * nOps * vec);
+    ProfScope ps(6, (double)L.nnz * DOF * DOF * 4.0 + 2.0 * L.nnz + 5.0 * vec + 2.0 * nOps * vec);
     SV_LAUNCH(ps, (k_ppoly<DOF, U>), dim3((unsigned)P.G), dim3((unsigned)P.maxLanes), lds, s, P.dev(), L.nNo,
               P.maxOwn + P.maxHalo, L.rowPtr.as<int>(), B, dinv, q, z, z64, coef, ops, nOps, lastLin, base, stop,
               abortFlag);
