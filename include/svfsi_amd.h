@@ -480,8 +480,8 @@ int svfsi_prof_enable(int on);
 /* kernel: 0 = FP64 SpMV, 1 = FP32 SpMV (including the inner solver's SpMV
  * fused with its multi-dot, and the polynomial preconditioner's steps where
  * each is a launch),
- * 2 = STRUCT element kernels (one per colour), 3 = STRUCT material-point
- * kernel, 4 = the NS solver's Schur-complement product SP = L P - Gt GP
+ * 2 = STRUCT element kernels of the VALU and MFMA selectors (one per
+ * colour), 3 = the MFMA selectors' material-point kernel, 4 = the NS solver's Schur-complement product SP = L P - Gt GP
  * (with its partial dot), 5 = FP32 SpMV of the multigrid inner
  * preconditioner's coarse levels (its finest level counts as 1), 6 =
  * matrix-resident applications of the polynomial preconditioner, 7 =

@@ -37,7 +37,7 @@ def _opt(t):
 
 
 class DeviceMesh:
-    """Mesh bound to an lhs pattern: coordinates, colour-sorted connectivity
+    """Mesh bound to an lhs pattern: coordinates, connectivity
     and the DOASSEM scatter map, resident on the device."""
 
     def __init__(self, lhs: Lhs, m: TetMesh):

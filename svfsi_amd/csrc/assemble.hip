@@ -1,16 +1,22 @@
 // assemble.hip -- element tangent/residual construction and DOASSEM scatter
 // for gfx950.
 //
-// Elements are processed colour by colour (no two elements of a colour share
-// a node), so every block of Val and every row of R receives at most one
-// contribution per launch and the summation order is fixed: the assembly is
-// deterministic bit for bit.  Within a colour, one thread owns one (a,b)
-// node pair of one element: it recomputes the element geometry and the
-// Gauss-point kinematics (cheap, register resident) and accumulates its
-// dof x dof block over the Gauss points exactly as the reference routine
-// does for that block, then adds it to Val through the precomputed scatter
-// map (the bisection of DOASSEM, svFSI/LHSA.f:282-292, done once at mesh
-// creation).  The thread with b = 0 also builds the residual rows of node a.
+// By default one launch over all elements writes what the elements contribute
+// (tet4: a record of 128 or 320 bytes per element; tet10: its blocks) and a
+// second one sums, for each block of Val or row of a node, its elements'
+// contributions in element-id order, the order of DOASSEM's loop
+// (svFSI/LHSA.f:266-298): deterministic bit for bit, and no two lanes write one
+// place.
+//
+// The coloured kernels (SVFSI_ASM_GATHER=0, STRUCT's kernel selectors, and
+// STRUCT where rows are too long for LDS or the scratch cannot be had) process
+// elements colour by colour: no two elements of a colour share a node, so a
+// launch adds at most one contribution to a block or row, again in a fixed
+// order.  There one thread owns one (a,b) node pair of one element, recomputes
+// the geometry and the Gauss-point kinematics, accumulates its block over the
+// points as the reference routine does, and adds it to Val through the scatter
+// map (the bisection of LHSA.f:282-292, done once at mesh creation); the thread
+// with b = 0 also builds the residual rows of node a.
 #include "internal.hpp"
 #include "devutil.hpp"
 #include "assemble.hpp"
@@ -21,6 +27,8 @@
 // FMAs, in the oracle's operation order: Delaunay meshes contain sliver
 // elements whose Jacobian inversion amplifies any difference in rounding, and
 // the FP64 assembly is to reproduce the CPU restatement to ~1e-12 on them too.
+// What comes behind the inversion (sums over points, blocks from records) is
+// contracted, by a pragma where it is.
 #pragma clang fp contract(off)
 
 namespace svfsi {
@@ -2287,13 +2295,12 @@ __global__ __launch_bounds__(256) void k_gather(size_t nItems, const int* __rest
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-// Gather assembly: one launch over all elements stores the element blocks
-// at their gather positions, then k_gather sums them into Val and R.  The
-// default for tet4, whose 16- and 9-double blocks; TET10 (STRUCT) keeps the
-// coloured scatter, which measured faster there (5.0 vs 5.8 ms on the 40^3
-// tet10 cube: its 72-byte blocks straddle cache lines, so the scattered
-// stores of the element blocks cost more than the coloured read-modify-
-// write).  SVFSI_ASM_GATHER = 0 / 1 overrides.
+// Whether tet4 assembly goes through records and a gather, and whether STRUCT's
+// matrix-core kernels, when selected, store their blocks for k_gather instead of
+// scattering them colour by colour.  Not by default there: 5.8 ms against 5.0
+// on the 40^3 tet10 cube, since 72-byte blocks straddle cache lines (the default
+// STRUCT kernels are others, launch_asm_struct).  SVFSI_ASM_GATHER = 0 / 1
+// overrides.
 static bool gather_enabled(int eNoN)
 {
     const char* v = getenv("SVFSI_ASM_GATHER");

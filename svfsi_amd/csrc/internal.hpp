@@ -214,7 +214,8 @@ struct Mesh {
     DBuf midNodes;   // tet10: the nodes that are a mid-edge node of some element
     int nMid = 0;
     int rule10nG[2] = {0, 0};
-    DBuf srec;       // TET10 material-point records (nEl x nG x 97 doubles), grown on demand
+    DBuf srec;       // TET10 point records, grown on demand: 30 doubles a point (default kernels, 4
+                     // points only) or 97 (matrix-core kernels)
     // Gather assembly: element block (slot p, a, b) is stored at position
     // gSlot[p*eNoN^2 + a*eNoN + b] of ke, so that the contributions to nnz
     // block j are ke positions gPtr[j] .. gPtr[j+1]-1, in element-id order
