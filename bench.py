@@ -451,7 +451,9 @@ def main() -> int:
     roof = None
     if gbs32 is not None:
         fused = dof == 4 and os.environ.get("SVFSI_FUSED_INNER", "0") == "1"
-        poly = dof in (3, 4) and os.environ.get("SVFSI_INNER_POLY", "1") != "0"
+        # saddle-point systems get the inner GMRES cycle by default
+        saddle = args.workload == "fluid-th"
+        poly = dof in (3, 4) and os.environ.get("SVFSI_INNER_POLY", "0" if saddle else "1") != "0"
         if amg_default:
             tt = 512 if nnzb >= (2 << 20) else 256
             fused = os.environ.get("SVFSI_AMG_FUSED", "") != "0"
@@ -481,6 +483,9 @@ def main() -> int:
         elif fused:
             nt = "true" if nnzb * 64 > (128 << 20) else "false"
             kname, what = f"k_gm_spmv_dots4<{nt}", "FP32 block SpMV fused with the inner multi-dot"
+        elif dof in (3, 4) and os.environ.get("SVFSI_SPMV_STREAM", "") != "0":
+            kname = f"k_sspmv<float, {dof}, {512 if nnzb >= (2 << 20) else 256}"
+            what = "FP32 CSR-stream block SpMV over row tiles, inner GMRES"
         else:
             kname = "k_bspmv4<float, 4" if dof == 4 else f"k_bspmv<{dof}, float, float"
             what = "FP32 block SpMV, inner GMRES"
