@@ -14,9 +14,10 @@
 // (every part reads all partials; two levels of 16 took 1.1 us more), the
 // exchange of R travels with the second and that of G P with the first, and
 // sums over a wavefront go by DPP (shuffles: 1 us more per iteration).  Per
-// iteration, 9,261-node elasticity cube: 12.4 us with three launches, 7.0 here
-// (step 5.4 -> 3.3 ms); 26,667-node cylinder, Schur complement: 18.6 us, here
-// 10.9 (NS step 8.3 -> 5.0 ms).
+// iteration, 9,261-node elasticity cube: 12.4 us with three launches, 6.2 here
+// (step 5.4 -> 2.8 ms); 26,667-node cylinder, Schur complement: 18.6 us, here
+// 10.3 (NS step 8.3 -> 4.8 ms).  The tables are 16-byte aligned: behind static
+// LDS of an odd number of doubles the steps took 3.2 and 5.0 ms.
 #include "persist.hpp"
 #include "devutil.hpp"
 #include "stream.hpp"
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(1024) void k_pcg3(PartsDev P, int tabN, int maxHalo
 {
     __shared__ ReduceLds L;
     if (leave_at_start(&st->done, &L.bad)) return;
-    extern __shared__ double ldsd[];
+    extern __shared__ __align__(16) double ldsd[]; // four doubles a node, read together
     double* tp = ldsd;                // P: own rows, then the halo, 4 per node
     double* tr = tp + 4 * tabN;       // R of the halo, 3 per node
     int* sH = reinterpret_cast<int*>(tr + 3 * maxHalo);
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(1024) void k_pcgs(PartsDev P, int tabN, int maxHalo
 {
     __shared__ ReduceLds L;
     if (leave_at_start(&st->done, &L.bad)) return;
-    extern __shared__ double ldsd[];
+    extern __shared__ __align__(16) double ldsd[]; // four doubles a node, read together
     double* tg = ldsd;                // G P: own rows, then the halo, 4 per node
     double* tp = tg + 4 * tabN;       // P: own rows, then the halo
     double* tr = tp + tabN;           // R of the halo

@@ -13,10 +13,10 @@
 // steps, 8.1 us each, 200 us per application with the launches around them;
 // here a step is one trip of the halo through memory and a few hundred ns of
 // LDS gathers, shuffles and FP64 updates, and the matrix is read once per
-// application: 97 us, the mixed step of that mesh 6.05 -> 4.06 ms (LELAS 20^3
-// 2.95 -> 2.21 ms, 4,918-node cylinder 2.50 -> 1.98 ms).  The table is 16-byte
-// aligned and indexed from its own name, so that a gather is one ds_read_b128;
-// through a pointer array it was a flat load (mixed step 4.04 against 3.77 ms).
+// application: 80 us, the mixed step of that mesh 6.05 -> 3.77 ms (LELAS 20^3
+// 2.95 -> 2.12 ms).  The table is 16-byte aligned and indexed from its own
+// name, so that a gather is one ds_read_b128; through a pointer array it was a
+// flat load (93 us, step 4.04 ms).
 // With dof 4 and five blocks a lane 4 of the 128 registers spill (20 bytes of
 // scratch a lane).  Tried before: parts of consecutive rows (160 us: twice the
 // halo), products through LDS with a second barrier (3.2 us of the 6.5 us per
